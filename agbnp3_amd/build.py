@@ -85,7 +85,7 @@ def build_oracle(verbose=True):
     odir = os.path.join(_paths.REPO_DIR, "oracle")
     _run(["make", "-C", odir, "oracle"], verbose)
     ref = os.environ.get("AGBNP3_REF_DIR", "/root/reference")
-    if os.path.isdir(ref) and shutil.which("gcc"):
+    if os.path.exists(os.path.join(ref, "agbnp3.c")) and shutil.which("gcc"):
         _run(["make", "-C", odir, "ref", f"AGBNP3_REF_DIR={ref}"], verbose)
 
 
