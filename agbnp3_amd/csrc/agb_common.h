@@ -26,8 +26,12 @@ constexpr float kHbSwA = 0.65f, kHbSwB = 1.0f, kHbSwA0 = 0.6f;
 // overlap-tree kept / evaluated totals spread over kCountSlots 64-byte lines
 // (kCountBase + 8 s, + 1), so the blocks' adds at exit do not queue on one
 // address
-// atoms from which a call runs the water-site kernels on a second stream
+// atoms from which a call runs the water-site kernels on a second stream, and
+// from which the second tier of the derivative pass has that stream
 constexpr int kForkAtoms = 16384;
+constexpr int kSideAtoms = 512;
+// most items of the descreening by tiles (measured: k_desc_sites)
+constexpr int kDtItems = 2048;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;
@@ -58,15 +62,13 @@ enum : int {
 // per-overlap-tree accumulator layout (int64 fixed point per heavy atom)
 enum : int { TG_GB = 0, TG_VW = 3, TG_CAV = 6, TG_HB = 9, TG_N = 12 };
 
-// water-site record written by the placement kernel
+// a placed water site (one record per wave of the free-volume kernel, in LDS)
 struct WSite {
   float pos[3];
   float khb;
   int parent[4];
   int nparents;
   int type;
-  int stale0;        // atom whose spe the reference reads first (quirk Q3); -1: none (0)
-  int sys;           // system of the site
   float dpos[4][3][3];   // d pos_i / d x_{parent p, j}
 };
 
@@ -88,6 +90,9 @@ struct GridParams {
   int ncell;
 };
 
+// radius types whose descreening tables a block holds in LDS
+constexpr int kLdsTypes = 16;
+
 // cells per system grid (LDS histogram of the binning kernel)
 constexpr int kMaxCells = 8192;
 
@@ -99,6 +104,7 @@ struct SysInfo {
   int ws0, nws;         // water sites [ws0, ws0 + nws)
   int blk0, nblk;       // atom blocks [blk0, blk0 + nblk) (energy partials)
   int tile0, ntile;     // GB tile-pair energy slots [tile0, tile0 + ntile)
+  int dp0;              // its descreening tile sums (dt_on): tile t of atom a0 + k at dpart[dp0 + t n + k]
   float df;             // dielectric factor -0.5 (1/eps_in - 1/eps_out), FP32
   float rmax_heavy;     // largest heavy-atom R (cell size)
   double df64;          // same factor in FP64
@@ -145,7 +151,7 @@ struct SgTrain {
 };
 
 // work-queue heads (cleared by the ingest kernel of every call)
-enum : int { Q_DESC = 0, Q_GB, Q_CHAIN, Q_TREE_A, Q_TREE_B, Q_TREE_BA, Q_TREE_BB, Q_TREE_FA, Q_TREE_FB, Q_COUNT };
+enum : int { Q_DESC = 0, Q_GB, Q_CHAIN, Q_TREE_A, Q_TREE_B, Q_TREE_BA, Q_TREE_BB, Q_COUNT };
 // each queue has kQueueSpread heads, kQueueStride uints (64 bytes) apart: a
 // block takes its later items from head blockIdx mod kQueueSpread
 constexpr int kQueueSpread = 8, kQueueStride = 16;
@@ -157,7 +163,7 @@ struct Dev {
   int nsys;
   int ntypes;            // radius types (union over the systems)
   int cap;               // neighbour-list row capacity
-  int nws, nwsdef;       // water sites, HB-active atoms
+  int nws;               // water sites
   int options;
   const SysInfo *sys;
   const int *asys;       // system of each atom
@@ -180,6 +186,12 @@ struct Dev {
   int nrow_blocks;
   const int *row_perm;   // [nrow_blocks][rows] pack atom or -1
   const int4 *rblk;      // per block: radius type, system, hydrogen rows only, -
+  // descreening by tiles (dt_on; a call that few row blocks make up): items
+  // of a row block x 256 columns (row block, column range, place of the sums
+  // before adding the atom's number), and the tiles per run of k_born's sum
+  int dt_on, ndt_items, dt_run;
+  const int4 *dt_items;
+  float *dpart;
   // work items, sorted by decreasing size, taken from the queues by
   // persistent blocks: descreening / chain (row block, column range), GB
   // tile pairs (row range, column range; diagonal when they start together)
@@ -201,7 +213,8 @@ struct Dev {
   const int2 *ablk;      // atom blocks: [start, end) inside one system
   int nablk;
   const WsDef *wsdef;
-  const int *ws_stale0;  // per site: atom whose spe the first subtraction reads
+  const int2 *ws_site;   // per site: its HB-active atom's entry of wsdef, its number there
+  const int *ws_stale0;  // per site: atom whose spe the first subtraction reads (quirk Q3); -1: none (0)
   // per-call state
   float4 *pos;           // x, y, z, R
   GridParams *grid;      // [nsys]
@@ -228,8 +241,8 @@ struct Dev {
   unsigned long long *counters;        // [0] kept overlaps [1] evaluated [2] nbl entries [3] max row
                                        // [4] roots queued for the second breadth-first tier (pass A; pass B
                                        //     takes the same list), [5] unused
-                                       // [6], [7] roots queued for the depth-first walk (pass A, B)
-  int *tree_ovf;                       // [4][nh] those roots' heavy rows
+                                       // [6], [7] roots walked depth first (pass A, B)
+  int *tree_ovf;                       // [2][nh] heavy rows of the roots queued for the second tier, for pass B's depth-first walk
   unsigned char *tree_tier;            // [nh] pass A's first tier: 0 walked there, 1 queued for the next
   double *volumep_raw, *sa_raw, *sa_f, *sp, *spe, *psvol, *gammap;   // [n]
   float *sp_f, *spe_f;                 // FP32 copies for pair kernels
@@ -242,7 +255,6 @@ struct Dev {
   float *q2ab_f, *abrw_f;
   double *deru, *derv, *derus, *dervs, *derh;   // [n]
   float *deru_f, *derv_f, *derus_f, *dervs_f, *derh_f, *gammap_f;
-  WSite *ws;
   int *ws_ovf;                         // [nws] sites for the second free-volume launch
   int ws_cap1;                         // candidates the first launch takes (128; lower for tests)
   double *ws_part;                     // per-site energy khb*s
@@ -307,7 +319,7 @@ void launch_cells(const Dev &d, hipStream_t s);
 void launch_nblist(const Dev &d, hipStream_t s);
 void launch_tree(const Dev &d, const Tuning &t, int pass, hipStream_t s);
 // one tier of a pass: 0 breadth first, 1 breadth first with large levels (the
-// roots pass A's first tier queued), 2 depth first (after both others)
+// roots pass A's first tier queued; past those levels, depth first)
 void launch_tree_tier(const Dev &d, const Tuning &t, int pass, int tier, hipStream_t s);
 hipError_t prepare_tree();
 void launch_scale(const Dev &d, hipStream_t s);
@@ -318,8 +330,10 @@ void launch_q2ab(const Dev &d, hipStream_t s);
 void launch_chain(const Dev &d, const Tuning &t, hipStream_t s);
 void launch_uv(const Dev &d, hipStream_t s);
 hipError_t prepare_pairs(int ntypes);
-void launch_ws_place(const Dev &d, hipStream_t s);
 void launch_ws_free(const Dev &d, hipStream_t s);
+// descreening by tiles and the water sites' free volumes (dt_on)
+void launch_desc_sites(const Dev &d, hipStream_t s);
+hipError_t prepare_sites(int ntypes);
 void launch_sg_front(const Dev &d, hipStream_t s);
 void launch_sg_grad(const Dev &d, hipStream_t s);
 void launch_sg_audit(const Dev &d, hipStream_t s);
@@ -333,7 +347,6 @@ void launch_sg_adam(float *p, const float *g, float *mom, float *vel, float lr, 
 void launch_sg_pack(const float *p, unsigned short *w1, unsigned short *w2, unsigned short *w3, unsigned short *wt1,
                     unsigned short *wt2, unsigned short *wt3, hipStream_t s);
 void launch_final(const Dev &d, double *sp, double *br, double *sa, double *dgbdr, double *dvwdr,
-                  double *decav, double *dehb, hipStream_t s);
-void launch_energy(const Dev &d, double *energies, hipStream_t s);
+                  double *decav, double *dehb, double *energies, hipStream_t s);
 
 }  // namespace agb

@@ -41,17 +41,27 @@ __device__ __forceinline__ T incl_scan(T v) {
 __device__ __forceinline__ float lane63(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
-__device__ __forceinline__ double lane63(double v) {
+}  // namespace dpp
+
+// the value of one lane (wave-uniform index) in every lane
+__device__ __forceinline__ double lane_value(double v, int lane) {
   const long long b = __builtin_bit_cast(long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), 63);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), 63);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), lane);
   return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
 }
-}  // namespace dpp
+
+// order the LDS accesses of one wave (its LDS instructions execute in program
+// order; this keeps the compiler from moving them)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // the wave's total, in every lane (a fixed order of additions)
 __device__ __forceinline__ float wave_sum(float v) { return dpp::lane63(dpp::incl_scan(v)); }
-__device__ __forceinline__ double wave_sum(double v) { return dpp::lane63(dpp::incl_scan(v)); }
+__device__ __forceinline__ double wave_sum(double v) { return lane_value(dpp::incl_scan(v), 63); }
 __device__ __forceinline__ float wave_min(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o, 64));
@@ -283,6 +293,31 @@ __device__ __forceinline__ void fix_add(long long *p, double v) {
   if (v != 0.0) atomicAdd((unsigned long long *)p, (unsigned long long)__double2ll_rn(v * kFix));
 }
 __device__ __forceinline__ double fix_get(long long v) { return (double)v * kFixInv; }
+
+// ------------------------------------------------- U, V coefficients
+// deru = U/V_i, derus = df/(4pi) psvol deru, dervs = psvol derv/(4pi)
+// (kernels.c:861-875), from the chain rule's sums (which = 0: U, and H_i of
+// the water sites with it; 1: V)
+__device__ __forceinline__ void uv_coeffs(const Dev &d, int i, const SysInfo &S, int which, long long sum) {
+  const bool heavy = i < S.a0 + S.nh;
+  const double der = heavy ? fix_get(sum) / d.vols[i] : 0.0;
+  const double f4 = 1.0 / (4.0 * kPi);
+  if (which == 0) {
+    const double ders = S.df64 * f4 * d.psvol[i] * der, h = heavy ? fix_get(d.acc_derh[i]) : 0.0;
+    d.deru[i] = der;
+    d.derus[i] = ders;
+    d.derh[i] = h;
+    d.deru_f[i] = (float)der;
+    d.derus_f[i] = (float)ders;
+    d.derh_f[i] = (float)h;
+  } else {
+    const double ders = f4 * d.psvol[i] * der;
+    d.derv[i] = der;
+    d.dervs[i] = ders;
+    d.derv_f[i] = (float)der;
+    d.dervs_f[i] = (float)ders;
+  }
+}
 
 // ------------------------------------------------- overlap-volume switch
 // quintic smoothstep of the raw overlap volume on [0.01, 0.1]

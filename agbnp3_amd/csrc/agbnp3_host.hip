@@ -217,11 +217,15 @@ struct Pack {
   Dev d{};
   int device = 0;                      // the device the pack lives on
   int ntile = 0;                       // GB tile-pair energy slots of all systems
+  bool dt = false;                     // descreening by tiles (unless a surrogate is attached)
+  long long ndpart = 0;                // its tile sums
+  size_t call_ndpart() const { return dt ? (size_t)ndpart : 0; }
   // per-call working state (carve_call_state) and the host-API staging,
   // allocated by the first call that needs them (ensure_call_state), so an
   // instance evaluated only through agbnp3_ener_static never holds them
   void *call_block = nullptr;
   int call_nchain = 0;                 // chain-rule items the block's partial sums hold
+  size_t call_dpart = 0;               // descreening tile sums it holds
   double *dx = nullptr, *dy = nullptr, *dz = nullptr;      // coordinate staging (device)
   double *dout = nullptr;                                  // outputs: 15n + 7 nsys
   double *hstage = nullptr;                                // pinned host staging
@@ -547,9 +551,19 @@ int build_items(Pack &P) {
       for (int c = c0; c < c1; c += L) items.push_back(make_int4((int)k, c, std::min(c1, c + L), 0));
     }
     std::stable_sort(items.begin(), items.end(), [](const int4 &a, const int4 &b) { return a.z - a.y > b.z - b.y; });
-    return items;
+    return std::make_pair(items, L);
   };
-  std::vector<int4> desc = chunked(P.tune.desc_chunk, false);
+  const auto [desc, desc_cols] = chunked(P.tune.desc_chunk, false);
+  // the same by tiles (k_desc_sites), where these fill the chip a few times
+  // at most and the tables of every type fit in LDS
+  std::vector<int4> dt;
+  for (int k = 0; k < (int)rblk.size() && (int)dt.size() <= kDtItems; k++) {
+    const SysInfo &S = P.sinfo[rblk[k].y];
+    for (int c = 0, t = 0; c < S.nh; c += 256, t++)
+      dt.push_back(make_int4(k, S.a0 + c, S.a0 + std::min(S.nh, c + 256), S.dp0 + t * S.n - S.a0));
+  }
+  P.dt = P.tune.desc_chunk <= 0 && P.ntypes <= kLdsTypes && (int)dt.size() <= kDtItems;
+  if (!P.dt) dt.clear();
   // chain rule: pairs (P <= Q) of 256-atom blocks of one radius type, inside
   // one system, not both hydrogen-only
   std::vector<int> cperm;
@@ -670,7 +684,7 @@ int build_items(Pack &P) {
     gbs[k] = gb[k].second;
   }
   if (upload(P.item_allocs, &d.row_perm, row_perm) || upload(P.item_allocs, &d.rblk, rblk) ||
-      upload(P.item_allocs, &d.desc_items, desc) || upload(P.item_allocs, &d.chain_items, chain) ||
+      upload(P.item_allocs, &d.desc_items, desc) || upload(P.item_allocs, &d.dt_items, dt) || upload(P.item_allocs, &d.chain_items, chain) ||
       upload(P.item_allocs, &d.cperm, cperm) || upload(P.item_allocs, &d.cblk, cblk) ||
       upload(P.item_allocs, &d.ch_cstart, ch_cstart) || upload(P.item_allocs, &d.ch_contrib, ch_contrib) ||
       upload(P.item_allocs, &d.gb_items, gbi) || upload(P.item_allocs, &d.gb_eslot, gbs))
@@ -678,6 +692,8 @@ int build_items(Pack &P) {
   d.rows = rows;
   d.nrow_blocks = (int)rblk.size();
   d.ndesc_items = (int)desc.size();
+  d.ndt_items = (int)dt.size();
+  d.dt_run = desc_cols / 256;
   d.nchain_items = (int)chain.size();
   d.ncblk = (int)cblk.size();
   d.ngb_items = (int)gbi.size();
@@ -691,7 +707,7 @@ int build_items(Pack &P) {
 // on a 256-byte boundary of one block; with base == nullptr only the size is
 // computed.  The neighbour-list rows are `cap` wide.
 size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_, int nablk, int ntile, int cap,
-                        int nchain) {
+                        int nchain, size_t ndpart) {
   const size_t n = std::max(n_, 1), nh = std::max(nh_, 1), nws = std::max(nws_, 1);
   size_t off = 0;
   auto take = [&](auto *&ptr, size_t count) {
@@ -707,7 +723,7 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   take(d.cell_tmp, n);
   take(d.nne, nh);
   take(d.nbr, nh * (size_t)cap);
-  take(d.tree_ovf, 4 * nh);
+  take(d.tree_ovf, 2 * nh);
   take(d.tree_tier, nh);
   take(d.acc_vol, n);
   take(d.acc_sa, n);
@@ -727,28 +743,38 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   take(d.dcol, n);
   take(d.dcw, n);
   take(d.gb_epart, (size_t)std::max(ntile, 1));
-  take(d.ws, nws);
   take(d.ws_part, nws);
   take(d.ws_ovf, nws);
   take(d.epart, (size_t)EP_COUNT * std::max(nablk, 1));
+  take(d.dpart, ndpart);
   take(d.chpart, (size_t)nchain * 2 * 8 * 256);
   take(d.ch_done, (size_t)nchain);
   take(d.ch_flag, 4 * (size_t)std::max(d.ncblk, 1));
   return (off + 255) & ~(size_t)255;
 }
 
+// the second stream and its events
+int make_side(Pack &P) {
+  HIPCHK(hipStreamCreateWithFlags(&P.side, hipStreamNonBlocking));
+  HIPCHK(hipEventCreateWithFlags(&P.ev_fork, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&P.ev_join, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&P.ev_fork2, hipEventDisableTiming));
+  HIPCHK(hipEventCreateWithFlags(&P.ev_join2, hipEventDisableTiming));
+  return AGBNP_OK;
+}
+
 // the pack's own per-call state and host-API staging, on first use (calls
 // from agbnp3_ener_static use the library's static scratch instead)
 int ensure_call_state(Pack &P) {
   Dev &d = P.d;
-  if (P.call_block && d.nchain_items <= P.call_nchain) return AGBNP_OK;
-  if (P.call_block) {            // more chain-rule items than the block holds (a finer launch shape)
+  if (P.call_block && d.nchain_items <= P.call_nchain && P.call_ndpart() <= P.call_dpart) return AGBNP_OK;
+  if (P.call_block) {            // more items than the block holds (another launch shape)
     HIPCHK(hipStreamSynchronize(P.stream));
     if (P.side) HIPCHK(hipStreamSynchronize(P.side));
     (void)hipFree(P.call_block);
     P.call_block = nullptr;
   }
-  const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items);
+  const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
   const size_t nn = std::max(P.n, 1);
   const size_t stage = (18 * nn + 7 * (size_t)P.nsys + 8) * sizeof(double);   // outputs, inputs, status
   char *blk = nullptr;
@@ -758,7 +784,8 @@ int ensure_call_state(Pack &P) {
   }
   P.call_block = blk;
   P.call_nchain = d.nchain_items;
-  carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items);
+  P.call_dpart = P.call_ndpart();
+  carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
   double *st = reinterpret_cast<double *>(blk + bytes);
   P.dx = st;
   P.dy = st + nn;
@@ -766,6 +793,9 @@ int ensure_call_state(Pack &P) {
   P.dout = st + 3 * nn;
   HIPCHK(hipMemset(d.ws_part, 0, sizeof(double) * std::max(d.nws, 1)));
   if (!P.hstage) HIPCHK(hipHostMalloc((void **)&P.hstage, stage, hipHostMallocDefault));
+  // (a pack that is only copied into a batch, or called through
+  // agbnp3_ener_static, never comes here: no stream for it)
+  if (!P.side && P.n >= kSideAtoms && make_side(P) != AGBNP_OK) return AGBNP_ERR;
   return AGBNP_OK;
 }
 
@@ -793,7 +823,9 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
   std::vector<double> vols;
   std::vector<int2> ablk;
   std::vector<WsDef> wsdef;
+  std::vector<int2> ws_site;
   int a0 = 0, h0 = 0, ws0 = 0, blk0 = 0, tile0 = 0;
+  long long dp0 = 0;
   for (int b = 0; b < P.nsys; b++) {
     const Model &m = *ms[b];
     SysInfo S{};
@@ -802,6 +834,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
     S.blk0 = blk0; S.nblk = (m.natoms + 255) / 256;
     const int nb = (m.natoms + 255) / 256;
     S.tile0 = tile0; S.ntile = nb * (nb + 1) / 2;
+    S.dp0 = (int)std::min(dp0, (long long)INT_MAX);      // (read only where all of them fit: build_items)
     S.df64 = -0.5 * (1.0 / (double)m.eps_in - 1.0 / (double)m.eps_out);
     S.df = (float)S.df64;
     float rmax = 0.f;
@@ -825,13 +858,16 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
       w.atom += a0;
       for (int k = 0; k < 5; k++) w.p[k] += a0;
       w.first += ws0;
+      for (int k = 0; k < w.nsite; k++) ws_site.push_back(make_int2((int)wsdef.size(), k));
       wsdef.push_back(w);
     }
     for (int s : m.ws_stale0) ws_stale0.push_back(s >= 0 && s < m.natoms ? a0 + s : -1);
+    dp0 += (long long)m.natoms * ((m.nheavy + 255) / 256);
     a0 += m.natoms; h0 += m.nheavy; ws0 += m.nws; blk0 += S.nblk; tile0 += S.ntile;
   }
   P.n = a0;
   P.nh = h0;
+  P.ndpart = dp0;
   Dev &d = P.d;
   d = Dev{};
   d.n = P.n;
@@ -841,7 +877,6 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
   d.cap = P.cap;
   d.options = options;
   d.nws = ws0;
-  d.nwsdef = (int)wsdef.size();
   d.nablk = blk0;
   // water-site candidates the first free-volume launch takes: 128, or fewer
   // from AGBNP3_WS_FIRST_CAP (1..128) so tests can route sites to the second
@@ -868,7 +903,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
       upload(L, &d.galpha, galpha) || upload(L, &d.igamma, igamma) || upload(L, &d.sgamma, sgamma) ||
       upload(L, &d.ialpha, ialpha) || upload(L, &d.salpha, salpha) || upload(L, &d.hbcorr_f, hbcorr) ||
       upload(L, &d.vols, vols) || upload(L, &d.tbl, tb) || upload(L, &d.ctab, ctab) || upload(L, &d.ablk, ablk) ||
-      upload(L, &d.wsdef, wsdef) || upload(L, &d.ws_stale0, ws_stale0))
+      upload(L, &d.wsdef, wsdef) || upload(L, &d.ws_site, ws_site) || upload(L, &d.ws_stale0, ws_stale0))
     return AGBNP_ERR;
   P.ntile = tile0;
   // state that lives as long as the pack: status word, counters, queue heads
@@ -878,14 +913,9 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
   HIPCHK(hipMemset(d.counters, 0, sizeof(unsigned long long) * kCounters));
   HIPCHK(hipGetDevice(&P.device));
   HIPCHK(hipStreamCreateWithFlags(&P.stream, hipStreamNonBlocking));
-  if (P.n >= kForkAtoms) {              // only packs that fork (streams share few hardware queues)
-    HIPCHK(hipStreamCreateWithFlags(&P.side, hipStreamNonBlocking));
-    HIPCHK(hipEventCreateWithFlags(&P.ev_fork, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&P.ev_join, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&P.ev_fork2, hipEventDisableTiming));
-    HIPCHK(hipEventCreateWithFlags(&P.ev_join2, hipEventDisableTiming));
-  }
+  if (P.n >= kForkAtoms && make_side(P) != AGBNP_OK) return AGBNP_ERR;
   HIPCHK(prepare_pairs(P.ntypes));
+  HIPCHK(prepare_sites(P.ntypes));
   HIPCHK(prepare_tree());
   tune_apply_recorded(P);
   return build_items(P);
@@ -902,6 +932,7 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   d.cap = P.cap;
   d.skin = P.skin;
   d.reuse_every = P.reuse_every;
+  d.dt_on = P.dt && !d.sg_on;
   hipStream_t s = P.stream;
   const bool timed = !capturing && (P.options & AGBNP3_OPT_TIMING) != 0;
   int k = 0;
@@ -934,19 +965,21 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   mark("tree_volumes");
   launch_scale(d, s);
   mark("scale");
-  // with per-kernel timing every kernel stays on the one stream; below
-  // kForkAtoms atoms the fork and join cost more than the overlap saves
-  const bool fork = !timed && P.side && d.nws > 0 && d.n >= kForkAtoms;
+  // the water sites need only the self volumes: they share the tiled
+  // descreening's launch, or run on the second stream beside the descreening
+  // (with per-kernel timing every kernel stays on the one stream; below
+  // kForkAtoms atoms the fork and join cost more than the overlap saves)
+  const bool fork = !timed && P.side && d.nws > 0 && d.n >= kForkAtoms && !d.dt_on;
   if (fork) {
     HIPCHK(hipEventRecord(P.ev_fork, s));
     HIPCHK(hipStreamWaitEvent(P.side, P.ev_fork, 0));
-    launch_ws_place(d, P.side);
     launch_ws_free(d, P.side);
     HIPCHK(hipEventRecord(P.ev_join, P.side));
   }
   launch_sg_front(d, s);
   mark("sg_front");
-  launch_descreen(d, t, s);
+  if (d.dt_on) launch_desc_sites(d, s);
+  else launch_descreen(d, t, s);
   mark("descreen");
   launch_born(d, s);
   mark("born");
@@ -955,41 +988,34 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   launch_q2ab(d, s);
   mark("q2ab");
   launch_sg_audit(d, s);
+  if (fork) {
+    HIPCHK(hipStreamWaitEvent(s, P.ev_join, 0));
+  } else if (!d.dt_on) {
+    launch_ws_free(d, s);
+    mark("ws_free");
+  }
   launch_chain(d, t, s);
   mark("chain");
   launch_sg_grad(d, s);
   mark("sg_grad");
-  if (fork) {
-    HIPCHK(hipStreamWaitEvent(s, P.ev_join, 0));
-  } else {
-    launch_ws_place(d, s);
-    mark("ws_place");
-    launch_ws_free(d, s);
-    mark("ws_free");
-  }
   launch_uv(d, s);
   mark("uv");
   // derivative pass: its second tier takes the roots pass A's first tier
-  // queued, so it does not wait for the first tier and runs beside it (the
-  // largest trees start at once instead of after the rest); the depth-first
-  // tier follows both.  The energy reduction, whose partials are final here,
-  // follows the second tier on the second stream.
+  // queued, so it does not wait for the first tier and runs beside it on the
+  // second stream (the largest trees start at once instead of after the rest)
   const bool fork2 = !timed && P.side;
   if (fork2) {
     HIPCHK(hipEventRecord(P.ev_fork2, s));
     HIPCHK(hipStreamWaitEvent(P.side, P.ev_fork2, 0));
     launch_tree_tier(d, t, 1, 1, P.side);
-    launch_energy(d, energies, P.side);
     HIPCHK(hipEventRecord(P.ev_join2, P.side));
     launch_tree_tier(d, t, 1, 0, s);
     HIPCHK(hipStreamWaitEvent(s, P.ev_join2, 0));
-    launch_tree_tier(d, t, 1, 2, s);
   } else {
     launch_tree(d, t, 1, s);
   }
   mark("tree_derivs");
-  launch_final(d, sp, br, sa, dgbdr, dvwdr, decav, dehb, s);
-  if (!fork2) launch_energy(d, energies, s);
+  launch_final(d, sp, br, sa, dgbdr, dvwdr, decav, dehb, energies, s);
   mark("final");
   HIPCHK(hipGetLastError());
   return AGBNP_OK;
@@ -1613,13 +1639,15 @@ int agbnp3_ener_static(int tag, const double *x, const double *y, const double *
   char *base = nullptr;
   if (scratch_base(dev, &base) != AGBNP_OK) return AGBNP_ERR;
   Dev d = P.d;
-  const size_t need = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items);
+  const size_t need = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items,
+                                       P.call_ndpart());
   if (need > (size_t)AGBNP3_STATIC_SCRATCH_BYTES) {
     errprint("agbnp3_ener_static(): tag %d (%d atoms) needs %zu bytes of per-call state; the static scratch "
              "holds %zu (use agbnp3_ener_device).\n", tag, P.n, need, (size_t)AGBNP3_STATIC_SCRATCH_BYTES);
     return AGBNP_ERR;
   }
-  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items);
+  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items,
+                                       P.call_ndpart());
   // no per-kernel timing events here (creating them allocates)
   const int saved = P.options;
   P.options &= ~AGBNP3_OPT_TIMING;

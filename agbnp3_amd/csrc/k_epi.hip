@@ -25,11 +25,36 @@ __device__ void block_partials(const Dev &d, const int *slots, const double *v, 
   }
 }
 
+// near-pair total and longest row (counters 2, 3): one add and one max per
+// block rather than per row (same-address atomics serialise in L2).  The
+// grid has at least one block per 256 heavy rows.
+__device__ __forceinline__ void nbl_counts(const Dev &d) {
+  __shared__ unsigned ssum[kEpi / 64], smax[kEpi / 64];
+  const int h = blockIdx.x * kEpi + threadIdx.x;
+  if (blockIdx.x * kEpi >= d.nh) return;             // block-uniform
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  unsigned sum = h < d.nh ? (unsigned)d.nne[h] : 0u, mx = sum;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_xor((int)sum, o, 64);
+    mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
+  }
+  if (lane == 0) { ssum[w] = sum; smax[w] = mx; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned t = 0, m = 0;
+    for (int q = 0; q < kEpi / 64; q++) { t += ssum[q]; m = max(m, smax[q]); }
+    if (t) atomicAdd(&d.counters[2], (unsigned long long)t);
+    if (m) atomicMax(&d.counters[3], (unsigned long long)m);
+  }
+}
+
 // ------------------------------------------------------- scaling factors
 // agbnp3_scaling_factors (agbnp3_utils.c:524-613) with agbnp3_swf_area
 // (agbnp3.c:1104-1117); E_cav, E_corr_cav, molecular volume
 // (agbnp3.c:1390-1411)
 __global__ __launch_bounds__(kEpi) void k_scale(Dev d) {
+  nbl_counts(d);
   const int2 blk = d.ablk[blockIdx.x];
   const int i = blk.x + threadIdx.x;
   double ecav = 0.0, ecorr = 0.0, mv = 0.0;
@@ -91,7 +116,23 @@ __global__ __launch_bounds__(kEpi) void k_born(Dev d) {
   const int i = blk.x + threadIdx.x;
   double evdw = 0.0, ecorr = 0.0, eself = 0.0;
   if (i < blk.y) {
-    double s = fix_get(d.acc_beta[i]);
+    double s;
+    if (d.dt_on) {
+      // the tiles' FP32 sums, in runs of the columns that one of k_descreen's
+      // items covers: added in FP64, rounded to the fixed point once per run
+      const SysInfo &S = d.sys[d.asys[i]];
+      const int nt = (S.nh + 255) / 256;
+      const float *p = d.dpart + S.dp0 + (i - S.a0);
+      long long sum = 0;
+      for (int t0 = 0; t0 < nt; t0 += d.dt_run) {
+        double a = 0.0;
+        for (int t = t0; t < min(t0 + d.dt_run, nt); t++) a += (double)p[(size_t)t * S.n];
+        sum += __double2ll_rn(a * kFix);
+      }
+      s = fix_get(sum);
+    } else {
+      s = fix_get(d.acc_beta[i]);
+    }
     if (d.sg_on && d.sys_sg[d.asys[i]]) {
       // surrogate call: the model's sum plus the correction of the last
       // anchor (an atom out of the training window keeps its descreening
@@ -162,43 +203,70 @@ void launch_q2ab(const Dev &d, hipStream_t s) {
 }
 
 // ------------------------------------------------------ U, V coefficients
-// deru = U/V_i, derus = df/(4pi) psvol deru, dervs = psvol derv/(4pi)
-// (kernels.c:861-875); H_i from the water-site pass
+// for calls whose chain-rule sums k_chain_sum does not finish: a surrogate's
+// gradient pass adds to them, or there are none (no heavy atoms)
 __global__ __launch_bounds__(kEpi) void k_uv(Dev d) {
   const int i = blockIdx.x * kEpi + threadIdx.x;
   if (i >= d.n) return;
   const SysInfo &S = d.sys[d.asys[i]];
-  const bool heavy = i < S.a0 + S.nh;
-  double U = 0.0, V = 0.0;
-  if (heavy) {
-    U = fix_get(d.acc_ch[8 * (size_t)i + 6]);
-    V = fix_get(d.acc_ch[8 * (size_t)i + 7]);
-  }
-  const double vol = heavy ? d.vols[i] : 1.0;
-  const double du = heavy ? U / vol : 0.0, dv = heavy ? V / vol : 0.0;
-  const double f4 = 1.0 / (4.0 * kPi);
-  d.deru[i] = du;
-  d.derv[i] = dv;
-  d.derus[i] = S.df64 * f4 * d.psvol[i] * du;
-  d.dervs[i] = f4 * d.psvol[i] * dv;
-  d.derh[i] = heavy ? fix_get(d.acc_derh[i]) : 0.0;
-  d.deru_f[i] = (float)d.deru[i];
-  d.derv_f[i] = (float)d.derv[i];
-  d.derus_f[i] = (float)d.derus[i];
-  d.dervs_f[i] = (float)d.dervs[i];
-  d.derh_f[i] = (float)d.derh[i];
+  for (int q = 0; q < 2; q++) uv_coeffs(d, i, S, q, d.acc_ch[8 * (size_t)i + 6 + q]);
 }
 
 void launch_uv(const Dev &d, hipStream_t s) {
+  if (!d.sg_on && d.nchain_items) return;
   hipLaunchKernelGGL(k_uv, dim3((d.n + kEpi - 1) / kEpi), dim3(kEpi), 0, s, d);
+}
+
+// ---------------------------------------------------------------- energies
+// fixed-order reduction of the per-block energy partials, GB tile pairs and
+// site energies; one workgroup per system, energies[7 * system + k]; they need only the
+// partials, so they run in the final launch beside the gradients
+__device__ __forceinline__ void system_energies(const Dev &d, int sys, double *energies) {
+  __shared__ double red[EP_COUNT][4];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const SysInfo S = d.sys[sys];
+  double acc[EP_COUNT];
+  for (int k = 0; k < EP_COUNT; k++) acc[k] = 0.0;
+  // thread t sums partials t, t + 256, t + 512, ... in that order: a fixed
+  // order that depends only on the system's own counts, with coalesced loads
+  // (the loops unrolled so that several loads are in flight)
+  for (int k = 0; k < EP_PAIR; k++)
+#pragma unroll 8
+    for (int b = t; b < S.nblk; b += 256) acc[k] += d.epart[(size_t)k * d.nablk + S.blk0 + b];
+  // tile partials hold each unordered pair once; E_pair = 2 df sum_{i<j} q_i q_j / f
+#pragma unroll 8
+  for (int b = t; b < S.ntile; b += 256) acc[EP_PAIR] += 2.0 * S.df64 * d.gb_epart[S.tile0 + b];
+#pragma unroll 8
+  for (int b = t; b < S.nws; b += 256) acc[EP_HB] += d.ws_part[S.ws0 + b];
+  for (int k = 0; k < EP_COUNT; k++) {
+    const double s = wave_sum(acc[k]);
+    if (lane == 0) red[k][w] = s;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double e[EP_COUNT];
+    for (int k = 0; k < EP_COUNT; k++) e[k] = red[k][0] + red[k][1] + red[k][2] + red[k][3];
+    double *o = energies + 7 * (size_t)sys;
+    o[0] = kTokcal * (e[EP_SELF] + e[EP_PAIR]);
+    o[1] = e[EP_VDW];
+    o[2] = e[EP_CORR_VDW];
+    o[3] = e[EP_CAV];
+    o[4] = e[EP_CORR_CAV];
+    o[5] = e[EP_HB];
+    o[6] = e[EP_MOLVOL];
+  }
 }
 
 // ----------------------------------------------------------- final output
 // gradients: GB = 332 (pair + chain + tree), vdW = chain + tree,
 // cavity = tree, HB = direct + tree (agbnp3.c:1718-1786); caller order
 __global__ __launch_bounds__(kEpi) void k_final(Dev d, double *sp, double *br, double *sa, double *dgbdr,
-                                                double *dvwdr, double *decav, double *dehb) {
-  const int i = blockIdx.x * kEpi + threadIdx.x;
+                                                double *dvwdr, double *decav, double *dehb, double *energies) {
+  if ((int)blockIdx.x < d.nsys) {                    // the first blocks: a system's energies each
+    system_energies(d, blockIdx.x, energies);
+    return;
+  }
+  const int i = (blockIdx.x - d.nsys) * kEpi + threadIdx.x;
   if (i >= d.n) return;
   const int e = d.int2ext[i];
   const SysInfo &S = d.sys[d.asys[i]];
@@ -232,54 +300,10 @@ __global__ __launch_bounds__(kEpi) void k_final(Dev d, double *sp, double *br, d
   sa[e] = heavy ? d.sa_f[i] : 0.0;
 }
 
-// fixed-order reduction of the per-block energy partials, GB tile pairs and
-// site energies; one workgroup per system, energies[7 * system + k]
-__global__ __launch_bounds__(256) void k_energy(Dev d, double *energies) {
-  __shared__ double red[EP_COUNT][4];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const SysInfo S = d.sys[blockIdx.x];
-  double acc[EP_COUNT];
-  for (int k = 0; k < EP_COUNT; k++) acc[k] = 0.0;
-  // thread t sums partials t, t + 256, t + 512, ... in that order: a fixed
-  // order that depends only on the system's own counts, with coalesced loads
-  // (the loops unrolled so that several loads are in flight)
-  for (int k = 0; k < EP_PAIR; k++)
-#pragma unroll 8
-    for (int b = t; b < S.nblk; b += 256) acc[k] += d.epart[(size_t)k * d.nablk + S.blk0 + b];
-  // tile partials hold each unordered pair once; E_pair = 2 df sum_{i<j} q_i q_j / f
-#pragma unroll 8
-  for (int b = t; b < S.ntile; b += 256) acc[EP_PAIR] += 2.0 * S.df64 * d.gb_epart[S.tile0 + b];
-#pragma unroll 8
-  for (int b = t; b < S.nws; b += 256) acc[EP_HB] += d.ws_part[S.ws0 + b];
-  for (int k = 0; k < EP_COUNT; k++) {
-    const double s = wave_sum(acc[k]);
-    if (lane == 0) red[k][w] = s;
-  }
-  __syncthreads();
-  if (t == 0) {
-    double e[EP_COUNT];
-    for (int k = 0; k < EP_COUNT; k++) e[k] = red[k][0] + red[k][1] + red[k][2] + red[k][3];
-    double *o = energies + 7 * (size_t)blockIdx.x;
-    o[0] = kTokcal * (e[EP_SELF] + e[EP_PAIR]);
-    o[1] = e[EP_VDW];
-    o[2] = e[EP_CORR_VDW];
-    o[3] = e[EP_CAV];
-    o[4] = e[EP_CORR_CAV];
-    o[5] = e[EP_HB];
-    o[6] = e[EP_MOLVOL];
-  }
-}
-
 void launch_final(const Dev &d, double *sp, double *br, double *sa, double *dgbdr, double *dvwdr, double *decav,
-                  double *dehb, hipStream_t s) {
-  hipLaunchKernelGGL(k_final, dim3((d.n + kEpi - 1) / kEpi), dim3(kEpi), 0, s, d, sp, br, sa, dgbdr, dvwdr, decav,
-                     dehb);
-}
-
-// the energies need only the energy partials, which are final once the water
-// sites and the pair kernels are done (before the derivative pass)
-void launch_energy(const Dev &d, double *energies, hipStream_t s) {
-  hipLaunchKernelGGL(k_energy, dim3(d.nsys), dim3(256), 0, s, d, energies);
+                  double *dehb, double *energies, hipStream_t s) {
+  hipLaunchKernelGGL(k_final, dim3(d.nsys + (d.n + kEpi - 1) / kEpi), dim3(kEpi), 0, s, d, sp, br, sa, dgbdr, dvwdr,
+                     decav, dehb, energies);
 }
 
 }  // namespace agb

@@ -1,13 +1,15 @@
 // Hydrogen-bond (water-site) term.
 //
-// Placement: one thread per HB-active atom writes its 1-4 pseudo-atoms of
-// radius 1.4 A (straight into their records: a private copy indexed by a
-// run-time parent number would live in scratch memory) and the Jacobians dpos[p][i][j] = d pos_i / d x_{parent p, j}
-// for the eight geometries of the reference (agbnp3.c:2014-3761).  Which
-// atoms get which geometry is fixed by the topology and decided on the host
-// when the instance is created.
+// One wavefront per site.  Its first lane places the site, a pseudo-atom of
+// radius 1.4 A, and forms the Jacobians dpos[p][i][j] = d pos_i / d x_{parent
+// p, j} of its geometry, one of the reference's eight (agbnp3.c:2014-3761),
+// in the wave's LDS record.  Which atoms get which geometry is fixed by the
+// topology and decided on the host when the instance is created.  (A launch
+// of its own that wrote every site's 240-byte record to memory, one thread
+// per HB-active atom, took 12 us at 2,000 atoms, its wave running all eight
+// geometries in turn, and 16 us at 25,000.)
 //
-// Free volume: one wavefront per site.  Heavy atoms passing the FP32 test
+// Free volume: heavy atoms passing the FP32 test
 // d2 < ((R + 1.4) * 1.6)^2 are collected from the cell grid and sorted by
 // atom index; their Gaussian overlaps are evaluated lane-parallel, then one
 // lane walks them in index order exactly as the reference does
@@ -17,6 +19,8 @@
 // given by the previous site's last parent); AGBNP3_OPT_HB_FIXED uses the
 // partner's own.  E_HB = sum khb s(V_free / V_w; 0.65, 1).
 #include <float.h>
+
+#include <type_traits>
 
 #include "agb_common.h"
 #include "agb_device.h"
@@ -64,22 +68,18 @@ __device__ __forceinline__ void site_init(WSite &w, f3 pos, float khb, int type,
       for (int j = 0; j < 3; j++) w.dpos[p][i][j] = 0.f;
 }
 
-__global__ __launch_bounds__(256) void k_ws_place(Dev d) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= d.nwsdef) return;
-  const WsDef def = d.wsdef[t];
+// Site number `which` of HB-active atom `def`, into record w
+__device__ void ws_place_site(const Dev &d, const WsDef &def, int which, WSite &w) {
   const float L = kHbLength;
   const int A = def.atom;
   const f3 xa = ld3(d.pos[A]);
   const float khb = d.hbcorr_f[A];
-  WSite *W = d.ws + def.first;
   switch (def.kind) {
     case WS_POLARH: {     // agbnp3_place_wat_hydrogen (agbnp3.c:2098-2150)
       const int D = def.p[1];
       const f3 xd = ld3(d.pos[D]);
       float inv;
       const f3 u = unit(xa - xd, inv);
-      WSite &w = W[0];
       site_init(w, xd + L * u, khb, 1, 2, A, D, -1, -1);
       const float c = L * inv;
       for (int i = 0; i < 3; i++)
@@ -95,10 +95,10 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
       const int R = def.p[1], R1 = def.p[2], R2 = def.p[3];
       const f3 xr = ld3(d.pos[R]);
       const int type = def.kind == WS_TRIGONAL1 ? 11 : 30;
-      for (int s = 0; s < 2; s++) {
+      if (which < 2) {
+        const int s = which;
         float inv;
         const f3 u = unit(ld3(d.pos[s == 0 ? R1 : R2]) - xr, inv);
-        WSite &w = W[s];
         site_init(w, xa - L * u, khb, type, 4, A, R, R1, R2);
         const float c = L * inv;
         for (int i = 0; i < 3; i++) {
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
           }
         }
       }
-      if (def.kind == WS_TRIGONAL_S) {   // agbnp3_place_wat_trigonal_s (agbnp3.c:2590-2697)
+      if (which >= 2) {   // agbnp3_place_wat_trigonal_s (agbnp3.c:2590-2697)
         const float cs = 0.5f, sn = 0.866025f;
         const f3 dx0 = xa - xr, dx1 = ld3(d.pos[R1]) - xr;
         float d0i, d2i;
@@ -124,9 +124,8 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
           t1[i][0] = a.x; t1[i][1] = a.y; t1[i][2] = a.z;
           t2[i][0] = b.x; t2[i][1] = b.y; t2[i][2] = b.z;
         }
-        for (int s = 0; s < 2; s++) {
-          const float sg = s == 0 ? 1.f : -1.f;
-          WSite &w = W[2 + s];
+        {
+          const float sg = which == 2 ? 1.f : -1.f;
           site_init(w, xa + L * (cs * uin + (sg * sn) * uout), khb, 30, 4, A, R, R1, R2);
           for (int i = 0; i < 3; i++)
             for (int j = 0; j < 3; j++) {
@@ -156,9 +155,8 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
       mm3(P, J1, M1);
       mm3(P, J2, M2);
       const float dn = dd / nun;
-      for (int s = 0; s < 2; s++) {
-        const float sg = s == 0 ? 1.f : -1.f;
-        WSite &w = W[s];
+      {
+        const float sg = which == 0 ? 1.f : -1.f;
         site_init(w, xa + (sg * dd) * nu, khb, 13, 4, A, R1, R2, R3);
         for (int i = 0; i < 3; i++)
           for (int j = 0; j < 3; j++) {
@@ -176,18 +174,21 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
       f3 dk[3];
       float inv[3];
       f3 sum = {0.f, 0.f, 0.f};
-      for (int k = 0; k < nr; k++) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        if (k >= nr) break;
         dk[k] = unit(ld3(d.pos[def.p[1 + k]]) - xa, inv[k]);
         sum = sum + dk[k];
       }
       float iw;
       const f3 dw = unit(sum, iw);
-      WSite &w = W[0];
       site_init(w, xa - L * dw, khb, nr == 2 ? 12 : 23, nr + 1, A, def.p[1], def.p[2], nr == 3 ? def.p[3] : -1);
       float Dw[3][3];
       unit_der(dw, iw, Dw);
       for (int i = 0; i < 3; i++) w.dpos[0][i][i] = 1.f;
-      for (int k = 0; k < nr; k++) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        if (k >= nr) break;
         float Dk[3][3], M[3][3];
         unit_der(dk[k], inv[k], Dk);
         mm3(Dw, Dk, M);
@@ -219,9 +220,8 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
         t1[i][0] = a.x; t1[i][1] = a.y; t1[i][2] = a.z;
         t2[i][0] = b.x; t2[i][1] = b.y; t2[i][2] = b.z;
       }
-      for (int s = 0; s < 2; s++) {
-        const float sg = s == 0 ? 1.f : -1.f;
-        WSite &w = W[s];
+      {
+        const float sg = which == 0 ? 1.f : -1.f;
         site_init(w, xa + L * (cs * pin + (sg * sn) * out), khb, 22, 3, A, R1, R2, -1);
         for (int i = 0; i < 3; i++)
           for (int j = 0; j < 3; j++) {
@@ -237,11 +237,11 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
     case WS_TETRAHEDRAL1: {   // agbnp3_place_wat_tetrahedral1_one (agbnp3.c:3689-3761)
       const int R = def.p[1];
       const f3 xr = ld3(d.pos[R]);
-      for (int s = 0; s < 3; s++) {
+      {
+        const int s = which;
         const int Rk = def.p[2 + s];
         float inv;
         const f3 u = unit(ld3(d.pos[Rk]) - xr, inv);
-        WSite &w = W[s];
         site_init(w, xa - L * u, khb, 21, 3, A, R, Rk, -1);
         const float c = L * inv;
         for (int i = 0; i < 3; i++) {
@@ -256,24 +256,14 @@ __global__ __launch_bounds__(256) void k_ws_place(Dev d) {
       break;
     }
   }
-  const int sys = d.asys[A];
-  for (int s = 0; s < def.nsite; s++) {
-    W[s].stale0 = d.ws_stale0[def.first + s];
-    W[s].sys = sys;
-  }
-}
-
-void launch_ws_place(const Dev &d, hipStream_t s) {
-  if (d.nwsdef == 0) return;
-  hipLaunchKernelGGL(k_ws_place, dim3((d.nwsdef + 255) / 256), dim3(256), 0, s, d);
 }
 
 // ------------------------------------------------------------ free volume
 // One wave per site, WAVES sites per block, candidate buffers of CAP atoms.
-// The first launch (4 x 128) lists the sites with more candidates than it
-// holds (up to d.ws_cap1, 128 unless lowered for tests) for the second
+// The first pass (4 x 128) leaves the sites with more candidates than it
+// holds (up to d.ws_cap1, 128 unless lowered for tests) for a second
 // (1 x 1024), which takes them one per wave; the per-site arithmetic is the
-// same in both, so results do not depend on which launch took a site.  A
+// same in both, so results do not depend on which pass took a site.  A
 // site with more than 1024 candidates fails the call.
 constexpr int kWsWaves = 4;
 constexpr int kWsCap = 128, kWsCapBig = 1024;
@@ -284,30 +274,41 @@ struct WsLds {
   int cs[WAVES][CAP];        // sorted candidate atoms
   float cvp[WAVES][CAP];
   float cgw[WAVES][CAP][3];
-  int ckeep[WAVES][CAP];
-  double cspe[WAVES][CAP];   // spe of the sorted candidates (read in parallel)
-  double sfree[WAVES];
+  double cspe[WAVES][CAP];   // spe of the sorted candidates
+  unsigned long long keep[WAVES][CAP / 64];   // which of them the walk took
+  WSite rec[WAVES];
 };
 
-// the free volume of one site and its derivatives (wave w of the block;
-// every wave of the block calls it together: it holds block barriers)
-template <int WAVES, int CAP, bool LIST>
-__device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
+// what becomes of a site with more candidates than CAP: listed for the second
+// launch, a failed call, or returned to the caller
+enum : int { WS_LIST = 0, WS_FAIL = 1, WS_RETURN = 2 };
+
+// The free volume of one site and its derivatives by one wave with the LDS of
+// slot w (every wave of the block calls it together: it holds block barriers;
+// a wave without a site, site >= nws, touches no LDS).  True when the site had
+// more candidates than this pass holds (it then adds nothing).
+template <int WAVES, int CAP, int MORE>
+__device__ bool ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site, int w) {
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   const bool active = site < d.nws;
+  if (active && lane == 0) {
+    const int2 ds = d.ws_site[site];
+    ws_place_site(d, d.wsdef[ds.x], ds.y, L.rec[w]);
+  }
+  __syncthreads();
   // the fields every lane uses, in registers; the parents and Jacobians are
   // read from the record only by the lanes that project onto them
-  const WSite *Wg = d.ws + (active ? site : 0);
+  const WSite *Wg = &L.rec[w];
   float wpos[3] = {0.f, 0.f, 0.f};
   float wkhb = 0.f;
   int wstale0 = -1, wnparents = 0, sys = 0;
   if (active) {
     wpos[0] = Wg->pos[0]; wpos[1] = Wg->pos[1]; wpos[2] = Wg->pos[2];
     wkhb = Wg->khb;
-    wstale0 = Wg->stale0;
     wnparents = Wg->nparents;
-    sys = Wg->sys;
+    wstale0 = d.ws_stale0[site];
+    sys = d.asys[Wg->parent[0]];
   }
   const GridParams g = d.grid[sys];
   const int *cstart = d.cell_start + (size_t)sys * (kMaxCells + 1);
@@ -340,18 +341,15 @@ __device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
       cnt += __popcll(m);
     }
   }
-  // a site past this launch's buffers: listed for the second launch (first
-  // launch), or a failed call (second); either way it adds nothing here
-  bool mine = active;
-  if (cnt > (LIST ? CAP : min(CAP, d.ws_cap1))) {
-    if (lane == 0) {
-      if (LIST) {
-        atomicOr(d.status, ST_WS_OVERFLOW);
-      } else {
-        const unsigned q = atomicAdd(&d.counters[kCountWs], 1ull);
-        d.ws_ovf[q] = site;
-      }
+  // a site past these buffers adds nothing here
+  bool mine = active, more = false;
+  if (cnt > (MORE == WS_FAIL ? CAP : min(CAP, d.ws_cap1))) {
+    if (MORE == WS_FAIL && lane == 0) atomicOr(d.status, ST_WS_OVERFLOW);
+    if (MORE == WS_LIST && lane == 0) {
+      const unsigned q = atomicAdd(&d.counters[kCountWs], 1ull);
+      d.ws_ovf[q] = site;
     }
+    more = true;
     mine = false;
     cnt = 0;
   }
@@ -360,6 +358,7 @@ __device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
   for (int e = lane; e < cnt; e += 64) {
     const int je = L.cj[w][e];
     int rank = 0;
+#pragma unroll 8
     for (int f = 0; f < cnt; f++) rank += L.cj[w][f] < je;
     L.cs[w][rank] = je;
   }
@@ -390,29 +389,39 @@ __device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
   }
   __syncthreads();
   const double vw = 4.0 / 3.0 * kPi * (double)kHbRadius * (double)kHbRadius * (double)kHbRadius;
-  if (lane == 0 && mine) {
-    // the reference's sequential walk with early stop (kernels.c:2818-2860)
+  if (!mine) return more;                // (no barrier follows)
+  // The reference's sequential walk with early stop (kernels.c:2818-2860), 64
+  // candidates at a time: the terms spe V' in parallel (by default the spe of
+  // the candidate taken before, the site's stale partner's first), then one
+  // subtraction after the other in index order, each term read from its lane
+  // into every lane.  (Walked by one lane out of LDS, a site's ~50 candidates
+  // cost it more than everything else together.)
+  double freev = vw;
+  {
     const bool fixed = (d.options & 1) != 0;
-    double freev = vw;
     const double cutoff = (double)kHbSwA0 * vw;
-    // spe of the previously kept atom (the site's own stale partner first)
-    double stale_sp = wstale0 >= 0 ? d.spe[wstale0] : 0.0;
-    for (int e = 0; e < cnt; e++) L.ckeep[w][e] = 0;
-    for (int e = 0; e < cnt; e++) {
-      if (!(freev > cutoff)) break;
-      const float vp = L.cvp[w][e];
-      if (vp > 0.f) {
-        const double spk = L.cspe[w][e];
-        freev -= (fixed ? spk : stale_sp) * (double)vp;
-        stale_sp = spk;
-        L.ckeep[w][e] = 1;
+    double stale = wstale0 >= 0 ? d.spe[wstale0] : 0.0;
+    for (int base = 0; base < cnt; base += 64) {
+      const int e = base + lane;
+      const float vp = e < cnt ? L.cvp[w][e] : 0.f;
+      const double spk = e < cnt ? L.cspe[w][e] : 0.0;
+      const unsigned long long taken = __ballot(vp > 0.f);      // (as far as the walk goes)
+      const unsigned long long below = taken & ((1ull << lane) - 1ull);
+      const double before = __shfl(spk, below ? 63 - __clzll(below) : 0, 64);
+      const double term = (fixed ? spk : (below ? before : stale)) * (double)vp;
+      unsigned long long todo = taken, keep = 0ull;
+      while (todo != 0ull && __ballot(freev > cutoff) != 0ull) {  // (the same in every lane)
+        const int b = __builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        keep |= 1ull << b;
+        freev -= lane_value(term, b);
       }
+      if (lane == 0) L.keep[w][base / 64] = keep;
+      if (taken != 0ull) stale = lane_value(spk, 63 - __clzll(taken));
     }
-    L.sfree[w] = freev;
   }
-  __syncthreads();
-  if (!mine) return;                     // (no barrier follows)
-  const double spw = L.sfree[w] / vw;
+  wave_sync();
+  const double spw = freev / vw;
   double fp = 0.0, sw;
   {
     const double xa = kHbSwA, xb = kHbSwB;
@@ -428,7 +437,7 @@ __device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
   if (lane == 0) d.ws_part[site] = (double)wkhb * sw;
   double jw[3] = {0.0, 0.0, 0.0};
   for (int e = lane; e < cnt; e += 64) {
-    if (!L.ckeep[w][e]) continue;
+    if (!((L.keep[w][e / 64] >> lane) & 1ull)) continue;
     const int k = L.cs[w][e];
     const double spk = L.cspe[w][e];
 #pragma unroll
@@ -446,27 +455,153 @@ __device__ void ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site) {
     const double g = jw[0] * Wg->dpos[p][0][j] + jw[1] * Wg->dpos[p][1][j] + jw[2] * Wg->dpos[p][2][j];
     fix_add(&d.acc_hb[3 * (size_t)Wg->parent[p] + j], g);
   }
+  return false;
 }
 
-template <int WAVES, int CAP, bool LIST>
+template <int WAVES, int CAP, int MORE>
 __global__ __launch_bounds__(64 * WAVES) void k_ws_free(Dev d) {
   __shared__ WsLds<WAVES, CAP> L;
-  if (!LIST) {
-    ws_free_site<WAVES, CAP, false>(d, L, (int)blockIdx.x * WAVES + (int)(threadIdx.x >> 6));
+  const int w = (int)(threadIdx.x >> 6);
+  if (MORE == WS_LIST) {
+    ws_free_site<WAVES, CAP, MORE>(d, L, (int)blockIdx.x * WAVES + w, w);
     return;
   }
   const int nlist = (int)d.counters[kCountWs];
   for (int item = blockIdx.x; item < nlist; item += gridDim.x) {
-    ws_free_site<WAVES, CAP, true>(d, L, d.ws_ovf[item]);
+    ws_free_site<WAVES, CAP, MORE>(d, L, d.ws_ovf[item], w);
     __syncthreads();                     // the next listed site reuses the buffers
   }
 }
 
 void launch_ws_free(const Dev &d, hipStream_t s) {
   if (d.nws == 0) return;
-  hipLaunchKernelGGL((k_ws_free<kWsWaves, kWsCap, false>), dim3((d.nws + kWsWaves - 1) / kWsWaves),
+  hipLaunchKernelGGL((k_ws_free<kWsWaves, kWsCap, WS_LIST>), dim3((d.nws + kWsWaves - 1) / kWsWaves),
                      dim3(64 * kWsWaves), 0, s, d);
-  hipLaunchKernelGGL((k_ws_free<1, kWsCapBig, true>), dim3(std::min(d.nws, 64)), dim3(64), 0, s, d);
+  hipLaunchKernelGGL((k_ws_free<1, kWsCapBig, WS_FAIL>), dim3(std::min(d.nws, 64)), dim3(64), 0, s, d);
+}
+
+// ------------------------------------- descreening by tiles, beside the sites
+// The descreening sums (k_descreen) of small and middle-sized calls, whose
+// items are too few to fill the chip.  There a wave walks 512 columns, four
+// behind each scalar load, a branch and an LDS wait per column: that one
+// wave's latency, 100 us, is the launch's at 2,000 and at 8,000 atoms alike.
+// Here an item is a row block against one 256-column tile; its columns and
+// tables come to LDS in one round of vector loads, and the lookups of eight
+// columns are in flight together.  A row's FP32 sum runs over the tile's
+// columns in the same order, with the same operations, as k_descreen's, and
+// leaves as a plain store of the tile's sum (k_born adds the tiles).  The
+// water sites' free volumes, which need only the self volumes too, take the
+// launch's first blocks.
+// Descreening and sites, before (three launches) and after: 61 atoms 30 -> 10
+// us, 2,000 142 -> 22, 6,000 134 -> 35, 11,000 130 -> 72, 14,000 132 -> 98
+// (bound there by LDS: two broadcast reads per column and wave beside the
+// table's).  Past kDtItems items the plain kernel's scalar loads are the
+// better form: 25,000 atoms 169 us against 239 here.
+constexpr int kDtCols = 256, kDtUnroll = 4;
+constexpr size_t dt_lds(int ntypes) {
+  return (size_t)ntypes * kTblN * sizeof(float2) + kDtCols * (sizeof(float4) + sizeof(float2));
+}
+
+__device__ __forceinline__ void desc_tile(const Dev &d, char *lds, int item) {
+  float2 *tab = reinterpret_cast<float2 *>(lds);
+  float4 *col = reinterpret_cast<float4 *>(tab + d.ntypes * kTblN);
+  float2 *cwt = reinterpret_cast<float2 *>(col + kDtCols);
+  const int4 it = d.dt_items[item];                 // row block, columns [y, z), place of the sums
+  const int nc = it.z - it.y, nrow = d.rows;
+  const int i = (int)threadIdx.x < nrow ? d.row_perm[it.x * nrow + threadIdx.x] : -1;
+  const float dp2 = d.tdx * (d.tdx / 6.0f);         // the nodes carry dx^2 / 6 (as k_descreen's)
+  const float2 *src = d.tbl + (size_t)d.rblk[it.x].x * d.ntypes * kTblN;
+  float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), pc = pi;
+  float2 wc = make_float2(0.f, 0.f);
+  if ((int)threadIdx.x < nc) {
+    pc = d.dcol[it.y + threadIdx.x];
+    wc = d.dcw[it.y + threadIdx.x];
+  }
+  if (i >= 0) pi = d.pos[i];
+#pragma unroll 10
+  for (int k = threadIdx.x; k < d.ntypes * kTblN; k += 256) {
+    const float2 v = src[k];
+    tab[k] = make_float2(v.x, v.y * dp2);
+  }
+  col[threadIdx.x] = pc;
+  cwt[threadIdx.x] = wc;
+  __syncthreads();
+  if (__ballot(i >= 0) == 0ull) return;             // a wave of padding rows (no barrier follows)
+  float acc = 0.f;
+  auto tile = [&](auto self) {
+    auto columns = [&](int c, auto count) {
+      constexpr int N = decltype(count)::value;
+      float q[N], w[N];
+#pragma unroll
+      for (int u = 0; u < N; u++) {
+        const float4 pj = col[c + u];
+        const float2 cw = cwt[c + u];
+        const float ex = pj.x - pi.x, ey = pj.y - pi.y, ez = pj.z - pi.z;
+        const float xh = __builtin_amdgcn_sqrtf(fmaf(ez, ez, fmaf(ex, ex, ey * ey))) * pj.w;
+        // q4_value without its branch
+        const unsigned k = (unsigned)(int)xh;
+        const float2 *n = tab + __float_as_int(cw.y) * kTblN + min(k, (unsigned)(kTblN - 2));
+        const float2 n0 = n[0], n1 = n[1];
+        const float B = __builtin_amdgcn_fractf(xh), A = 1.f - B;
+        const float s = fmaf(B, n1.y, fmaf(A, n0.y, n0.y + n1.y));
+        const float v = fmaf(-(A * B), s, fmaf(A, n0.x, B * n1.x));
+        q[u] = k <= (unsigned)(kTblN - 2) ? v : 0.f;
+        w[u] = decltype(self)::value && it.y + c + u == i ? 0.f : cw.x;
+      }
+#pragma unroll
+      for (int u = 0; u < N; u++) acc = fmaf(q[u], w[u], acc);      // in column order
+    };
+    int c = 0;
+#pragma unroll 1
+    for (; c + kDtUnroll <= nc; c += kDtUnroll) columns(c, std::integral_constant<int, kDtUnroll>{});
+#pragma unroll 1
+    for (; c < nc; c++) columns(c, std::integral_constant<int, 1>{});
+  };
+  if (__ballot(i >= it.y && i < it.z) != 0ull) tile(std::true_type{});
+  else tile(std::false_type{});
+  if (i >= 0) d.dpart[it.w + i] = acc;
+}
+
+__global__ __launch_bounds__(256) void k_desc_sites(Dev d, int nsite_blocks) {
+  extern __shared__ __align__(16) char lds[];
+  if ((int)blockIdx.x >= nsite_blocks) {
+    desc_tile(d, lds, (int)blockIdx.x - nsite_blocks);
+    return;
+  }
+  // four sites, then those with more candidates than 128 one by one
+  __shared__ int more[kWsWaves];
+  const int w = (int)(threadIdx.x >> 6), site = (int)blockIdx.x * kWsWaves + w;
+  const bool again = ws_free_site<kWsWaves, kWsCap, WS_RETURN>(
+      d, *reinterpret_cast<WsLds<kWsWaves, kWsCap> *>(lds), site, w);
+  if ((threadIdx.x & 63) == 0) more[w] = again ? site : d.nws;
+  __syncthreads();
+  for (int k = 0; k < kWsWaves; k++) {
+    const int s = more[k];
+    if (s >= d.nws) continue;                       // block-uniform
+    ws_free_site<1, kWsCapBig, WS_FAIL>(d, *reinterpret_cast<WsLds<1, kWsCapBig> *>(lds), w == 0 ? s : d.nws, 0);
+    __syncthreads();
+  }
+}
+
+static size_t desc_sites_lds(const Dev &d) {
+  return std::max(dt_lds(d.ntypes), std::max(sizeof(WsLds<kWsWaves, kWsCap>), sizeof(WsLds<1, kWsCapBig>)));
+}
+
+hipError_t prepare_sites(int ntypes) {
+  static int limit = 0;                             // raised to the largest any pack has needed
+  Dev d{};
+  d.ntypes = std::min(ntypes, kLdsTypes);
+  const int need = (int)desc_sites_lds(d);
+  if (need <= limit) return hipSuccess;
+  const hipError_t e = hipFuncSetAttribute((const void *)k_desc_sites, hipFuncAttributeMaxDynamicSharedMemorySize, need);
+  if (e == hipSuccess) limit = need;
+  return e;
+}
+
+void launch_desc_sites(const Dev &d, hipStream_t s) {
+  const int ns = (d.nws + kWsWaves - 1) / kWsWaves;
+  if (ns + d.ndt_items)
+    hipLaunchKernelGGL(k_desc_sites, dim3(ns + d.ndt_items), dim3(256), desc_sites_lds(d), s, d, ns);
 }
 
 }  // namespace agb

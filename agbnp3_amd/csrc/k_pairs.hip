@@ -17,9 +17,9 @@
 // (descreening, GB pairs) or as per-item partial sums that k_chain_sum adds
 // in a fixed order (chain rule), so results are bitwise reproducible
 // whatever the schedule.
-#include <climits>
 #include <type_traits>
 
+#include <climits>
 #include "agb_common.h"
 #include "agb_device.h"
 
@@ -46,7 +46,6 @@ __device__ __forceinline__ void stage_tables(const Dev &d, float2 *dst, int t, b
 // (reference agbnp3_inverse_born_radii_nolist_soa, kernels.c:500-678)
 // GTAB: more radius types than kLdsTypes; the tables are read through the
 // caches from the pack's table array instead of LDS.
-constexpr int kLdsTypes = 16;
 
 template <int ROWS, bool GTAB>
 __global__ __launch_bounds__(ROWS) void k_descreen(Dev d, const float4 *__restrict__ ccol,
@@ -593,10 +592,11 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
 
 // Chain-rule sums per atom: the partial sums of every item holding its block,
 // in the block's fixed slot order, added in FP64 and stored as the call's
-// fixed-point accumulators (no atomics: k_ingest cleared them; systems on
-// the surrogate this call keep what k_sg_grad adds).  Grid (blocks, 8
+// fixed-point accumulators (no atomics; systems on the surrogate this call
+// keep what k_sg_grad adds to the values k_ingest cleared).  Grid (blocks, 8
 // quantities), one thread per atom slot of a block; slots loaded four ahead
-// of the sum.
+// of the sum.  Without a surrogate the sums of U and V are final here, and
+// their threads form the derivative pass's coefficients (uv_coeffs) at once.
 __global__ __launch_bounds__(256) void k_chain_sum(Dev d) {
   const int b = blockIdx.x, q = blockIdx.y;
   const int a = d.cperm[b * 256 + threadIdx.x];
@@ -627,7 +627,9 @@ __global__ __launch_bounds__(256) void k_chain_sum(Dev d) {
     for (; c < c1; c++) acc += (double)base[(size_t)d.ch_contrib[c] * 8 * 256];
   }
   if (q >= 6) acc *= (double)(1.0f / d.pos[d.cperm[b * 256]].w);   // U, V: 1/R of the block
-  d.acc_ch[8 * (size_t)a + q] = __double2ll_rn(acc * kFix);
+  const long long fix = __double2ll_rn(acc * kFix);
+  d.acc_ch[8 * (size_t)a + q] = fix;
+  if (q >= 6 && !d.sg_on) uv_coeffs(d, a, d.sys[blk.y], q - 6, fix);
 }
 
 // surrogate calls with out-of-range atoms (mode 2): per 64-atom chunk of a

@@ -38,8 +38,9 @@ __global__ __launch_bounds__(256) void k_ingest(Dev d, const double *__restrict_
       d.acc_hb[3 * (size_t)i + q] = 0;
       d.acc_gbg[3 * (size_t)i + q] = 0;
     }
+    if (d.sg_on || !d.nchain_items)          // (else k_chain_sum stores every one)
 #pragma unroll
-    for (int q = 0; q < 8; q++) d.acc_ch[8 * (size_t)i + q] = 0;
+      for (int q = 0; q < 8; q++) d.acc_ch[8 * (size_t)i + q] = 0;
   }
   if (i < Q_COUNT * kQueueSpread) d.queue[i * kQueueStride] = 0;
   if (i < kCountSlots) {
@@ -219,31 +220,6 @@ __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
   if (lane == 0) d.nne[h] = m;
 }
 
-// near-pair total and longest row (counters 2, 3): one add and one max per
-// block rather than per row (same-address atomics serialise in L2)
-__global__ __launch_bounds__(256) void k_nbl_count(Dev d) {
-  __shared__ unsigned long long ssum[4];
-  __shared__ unsigned smax[4];
-  const int h = blockIdx.x * 256 + threadIdx.x;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  unsigned v = h < d.nh ? (unsigned)d.nne[h] : 0u;
-  unsigned long long sum = v;
-  unsigned mx = v;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sum += __shfl_xor(sum, o, 64);
-    mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
-  }
-  if (lane == 0) { ssum[w] = sum; smax[w] = mx; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned long long t = ssum[0] + ssum[1] + ssum[2] + ssum[3];
-    const unsigned m = max(max(smax[0], smax[1]), max(smax[2], smax[3]));
-    if (t) atomicAdd(&d.counters[2], t);
-    if (m) atomicMax(&d.counters[3], (unsigned long long)m);
-  }
-}
-
 // rebuild decision of the neighbour-list reuse: any heavy atom farther than
 // skin/2 from where the kept candidates were built
 __global__ __launch_bounds__(256) void k_guard(Dev d) {
@@ -266,7 +242,6 @@ void launch_nblist(const Dev &d, hipStream_t s) {
     hipLaunchKernelGGL(k_nblist<128>, dim3(nblk), dim3(64 * kNbWaves), 0, s, d);
   else
     hipLaunchKernelGGL(k_nblist<256>, dim3(nblk), dim3(64 * kNbWaves), 0, s, d);
-  hipLaunchKernelGGL(k_nbl_count, dim3((d.nh + 255) / 256), dim3(256), 0, s, d);
 }
 
 }  // namespace agb

@@ -308,16 +308,16 @@ __device__ __forceinline__ int eval_children(TreeLds<CAP, PB> &S, const Gauss &p
     cnt += __popcll(bal);
   }
   nkept += (unsigned)cnt;
-  __syncthreads();
+  wave_sync();
   return cnt;
 }
 
-// depth-first walk of the roots the breadth-first kernel queued (overflow);
-// the grid covers every heavy row, blocks past the queue length exit
+// depth-first walk of one root by one wave (the other waves of its block are
+// past their last access to the LDS it reuses, and take no part)
 template <int CAP, bool PB>
 __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned long long &tk,
                               unsigned long long &te) {
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int i = d.hrow[h];
   const int m = d.nne[h];
   // stage the slot atoms, positions relative to the root (root_frame)
@@ -335,7 +335,7 @@ __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned
 #pragma unroll
     for (int v = 0; v < (PB ? TG_N : 2); v++) S.acc[v][s] = 0.0;
   }
-  __syncthreads();
+  wave_sync();
   double root[TG_N];
 #pragma unroll
   for (int v = 0; v < TG_N; v++) root[v] = 0.0;
@@ -369,7 +369,7 @@ __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned
     const double r = wave_sum(root[v]);
     if (lane == 0) S.acc[v][0] += r;
   }
-  __syncthreads();
+  wave_sync();
   for (int s = lane; s <= m; s += 64) {
     const int at = S.idx[s];
     if (!PB) {
@@ -382,24 +382,7 @@ __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned
   }
   tk += nkept;                          // wave-uniform; added to the counters once per block
   te += neval;
-  __syncthreads();
-}
-
-// the depth-first walk of the roots both breadth-first tiers queued
-template <int CAP, bool PB>
-__global__ __launch_bounds__(64) void k_tree(Dev d) {
-  __shared__ TreeLds<CAP, PB> S;
-  __shared__ int slot;
-  const int count = (int)d.counters[6 + (PB ? 1 : 0)];
-  unsigned *head = queue_head(d.queue, PB ? Q_TREE_FB : Q_TREE_FA);
-  unsigned long long tk = 0, te = 0;
-  for (int k = first_item(); k < count; k = next_item(head, &slot))
-    tree_dfs_root<CAP, PB>(d, S, d.tree_ovf[(size_t)(2 + (PB ? 1 : 0)) * d.nh + k], tk, te);
-  if (!PB && threadIdx.x == 0 && (tk | te)) {
-    unsigned long long *c = d.counters + kCountBase + 8 * (blockIdx.x % kCountSlots);
-    atomicAdd(c, tk);
-    atomicAdd(c + 1, te);
-  }
+  wave_sync();
 }
 
 // ------------------------------------------------------ breadth-first tree
@@ -565,30 +548,31 @@ __device__ __forceinline__ int bfs_order(BfsLds<CAP, PB, LC, W> &S, int cb, int 
 // the block's waves split every order's candidates and the per-slot sums are
 // fixed point, so the result does not depend on the waves' timing.
 template <int CAP, bool PB, int LC, int W>
-__device__ void tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, int list, unsigned long long &tk,
+__device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, int list, unsigned long long &tk,
                               unsigned long long &te) {
   constexpr int NT = 64 * W;
   const int tid = threadIdx.x, lane = tid & 63;
   // pass B's first tier leaves the roots pass A queued to the second tier,
   // which takes pass A's list: both passes walk the same tree, so they
   // outgrow the same buffers
-  if (PB && list == 0 && d.tree_tier[h]) return;       // block-uniform
+  if (PB && list == 0 && d.tree_tier[h]) return true;  // block-uniform
   const int i = d.hrow[h];
   const int m = d.nne[h];
-  // queue this root for the next tier: pass A's first tier to the second
-  // (and it records that), everything else to the depth-first walk
+  // a root that outgrows these buffers: pass A's first tier queues it for the
+  // second (and records that); past the second tier it is walked depth first,
+  // in pass A by the caller, in pass B from a list
   auto queue_next = [&]() {
     if (tid == 0) {
-      const int q = (!PB && list == 0) ? 4 : 6 + (PB ? 1 : 0);
-      const unsigned k = atomicAdd(&d.counters[q], 1ull);
-      d.tree_ovf[(size_t)(q - 4) * d.nh + k] = h;
-      if (!PB && list == 0) d.tree_tier[h] = 1;
+      const bool first = !PB && list == 0;
+      const unsigned k = atomicAdd(&d.counters[first ? 4 : 6 + (PB ? 1 : 0)], 1ull);
+      if (first || PB) d.tree_ovf[(PB ? (size_t)d.nh : 0) + k] = h;
+      if (first) d.tree_tier[h] = 1;
     }
     __syncthreads();
   };
   if (m > CAP) {                          // block-uniform: a row longer than these slot arrays, next tier
     queue_next();
-    return;
+    return false;
   }
   const float4 pr = d.pos[i];
   for (int s = tid; s <= m; s += NT) {
@@ -658,9 +642,9 @@ __device__ void tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
       else if (n > 1) bfs_order<5, CAP, PB, LC, W, false>(S, 0, n, root, df, nkept, neval);
     }
   }
-  if (ovf) {                              // block-uniform: the next tier takes this root
+  if (ovf) {                              // block-uniform
     queue_next();
-    return;
+    return false;
   }
   if (!PB && list == 0 && tid == 0) d.tree_tier[h] = 0;
   // the root's own sums (slot 0 takes no member adds): lane 0 of the wave,
@@ -695,6 +679,7 @@ __device__ void tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
   tk += nkept;                          // block-uniform: wave 0 reports it
   te += neval;                          // this wave's evaluations
   if (W > 1) __syncthreads();           // the next root restages the slots
+  return true;
 }
 
 // overlaps kept (block totals) and evaluated (per wave) by one persistent
@@ -726,8 +711,10 @@ __global__ __launch_bounds__(64 * kFirstWaves, PB ? 4 : 7) void k_tree_bfs(Dev d
   __shared__ int slot;
   unsigned *head = queue_head(d.queue, PB ? Q_TREE_B : Q_TREE_A);
   // roots in runs of `run` per queue grab (one returning atomic on the queue
-  // head per grab; at least two: the grabs serialise on that one address)
-  const int run = max(2, min(8, d.nh / (int)(gridDim.x * 8)));
+  // head per grab; at least two: the grabs serialise on that one address),
+  // one by one where the grid has a block for each: half the blocks would
+  // otherwise walk two in a row beside an idle half
+  const int run = (int)gridDim.x >= d.nh ? 1 : max(2, min(8, d.nh / (int)(gridDim.x * 8)));
   // queue position k takes root (k * P) mod nh, P a prime that does not
   // divide nh: roots in flight together lie far apart in the atom order, so
   // their fixed-point scatters rarely meet on one atom
@@ -744,7 +731,11 @@ __global__ __launch_bounds__(64 * kFirstWaves, PB ? 4 : 7) void k_tree_bfs(Dev d
 // registers).  The largest level of a 25,000-atom solute holds ~300 nodes;
 // 1536-node levels with 16 waves per root (one block per CU) took 7 % longer
 // on a batch of 50 6000-atom solutes, whose 3,200 queued roots keep every CU
-// busy.  What still overflows goes to the depth-first kernel.
+// busy.  What still overflows is walked depth first: in pass A by the block's
+// first wave in the same LDS (a launch of its own for those few roots cost
+// 4.5 us on every call, mostly with nothing to walk), in pass B, whose walk
+// would take this kernel past 128 registers (220 bytes of scratch per lane),
+// by k_tree_dfs behind this kernel, beside the first tier.
 constexpr int kBigWaves = 8;
 template <int CAP, bool PB>
 __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
@@ -755,13 +746,30 @@ __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
   const int count = (int)d.counters[4];
   unsigned *head = queue_head(d.queue, PB ? Q_TREE_BB : Q_TREE_BA);
   unsigned long long tk = 0, te = 0;
-  for (int k = first_item(); k < count; k = next_item(head, &slot))
-    tree_bfs_root<CAP, PB, kLevelCapBig, kBigWaves>(d, S, d.tree_ovf[k], 1, tk, te);
+  for (int k = first_item(); k < count; k = next_item(head, &slot)) {
+    const int h = d.tree_ovf[k];
+    const bool done = tree_bfs_root<CAP, PB, kLevelCapBig, kBigWaves>(d, S, h, 1, tk, te);
+    if constexpr (!PB) {
+      if (!done && threadIdx.x < 64)
+        tree_dfs_root<CAP, PB>(d, *reinterpret_cast<TreeLds<CAP, PB> *>(lds_raw), h, tk, te);
+    }
+  }
   add_tree_counts(d, PB, tk, te);
 }
 
+// pass B's depth-first walk of the roots its second tier listed
+template <int CAP>
+__global__ __launch_bounds__(64) void k_tree_dfs(Dev d) {
+  __shared__ TreeLds<CAP, true> S;
+  const int count = (int)d.counters[7];
+  unsigned long long tk = 0, te = 0;
+  for (int k = blockIdx.x; k < count; k += gridDim.x) tree_dfs_root<CAP, true>(d, S, d.tree_ovf[d.nh + k], tk, te);
+}
+
 template <int CAP, bool PB>
-static size_t big_lds() { return sizeof(BfsLds<CAP, PB, kLevelCapBig, kBigWaves>); }
+static size_t big_lds() {
+  return std::max(sizeof(BfsLds<CAP, PB, kLevelCapBig, kBigWaves>), PB ? 0 : sizeof(TreeLds<CAP, PB>));
+}
 
 hipError_t prepare_tree() {
   hipError_t e = hipSuccess;
@@ -778,20 +786,19 @@ hipError_t prepare_tree() {
 }
 
 // persistent grids: resident blocks for the breadth-first pass, two per CU
-// for the second tier, small grids for the (short) depth-first queue
+// for the second tier
 template <int CAP>
 static void launch_tree_cap(const Dev &d, const Tuning &t, int pass, int tier, hipStream_t s) {
-  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : 256 * 16), gf = std::min(d.nh, 256);
+  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : 256 * 16), gf = std::min(d.nh, 64);
   const int gb = std::min(d.nh, 512);
   const size_t la = big_lds<CAP, false>(), lb = big_lds<CAP, true>();
   if (pass == 0) {
     if (tier == 0) hipLaunchKernelGGL((k_tree_bfs<first_cap(CAP), false>), dim3(g), dim3(64 * kFirstWaves), 0, s, d);
     if (tier == 1) hipLaunchKernelGGL((k_tree_bfs_big<CAP, false>), dim3(gb), dim3(64 * kBigWaves), la, s, d);
-    if (tier == 2) hipLaunchKernelGGL((k_tree<CAP, false>), dim3(gf), dim3(64), 0, s, d);
   } else {
     if (tier == 0) hipLaunchKernelGGL((k_tree_bfs<first_cap(CAP), true>), dim3(g), dim3(64 * kFirstWaves), 0, s, d);
     if (tier == 1) hipLaunchKernelGGL((k_tree_bfs_big<CAP, true>), dim3(gb), dim3(64 * kBigWaves), lb, s, d);
-    if (tier == 2) hipLaunchKernelGGL((k_tree<CAP, true>), dim3(gf), dim3(64), 0, s, d);
+    if (tier == 1) hipLaunchKernelGGL((k_tree_dfs<CAP>), dim3(gf), dim3(64), 0, s, d);
   }
 }
 
@@ -803,7 +810,7 @@ void launch_tree_tier(const Dev &d, const Tuning &t, int pass, int tier, hipStre
 }
 
 void launch_tree(const Dev &d, const Tuning &t, int pass, hipStream_t s) {
-  for (int tier = 0; tier < 3; tier++) launch_tree_tier(d, t, pass, tier, s);
+  for (int tier = 0; tier < 2; tier++) launch_tree_tier(d, t, pass, tier, s);
 }
 
 }  // namespace agb
