@@ -153,22 +153,41 @@ void launch_descreen(const Dev &d, const Tuning &t, hipStream_t s) {
 // they started (one column read and one rotation per four pairs).  A row's
 // sums over the four waves' chunks are added in wave order through LDS.
 // Diagonal tiles see each pair twice and keep only the row side.
+// Bound: VALU issue.  On this GPU two waves of a SIMD can each issue an FP32
+// add, multiply or multiply-add in the same four cycles, but a DPP move and a
+// transcendental stop both for about twenty; so the column sums rotate
+// through the LDS crossbar (ds_bpermute; LDS is otherwise nearly idle here)
+// instead of four DPP moves per step, and 98 registers, four waves per SIMD,
+// are enough.  With that and without the mask's compare and select per pair
+// off the diagonal: 25,000 atoms 0.262 -> 0.234 ms, 150,000 8.38 -> 7.95 ms
+// (the clock falls to 2.0 GHz there), 24 x 6000 0.364 -> 0.357 ms.
 __device__ __forceinline__ float wave_rot(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x13C, 0xF, 0xF, true));
 }
 __device__ __forceinline__ int wave_rot(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x13C, 0xF, 0xF, true); }
 
+// the same rotation through the LDS crossbar (rot_from: the byte address of
+// the lane that lane l takes its value from)
+__device__ __forceinline__ int rot_from(int lane) { return ((lane + 63) & 63) * 4; }
+__device__ __forceinline__ float lds_rot(float v, int from) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, v)));
+}
+
 // one row's GB pair terms with one column
 struct GbRow {
   float x, y, z, q, b, qib;     // position, charge, Born radius, -log2(e) / (4 B)
 };
-__device__ __forceinline__ void gb_pair(const GbRow &r, const float4 &cp, const float2 &cb, float &re, float &rA,
-                                        float &rx, float &ry, float &rz, float &cA, float &cgx, float &cgy,
+// MASK: the reference's mask (kernels.c:107), d2 > 0, which also drops the
+// self pair; without it the smallest d2 is kept instead
+template <bool MASK>
+__device__ __forceinline__ void gb_pair(const GbRow &r, const float4 &cp, const float2 &cb, float &d2min, float &re,
+                                        float &rA, float &rx, float &ry, float &rz, float &cA, float &cgx, float &cgy,
                                         float &cgz) {
   const float ex = cp.x - r.x, ey = cp.y - r.y, ez = cp.z - r.z;
   const float d2 = ex * ex + ey * ey + ez * ez;
-  // the reference's mask (kernels.c:107): d2 > 0, which also drops the self pair
-  const float qq = d2 > 0.f ? r.q * cp.w : 0.f;
+  float qq = r.q * cp.w;
+  if (MASK) qq = d2 > 0.f ? qq : 0.f;
+  else d2min = fminf(d2min, d2);
   const float bb = r.b * cb.x;
   const float et = __builtin_amdgcn_exp2f(d2 * (r.qib * cb.y));     // exp(-d2 / (4 B_i B_j))
   const float fgb = __builtin_amdgcn_rsqf(d2 + bb * et);
@@ -180,10 +199,10 @@ __device__ __forceinline__ void gb_pair(const GbRow &r, const float4 &cp, const 
   rx += mw * ex; ry += mw * ey; rz += mw * ez;
   rA += at;
   cA += at;
-  cgx -= mw * ex; cgy -= mw * ey; cgz -= mw * ez;
+  cgx = fmaf(mw, ex, cgx); cgy = fmaf(mw, ey, cgy); cgz = fmaf(mw, ez, cgz);     // (negated)
 }
 
-__global__ __launch_bounds__(256, 5) void k_gbpair(Dev d) {
+__global__ __launch_bounds__(256, 4) void k_gbpair(Dev d) {
   // tile columns per 64-column chunk, each chunk twice in a row so that
   // column (l - s) mod 64 sits at l + 64 - s: x, y, z, charge; Born radius,
   // its reciprocal
@@ -231,18 +250,31 @@ __global__ __launch_bounds__(256, 5) void k_gbpair(Dev d) {
           rz[4] = {0.f, 0.f, 0.f, 0.f}, re = 0.f;
     float cA = 0.f, cgx = 0.f, cgy = 0.f, cgz = 0.f;
     if (w < nch) {
-      // the column whose partial sums this lane holds at step s: (lane - s) mod 64
-      const float4 *cxc = &cxq[w][lane + 64];
-      const float2 *cbc = &cbr[w][lane + 64];
-#pragma unroll 1
-      for (int s = 0; s < 64; s++) {
-        const float4 cp = cxc[-s];
-        const float2 cb = cbc[-s];
+      auto sweep = [&](auto mask) {
+        constexpr bool M = decltype(mask)::value;
+        const int from = rot_from(lane);
+        float d2min = 1.f;
+        re = cA = cgx = cgy = cgz = 0.f;
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-          gb_pair(row[k], cp, cb, re, rA[k], rx[k], ry[k], rz[k], cA, cgx, cgy, cgz);
-        cA = wave_rot(cA); cgx = wave_rot(cgx); cgy = wave_rot(cgy); cgz = wave_rot(cgz);
-      }
+        for (int k = 0; k < 4; k++) rA[k] = rx[k] = ry[k] = rz[k] = 0.f;
+        // the column whose partial sums this lane holds at step s: (lane - s) mod 64
+        const float4 *cxc = &cxq[w][lane + 64];
+        const float2 *cbc = &cbr[w][lane + 64];
+#pragma unroll 1
+        for (int s = 0; s < 64; s++) {
+          const float4 cp = cxc[-s];
+          const float2 cb = cbc[-s];
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            gb_pair<M>(row[k], cp, cb, d2min, re, rA[k], rx[k], ry[k], rz[k], cA, cgx, cgy, cgz);
+          cA = lds_rot(cA, from); cgx = lds_rot(cgx, from); cgy = lds_rot(cgy, from); cgz = lds_rot(cgz, from);
+        }
+        return __ballot(d2min == 0.f) != 0ull;
+      };
+      // without a self pair the mask only matters for two atoms in one place:
+      // the sweep then runs again with it (a compare and a select per pair
+      // less otherwise)
+      if (diag || sweep(std::false_type{})) sweep(std::true_type{});
       // 64 rotations bring every column's sums back to its starting lane
     }
     const double e = wave_sum((double)re * (diag ? 0.5 : 1.0));
@@ -250,9 +282,9 @@ __global__ __launch_bounds__(256, 5) void k_gbpair(Dev d) {
     const int j = tp.z + threadIdx.x;
     if (!diag && j < tp.w) {             // the columns' sums (this wave's chunk)
       fix_add(&d.acc_gbA[j], (double)cA);
-      fix_add(&d.acc_gbg[3 * (size_t)j], (double)cgx);
-      fix_add(&d.acc_gbg[3 * (size_t)j + 1], (double)cgy);
-      fix_add(&d.acc_gbg[3 * (size_t)j + 2], (double)cgz);
+      fix_add(&d.acc_gbg[3 * (size_t)j], -(double)cgx);
+      fix_add(&d.acc_gbg[3 * (size_t)j + 1], -(double)cgy);
+      fix_add(&d.acc_gbg[3 * (size_t)j + 2], -(double)cgz);
     }
     // the rows' sums over the four waves' column chunks in wave order
     for (int g = 0; g < 4; g++) {
