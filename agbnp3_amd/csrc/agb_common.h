@@ -32,6 +32,8 @@ constexpr int kForkAtoms = 16384;
 constexpr int kSideAtoms = 512;
 // most items of the descreening by tiles (measured: k_desc_sites)
 constexpr int kDtItems = 2048;
+// most items of a chain-rule launch whose lookups are grouped: four per CU
+constexpr int kChainGroupItems = 1024;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;

@@ -362,14 +362,16 @@ enum : int { CK_GEN = 0, CK_HH = 1, CK_HX = 2, CK_HX0 = 3, CK_HHS = 4 };
 // the exact value (rounding of the coordinate differences, d^2, the hardware
 // reciprocal square root, c = 1 / (R dx) and the product); where that band
 // reaches a node, xh is recomputed in FP64 from the FP32 coordinates as
-// d / R * (1/dx) (a few lookups in 10^4).  u = xh - floor(xh) is exact
-// (xh >= 0), as is the FP64 path's.
-__device__ __forceinline__ void chain_coord(float xh, const float4 &pa, const float4 &pb, float R, float dxinv,
-                                            int &k, float &u) {
-  constexpr float kLast = (float)kTblN - 0.5f;
-  xh = fminf(xh, kLast);
+// d / R * (1/dx) (a few lookups in 10^4: chain_fix).  u = xh - floor(xh) is
+// exact (xh >= 0), as is the FP64 path's.
+__device__ __forceinline__ void chain_coord(float &xh, int &k, float &u) {
+  xh = fminf(xh, (float)kTblN - 0.5f);
   k = (int)xh;
   u = __builtin_amdgcn_fractf(xh);
+}
+__device__ __forceinline__ void chain_fix(float xh, const float4 &pa, const float4 &pb, float R, float dxinv, int &k,
+                                          float &u) {
+  constexpr float kLast = (float)kTblN - 0.5f;
   if (fabsf(u - 0.5f) > fmaf(-8e-7f, xh, 0.5f - 1e-6f)) {
     // the empty asm statements keep the FP64 conversions inside this rare
     // branch (hoisted, they cost three conversions on every pair), and keep
@@ -385,6 +387,9 @@ __device__ __forceinline__ void chain_coord(float xh, const float4 &pa, const fl
     u = (float)(x64 - (double)k);
   }
 }
+// A group of lookups tests for the band together, against its widest
+// (xh <= kTblN - 0.5): no lookup within |u - 0.5| <= kChainBand is in it.
+constexpr float kChainBand = 0.49958f;    // < 0.5 - 1e-6 - 8e-7 (kTblN - 0.5)
 
 // the derivative x dx of the interval record c as a quadratic in u,
 // (e0, e1, e2): e0 + e1 u + e2 u^2
@@ -409,6 +414,8 @@ __device__ __forceinline__ void chain_poly(const float4 &c, const float4 &e, flo
   dqx = fmaf(fmaf(e.z, u, e.y), u, e.x);
 }
 
+enum : int { CM_PLAIN = 0, CM_GROUP = 1 };
+
 // per 64-column chunk: the columns' records, and once every wave is past the
 // chunk, in the same bytes, its column sums [gb xyz, vw xyz, U, V][column]
 struct ChainChunk {
@@ -421,7 +428,14 @@ struct ChainChunk {
   };
 };
 
-template <int KIND, bool QUIRK>
+// CM_GROUP: where a CU holds one item at a time (one wave per SIMD), the pairs of
+// a column step (two steps with one row per lane) are met first, tested for
+// the band with one wave-uniform branch, and read the tables together: a
+// divergent branch per lookup serialises the lookups' LDS reads (2,000 atoms:
+// 76 -> 66 us).  With several items per CU their waves fill those waits, and
+// taking the lookups one by one is as fast or faster (150,000 atoms: 7.1 ms
+// against 7.3).
+template <int KIND, bool QUIRK, int MODE>
 __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &item, const float4 *__restrict__ tab_rc,
                                            const float4 *__restrict__ tab_cr, ChainChunk *ch) {
   // rows per lane: two where the registers allow 5 waves per SIMD (wave w
@@ -430,6 +444,10 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
   constexpr int NR = (KIND == CK_HH || KIND == CK_GEN) ? 1 : 2;
   constexpr int NW = 4 / NR;           // waves on one chunk
   constexpr int kUnroll = 3 - NR;      // column steps unrolled: 2 with one row, 1 with two
+  constexpr bool GROUP = MODE == CM_GROUP;
+  constexpr int NS = GROUP ? kUnroll : 1;                  // column steps of a group
+  constexpr bool kOne = KIND == CK_HX || KIND == CK_HX0;   // one direction: k (hydrogen) <- j
+  constexpr bool kTwo = KIND == CK_HH || KIND == CK_GEN;   // two lookups (CK_HHS: one serves both directions)
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int rh = NR == 2 ? w & 1 : w, cp = NR == 2 ? w >> 1 : 0;   // row group, chunk parity
   const int4 bp = d.cblk[item.x];
@@ -489,73 +507,132 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
     const int c = cbeg + cp + NR * ci;
     float ca[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (c < cend) {
-#pragma unroll kUnroll
-      for (int s = 0; s < 64; s++) {
-        const int col = (lane - s) & 63;                  // the column whose sums this lane holds
-        const float4 pj = ch[c].col.pos[col];
-        const float4 pp = ch[c].col.par[col];
-#pragma unroll
-        for (int k = 0; k < NR; k++) {
-          const float ex = pj.x - pk[k].x, ey = pj.y - pk[k].y, ez = pj.z - pk[k].z;
-          const float d2 = ex * ex + ey * ey + ez * ez;
-          float id = __builtin_amdgcn_rsqf(d2);           // hardware reciprocal square root (1 ulp)
-          float dist = d2 * id;
-          bool jheavy = true;
-          if (KIND == CK_GEN) {
-            // the self pair of a diagonal block, padding rows, hydrogen-hydrogen
-            // pairs: no weight, and a distance past the tables (zero interval)
-            jheavy = pp.z != 0.f;
-            const bool pair = kok[k] && (kheavy[k] || jheavy) && !(diag && c * 64 + col == rr[k]);
-            id = pair ? id : 0.f;
-            dist = pair ? dist : 1e6f;
-          }
-          float hgb, hvw = 0.f;
-          if (KIND == CK_HX || KIND == CK_HX0) {          // k (hydrogen) <- j
-            int k1;
-            float u1, q1, dq1;
-            chain_coord(dist * cQ, pk[k], pj, RQ, dxinv, k1, u1);
-            chain_poly(tab_rc[k1], tab_cr[k1], u1, q1, dq1);   // one direction: tab_cr holds tab_rc's derivatives
-            const float t1 = pj.w * dq1 * id;
-            hgb = q2k[k] * t1;
-            ca[6] = fmaf(q2k[k], q1, ca[6]);
-            if (KIND == CK_HX) {
-              hvw = abk[k] * t1;
-              ca[7] = fmaf(abk[k], q1, ca[7]);
-            }
-          } else {
-            int k1, k2;
-            float u1, u2, q1, dq1, q2, dq2;
-            chain_coord(dist * cQ, pk[k], pj, RQ, dxinv, k1, u1);
-            chain_poly<QUIRK>(tab_rc[k1], u1, q1, dq1);  // k <- j (weight 0 unless j heavy)
-            if (KIND == CK_HHS) {                         // j <- k: the same lookup
-              q2 = q1;
-              dq2 = dq1;
-            } else {
-              chain_coord(dist * cP, pj, pk[k], RP, dxinv, k2, u2);
-              chain_poly<QUIRK>(tab_cr[k2], u2, q2, dq2);  // j <- k
-            }
-            if (KIND == CK_GEN) {
-              q2 = kheavy[k] ? q2 : 0.f;
-              q1 = jheavy ? q1 : 0.f;
-            }
-            const float t1 = pj.w * dq1 * id, t2 = wk[k] * dq2 * id;
-            hgb = fmaf(q2k[k], t1, pp.x * t2);
-            hvw = fmaf(abk[k], t1, pp.y * t2);
-            rU[k] = fmaf(pp.x, q2, rU[k]);
-            rV[k] = fmaf(pp.y, q2, rV[k]);
-            ca[6] = fmaf(q2k[k], q1, ca[6]);
+      struct Pair {
+        float ex, ey, ez, id, x1, x2, u1, u2;
+        int k1, k2;
+      };
+      auto meet = [&](int k, int col, const float4 &pj, const float4 &pp) {
+        Pair m;
+        m.ex = pj.x - pk[k].x; m.ey = pj.y - pk[k].y; m.ez = pj.z - pk[k].z;
+        const float d2 = m.ex * m.ex + m.ey * m.ey + m.ez * m.ez;
+        m.id = __builtin_amdgcn_rsqf(d2);               // hardware reciprocal square root (1 ulp)
+        float dist = d2 * m.id;
+        if (KIND == CK_GEN) {
+          // the self pair of a diagonal block, padding rows, hydrogen-hydrogen
+          // pairs: no weight, and a distance past the tables (zero interval)
+          const bool pair = kok[k] && (kheavy[k] || pp.z != 0.f) && !(diag && c * 64 + col == rr[k]);
+          m.id = pair ? m.id : 0.f;
+          dist = pair ? dist : 1e6f;
+        }
+        m.x1 = dist * cQ;
+        chain_coord(m.x1, m.k1, m.u1);
+        if (!GROUP) chain_fix(m.x1, pk[k], pj, RQ, dxinv, m.k1, m.u1);
+        if (kTwo) {
+          m.x2 = dist * cP;
+          chain_coord(m.x2, m.k2, m.u2);
+          if (!GROUP) chain_fix(m.x2, pj, pk[k], RP, dxinv, m.k2, m.u2);
+        }
+        return m;
+      };
+      auto add = [&](int k, const Pair &m, const float4 &pj, const float4 &pp, const float4 &c1, const float4 &c2) {
+        float hgb, hvw = 0.f, q1, dq1;
+        if (kOne) {
+          chain_poly(c1, c2, m.u1, q1, dq1);            // tab_cr holds tab_rc's derivatives
+          const float t1 = pj.w * dq1 * m.id;
+          hgb = q2k[k] * t1;
+          ca[6] = fmaf(q2k[k], q1, ca[6]);
+          if (KIND == CK_HX) {
+            hvw = abk[k] * t1;
             ca[7] = fmaf(abk[k], q1, ca[7]);
           }
-          rg[k][0] = fmaf(hgb, ex, rg[k][0]); rg[k][1] = fmaf(hgb, ey, rg[k][1]); rg[k][2] = fmaf(hgb, ez, rg[k][2]);
-          ca[0] = fmaf(-hgb, ex, ca[0]); ca[1] = fmaf(-hgb, ey, ca[1]); ca[2] = fmaf(-hgb, ez, ca[2]);
-          if (KIND != CK_HX0) {
-            rv[k][0] = fmaf(hvw, ex, rv[k][0]); rv[k][1] = fmaf(hvw, ey, rv[k][1]); rv[k][2] = fmaf(hvw, ez, rv[k][2]);
-            ca[3] = fmaf(-hvw, ex, ca[3]); ca[4] = fmaf(-hvw, ey, ca[4]); ca[5] = fmaf(-hvw, ez, ca[5]);
+        } else {
+          float q2, dq2;
+          chain_poly<QUIRK>(c1, m.u1, q1, dq1);         // k <- j (weight 0 unless j heavy)
+          if (kTwo) {
+            chain_poly<QUIRK>(c2, m.u2, q2, dq2);       // j <- k
+          } else {
+            q2 = q1;
+            dq2 = dq1;
           }
+          if (KIND == CK_GEN) {
+            q2 = kheavy[k] ? q2 : 0.f;
+            q1 = pp.z != 0.f ? q1 : 0.f;
+          }
+          const float t1 = pj.w * dq1 * m.id, t2 = wk[k] * dq2 * m.id;
+          hgb = fmaf(q2k[k], t1, pp.x * t2);
+          hvw = fmaf(abk[k], t1, pp.y * t2);
+          rU[k] = fmaf(pp.x, q2, rU[k]);
+          rV[k] = fmaf(pp.y, q2, rV[k]);
+          ca[6] = fmaf(q2k[k], q1, ca[6]);
+          ca[7] = fmaf(abk[k], q1, ca[7]);
         }
+        rg[k][0] = fmaf(hgb, m.ex, rg[k][0]); rg[k][1] = fmaf(hgb, m.ey, rg[k][1]); rg[k][2] = fmaf(hgb, m.ez, rg[k][2]);
+        ca[0] = fmaf(-hgb, m.ex, ca[0]); ca[1] = fmaf(-hgb, m.ey, ca[1]); ca[2] = fmaf(-hgb, m.ez, ca[2]);
+        if (KIND != CK_HX0) {
+          rv[k][0] = fmaf(hvw, m.ex, rv[k][0]); rv[k][1] = fmaf(hvw, m.ey, rv[k][1]); rv[k][2] = fmaf(hvw, m.ez, rv[k][2]);
+          ca[3] = fmaf(-hvw, m.ex, ca[3]); ca[4] = fmaf(-hvw, m.ey, ca[4]); ca[5] = fmaf(-hvw, m.ez, ca[5]);
+        }
+      };
+      auto rotate = [&]() {
 #pragma unroll
         for (int q = 0; q < 8; q++)
           if (KIND != CK_HX0 || q < 3 || q == 6) ca[q] = wave_rot(ca[q]);   // (the vdW sums stay zero)
+      };
+      if constexpr (GROUP) {
+#pragma unroll 1
+        for (int s = 0; s < 64; s += NS) {
+          float4 pj[NS], pp[NS], c1[NS][NR], c2[NS][NR];
+          Pair m[NS][NR];
+          float band = 0.f;
+#pragma unroll
+          for (int t = 0; t < NS; t++) {
+            const int col = (lane - s - t) & 63;          // the column whose sums this lane holds
+            pj[t] = ch[c].col.pos[col];
+            pp[t] = ch[c].col.par[col];
+#pragma unroll
+            for (int k = 0; k < NR; k++) {
+              m[t][k] = meet(k, col, pj[t], pp[t]);
+              band = fmaxf(band, fabsf(m[t][k].u1 - 0.5f));
+              if (kTwo) band = fmaxf(band, fabsf(m[t][k].u2 - 0.5f));
+            }
+          }
+          if (__builtin_expect(__ballot(band > kChainBand) != 0ull, 0)) {
+#pragma unroll
+            for (int t = 0; t < NS; t++)
+#pragma unroll
+              for (int k = 0; k < NR; k++) {
+                chain_fix(m[t][k].x1, pk[k], pj[t], RQ, dxinv, m[t][k].k1, m[t][k].u1);
+                if (kTwo) chain_fix(m[t][k].x2, pj[t], pk[k], RP, dxinv, m[t][k].k2, m[t][k].u2);
+              }
+          }
+#pragma unroll
+          for (int t = 0; t < NS; t++)
+#pragma unroll
+            for (int k = 0; k < NR; k++) {
+              c1[t][k] = tab_rc[m[t][k].k1];
+              if (kTwo || kOne) c2[t][k] = tab_cr[kTwo ? m[t][k].k2 : m[t][k].k1];
+            }
+#pragma unroll
+          for (int t = 0; t < NS; t++) {
+#pragma unroll
+            for (int k = 0; k < NR; k++) add(k, m[t][k], pj[t], pp[t], c1[t][k], c2[t][k]);
+            rotate();
+          }
+        }
+      } else {
+#pragma unroll kUnroll
+        for (int s = 0; s < 64; s++) {
+          const int col = (lane - s) & 63;
+          const float4 pj = ch[c].col.pos[col], pp = ch[c].col.par[col];
+#pragma unroll
+          for (int k = 0; k < NR; k++) {
+            const Pair m = meet(k, col, pj, pp);
+            float4 c2;
+            if (kTwo || kOne) c2 = tab_cr[kTwo ? m.k2 : m.k1];
+            add(k, m, pj, pp, tab_rc[m.k1], c2);
+          }
+          rotate();
+        }
       }
     }
     // chunk c's column sums over its waves' row groups in a fixed order
@@ -674,7 +751,7 @@ __global__ __launch_bounds__(256) void k_chain_flags(Dev d) {
   if ((threadIdx.x & 63) == 0) d.ch_flag[slot >> 6] = m != 0ull ? 1 : 0;
 }
 
-template <bool QUIRK>
+template <bool QUIRK, int MODE>
 __global__ __launch_bounds__(256) void k_chain(Dev d) {
   // row <- column and column <- row interval cubics; for hydrogen rows (one
   // direction) the row <- column cubics and their derivative records
@@ -715,11 +792,11 @@ __global__ __launch_bounds__(256) void k_chain(Dev d) {
       staged_rc = trc;
       staged_cr = kcr;
     }
-    if (item.z == CK_HH && bp.x == bq.x) chain_item<CK_HHS, QUIRK>(d, it, item, tab_rc, tab_cr, ch);
-    else if (item.z == CK_HH) chain_item<CK_HH, QUIRK>(d, it, item, tab_rc, tab_cr, ch);
-    else if (item.z == CK_HX0) chain_item<CK_HX0, QUIRK>(d, it, item, tab_rc, tab_cr, ch);
-    else if (item.z == CK_HX) chain_item<CK_HX, QUIRK>(d, it, item, tab_rc, tab_cr, ch);
-    else chain_item<CK_GEN, QUIRK>(d, it, item, tab_rc, tab_cr, ch);
+    if (item.z == CK_HH && bp.x == bq.x) chain_item<CK_HHS, QUIRK, MODE>(d, it, item, tab_rc, tab_cr, ch);
+    else if (item.z == CK_HH) chain_item<CK_HH, QUIRK, MODE>(d, it, item, tab_rc, tab_cr, ch);
+    else if (item.z == CK_HX0) chain_item<CK_HX0, QUIRK, MODE>(d, it, item, tab_rc, tab_cr, ch);
+    else if (item.z == CK_HX) chain_item<CK_HX, QUIRK, MODE>(d, it, item, tab_rc, tab_cr, ch);
+    else chain_item<CK_GEN, QUIRK, MODE>(d, it, item, tab_rc, tab_cr, ch);
     __syncthreads();
   }
 }
@@ -731,8 +808,10 @@ void launch_chain(const Dev &d, const Tuning &t, hipStream_t s) {
     grid = std::min(grid, kSgPersistentGrid);
     if (d.ncblk) hipLaunchKernelGGL(k_chain_flags, dim3(d.ncblk), dim3(256), 0, s, d);
   }
-  if (d.options & 2) hipLaunchKernelGGL(k_chain<false>, dim3(grid), dim3(256), 0, s, d);
-  else hipLaunchKernelGGL(k_chain<true>, dim3(grid), dim3(256), 0, s, d);
+  const bool fixed = (d.options & 2) != 0;
+  auto k = fixed ? k_chain<false, CM_PLAIN> : k_chain<true, CM_PLAIN>;
+  if (d.nchain_items <= kChainGroupItems) k = fixed ? k_chain<false, CM_GROUP> : k_chain<true, CM_GROUP>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, d);
   if (d.ncblk) hipLaunchKernelGGL(k_chain_sum, dim3(d.ncblk, 8), dim3(256), 0, s, d);
 }
 
