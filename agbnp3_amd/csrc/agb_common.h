@@ -30,6 +30,16 @@ constexpr float kHbSwA = 0.65f, kHbSwB = 1.0f, kHbSwA0 = 0.6f;
 // from which the second tier of the derivative pass has that stream
 constexpr int kForkAtoms = 16384;
 constexpr int kSideAtoms = 512;
+// columns of a descreening group with a box of its own
+constexpr int kBoxCols = 16;
+// extents of a solute, in units of the longest table's reach (46 A for heavy
+// atoms of up to 1.8 A), from which the descreening and the chain rule skip
+// far columns by boxes.  Share of the pairs skipped and time, synthetic
+// solutes: descreening 25,000 atoms (1.7 reaches across) 7 %, 169 -> 183 us;
+// 40,000 (2.0) 19 %, 431 -> 391 us; 150,000 (3.1) 60 %, 3.66 -> 2.15 ms.
+// Chain rule, whose sums fix the order of the atoms inside its blocks: 40,000
+// 0.4 %, 567 -> 585 us; 150,000 14 %, 6.94 -> 6.64 ms.
+constexpr float kCullDesc = 1.85f, kCullChain = 2.6f;
 // most items of the descreening by tiles (measured: k_desc_sites)
 constexpr int kDtItems = 2048;
 // most items of a chain-rule launch whose lookups are grouped: four per CU
@@ -250,6 +260,12 @@ struct Dev {
   float *sp_f, *spe_f;                 // FP32 copies for pair kernels
   float4 *dcol;                        // heavy atoms as descreening columns: x, y, z, 1/(R dx)
   float2 *dcw;                         // and (sp / R, radius type as int bits)
+  // boxes the spline kernels skip far columns by: per 16 descreening columns
+  // ([nablk][16], a system's from blk0) low corner and smallest 1/(R dx),
+  // high corner; per 64-atom chunk of a chain-rule block its corners
+  int cull_desc, cull_chain;
+  float4 *cbox;
+  float4 *chbox;
   double *beta, *br, *brw, *swf;       // [n]
   float *br_f;
   double *gb_epart;                    // per GB energy slot: sum of q_i q_j / f

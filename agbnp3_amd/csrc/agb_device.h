@@ -74,6 +74,46 @@ __device__ __forceinline__ float wave_max(float v) {
 }
 __device__ __forceinline__ int wave_incl_scan(int v) { return dpp::incl_scan(v); }
 
+// --------------------------------------------------------------- far boxes
+// The spline tables end in a zero interval (coordinate d / (R dx) >= kTblN - 1
+// in FP32), so pairs past it add exact zeros and leave every sum as it is.
+// Boxes of atoms decide it for many pairs at once: kFarCoord leaves 0.1 % for
+// the rounding of boxes and coordinates.  A box with an atom that is not
+// finite is the whole space, so its pairs are evaluated.
+constexpr float kFarCoord = (float)(kTblN - 1) * 1.001f;
+struct Box {
+  float lo[3], hi[3];
+};
+__device__ __forceinline__ Box box_of(bool valid, const float4 &p) {
+  Box b;
+  const float v[3] = {p.x, p.y, p.z};
+  const bool fin = fabsf(p.x) < INFINITY && fabsf(p.y) < INFINITY && fabsf(p.z) < INFINITY;
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    b.lo[k] = !valid ? INFINITY : (fin ? v[k] : -INFINITY);
+    b.hi[k] = !valid ? -INFINITY : (fin ? v[k] : INFINITY);
+  }
+  return b;
+}
+// the union over groups of W lanes, in every lane of the group
+template <int W>
+__device__ __forceinline__ void box_union(Box &b) {
+#pragma unroll
+  for (int o = W / 2; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      b.lo[k] = fminf(b.lo[k], __shfl_xor(b.lo[k], o, 64));
+      b.hi[k] = fmaxf(b.hi[k], __shfl_xor(b.hi[k], o, 64));
+    }
+}
+// squared distance between two boxes (infinite when one is empty)
+__device__ __forceinline__ float box_gap2(const Box &a, const float4 &lo, const float4 &hi) {
+  const float x = fmaxf(0.f, fmaxf(a.lo[0] - hi.x, lo.x - a.hi[0]));
+  const float y = fmaxf(0.f, fmaxf(a.lo[1] - hi.y, lo.y - a.hi[1]));
+  const float z = fmaxf(0.f, fmaxf(a.lo[2] - hi.z, lo.z - a.hi[2]));
+  return x * x + y * y + z * z;
+}
+
 // ------------------------------------------------------------ work queues
 // Persistent blocks take work items from a queue head in memory; every block
 // leaves once the head has passed the item count, so the grid always drains.

@@ -188,6 +188,10 @@ struct Model {
   std::vector<WsDef> wsdef;
   std::vector<int> ws_stale0;          // per site; -1: no atom (spe 0)
   int nws = 0;
+  // place of each atom along a space-filling curve through the coordinates
+  // the instance was created with
+  std::vector<unsigned> curve;
+  float extent = 0;                    // longest edge of their box
 };
 
 // ------------------------------------------------------------- pack
@@ -206,6 +210,7 @@ struct Pack {
   std::vector<int> rtype;              // per atom
   std::vector<char> heavy;             // per atom
   std::vector<float> alpha_sum;        // per atom: ialpha + salpha
+  std::vector<unsigned> curve;         // per atom: Model::curve
   hipStream_t stream = nullptr;
   // second stream for the water-site kernels, which need only the self
   // volumes: they run beside the descreening and pair kernels (fork and join
@@ -518,6 +523,9 @@ int build_items(Pack &P) {
       std::vector<int> r;
       for (int i = S.a0; i < S.a0 + S.n; i++)
         if (P.rtype[i] == t) r.push_back(i);
+      // (a row's sum does not depend on the rows beside it: rows close in
+      // space share a wave, so that it can pass over far columns)
+      std::stable_sort(r.begin(), r.end(), [&](int a, int b) { return P.curve[a] < P.curve[b]; });
       for (size_t k = 0; k < r.size(); k += rows) {
         int allh = 1;
         for (int q = 0; q < rows; q++) {
@@ -742,6 +750,8 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
     take(*q, n);
   take(d.dcol, n);
   take(d.dcw, n);
+  take(d.cbox, 2 * (size_t)std::max(nablk, 1) * (256 / kBoxCols));
+  take(d.chbox, 8 * (size_t)std::max(d.ncblk, 1));
   take(d.gb_epart, (size_t)std::max(ntile, 1));
   take(d.ws_part, nws);
   take(d.ws_ovf, nws);
@@ -847,6 +857,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
       P.rtype.push_back(lmap[b][m.rtype[i]]);
       P.heavy.push_back(i < m.nheavy);
       P.alpha_sum.push_back(m.ialpha[i] + m.salpha[i]);
+      P.curve.push_back(m.curve[i]);
       R.push_back(m.R[i]); q.push_back(m.q[i]); galpha.push_back(m.galpha[i]);
       igamma.push_back(m.igamma[i]); sgamma.push_back(m.sgamma[i]);
       ialpha.push_back(m.ialpha[i]); salpha.push_back(m.salpha[i]);
@@ -906,6 +917,11 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
       upload(L, &d.wsdef, wsdef) || upload(L, &d.ws_site, ws_site) || upload(L, &d.ws_stale0, ws_stale0))
     return AGBNP_ERR;
   P.ntile = tile0;
+  float reaches = 0.f;                  // of the widest solute (as created; only a choice of kernels)
+  for (int b = 0; b < P.nsys; b++)
+    if (P.sinfo[b].nh) reaches = std::max(reaches, ms[b]->extent / (kTblAmax * P.sinfo[b].rmax_heavy));
+  d.cull_desc = reaches > kCullDesc && P.ntypes <= kLdsTypes;
+  d.cull_chain = reaches > kCullChain;
   // state that lives as long as the pack: status word, counters, queue heads
   if (dalloc(L, &d.status, 1) || dalloc(L, &d.queue, kQueueWords) || dalloc(L, &d.counters, kCounters))
     return AGBNP_ERR;
@@ -1444,6 +1460,34 @@ void agbnp3_terminate(void) {
   g_initialized = false;
 }
 
+// Morton keys (10 bits per axis) of the coordinates; coordinates that are not
+// finite (they are only meant to be replaced by ener) go to one end
+static void curve_keys(int n, const float_i *x, const float_i *y, const float_i *z, const std::vector<int> &int2ext,
+                       std::vector<unsigned> &key, float &extent) {
+  const float_i *c[3] = {x, y, z};
+  double lo[3] = {0, 0, 0}, ext = 0;
+  for (int k = 0; k < 3; k++) {
+    double a = INFINITY, b = -INFINITY;
+    for (int i = 0; i < n; i++)
+      if (std::isfinite((double)c[k][i])) {
+        a = std::min(a, (double)c[k][i]);
+        b = std::max(b, (double)c[k][i]);
+      }
+    if (a <= b) {
+      lo[k] = a;
+      ext = std::max(ext, b - a);
+    }
+  }
+  extent = (float)ext;
+  key.assign(n, 0u);
+  for (int i = 0; i < n; i++)
+    for (int k = 0; k < 3; k++) {
+      const double u = ((double)c[k][int2ext[i]] - lo[k]) / ext * 1023.0;     // (NaN where every atom is in one place)
+      const unsigned q = u >= 0.0 ? (unsigned)std::min(u, 1023.0) : 0u;
+      for (int b = 0; b < 10; b++) key[i] |= ((q >> b) & 1u) << (3 * b + k);
+    }
+}
+
 int agbnp3_new(int *tag, int natoms, float_i *x, float_i *y, float_i *z, float_i *r, float_i *charge,
                float_i dielectric_in, float_i dielectric_out, float_i *igamma, float_i *sgamma, float_i *ialpha,
                float_i *salpha, int *hbtype, float_i *hbcorr, int nhydrogen, int *ihydrogen, NeighList *conntbl,
@@ -1490,6 +1534,7 @@ int agbnp3_new(int *tag, int natoms, float_i *x, float_i *y, float_i *z, float_i
       I->ext2int[i] = slot;
     }
   }
+  curve_keys(n, x, y, z, I->int2ext, I->curve, I->extent);
   auto f = [](double v) { return (float)v; };
   I->R.resize(n); I->q.resize(n); I->igamma.resize(n); I->sgamma.resize(n); I->ialpha.resize(n);
   I->salpha.resize(n); I->hbcorr.resize(n); I->hbtype.resize(n); I->vols.resize(n); I->galpha.resize(n);

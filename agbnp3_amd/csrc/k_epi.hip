@@ -99,6 +99,21 @@ __global__ __launch_bounds__(kEpi) void k_scale(Dev d) {
       d.sp_f[i] = d.spe_f[i] = d.gammap_f[i] = 0.f;
     }
   }
+  if (d.cull_desc) {                    // boxes of the descreening's column groups
+    const bool col = i < blk.y && i < d.sys[d.asys[blk.x]].a0 + d.sys[d.asys[blk.x]].nh;
+    float4 p = make_float4(0.f, 0.f, 0.f, 1.f);
+    if (col) p = d.pos[i];
+    Box b = box_of(col, p);
+    float w = col ? 1.0f / p.w * d.tdxinv : INFINITY;
+    box_union<kBoxCols>(b);
+#pragma unroll
+    for (int o = kBoxCols / 2; o > 0; o >>= 1) w = fminf(w, __shfl_xor(w, o, 64));
+    if (threadIdx.x % kBoxCols == 0) {
+      float4 *o = d.cbox + 2 * ((size_t)blockIdx.x * (kEpi / kBoxCols) + threadIdx.x / kBoxCols);
+      o[0] = make_float4(b.lo[0], b.lo[1], b.lo[2], w);
+      o[1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.f);
+    }
+  }
   const int slots[3] = {EP_CAV, EP_CORR_CAV, EP_MOLVOL};
   const double v[3] = {ecav, ecorr, mv};
   block_partials(d, slots, v, 3);
@@ -185,6 +200,19 @@ void launch_born(const Dev &d, hipStream_t s) {
 // descreening, so every other atom's chain-rule weight is zero (the
 // surrogate's gradient pass weighs them from the FP64 values)
 __global__ __launch_bounds__(kEpi) void k_q2ab(Dev d) {
+  const int nblk = (d.n + kEpi - 1) / kEpi;
+  if ((int)blockIdx.x >= nblk) {        // further blocks: the boxes of the chain rule's chunks
+    const int slot = (blockIdx.x - nblk) * kEpi + threadIdx.x, a = d.cperm[slot];
+    float4 p = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (a >= 0) p = d.pos[a];
+    Box b = box_of(a >= 0, p);
+    box_union<64>(b);
+    if ((threadIdx.x & 63) == 0) {
+      d.chbox[2 * (slot >> 6)] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.f);
+      d.chbox[2 * (slot >> 6) + 1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.f);
+    }
+    return;
+  }
   const int i = blockIdx.x * kEpi + threadIdx.x;
   if (i < d.n) {
     const double A = fix_get(d.acc_gbA[i]);
@@ -199,7 +227,8 @@ __global__ __launch_bounds__(kEpi) void k_q2ab(Dev d) {
 }
 
 void launch_q2ab(const Dev &d, hipStream_t s) {
-  hipLaunchKernelGGL(k_q2ab, dim3((d.n + kEpi - 1) / kEpi), dim3(kEpi), 0, s, d);
+  const int boxes = d.cull_chain && d.nchain_items > kChainGroupItems ? d.ncblk : 0;
+  hipLaunchKernelGGL(k_q2ab, dim3((d.n + kEpi - 1) / kEpi + boxes), dim3(kEpi), 0, s, d);
 }
 
 // ------------------------------------------------------ U, V coefficients

@@ -47,7 +47,9 @@ __device__ __forceinline__ void stage_tables(const Dev &d, float2 *dst, int t, b
 // GTAB: more radius types than kLdsTypes; the tables are read through the
 // caches from the pack's table array instead of LDS.
 
-template <int ROWS, bool GTAB>
+// CULL (large solutes): columns are taken in groups of 16 whose boxes
+// (k_scale) the wave's rows, close in space, may pass over as past the tables.
+template <int ROWS, bool GTAB, bool CULL>
 __global__ __launch_bounds__(ROWS) void k_descreen(Dev d, const float4 *__restrict__ ccol,
                                                   const float2 *__restrict__ cwt) {
   extern __shared__ float2 dyn_tab[];     // [ntypes][512]: tables [t_row][*]
@@ -81,9 +83,28 @@ __global__ __launch_bounds__(ROWS) void k_descreen(Dev d, const float4 *__restri
     float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i >= 0) pi = d.pos[i];
     const int c0 = item.y, c1 = item.z;
+    constexpr int kGroups = kTile / kBoxCols;
+    const SysInfo &S = d.sys[d.rblk[item.x].y];
+    Box rows{};
+    if (CULL) {
+      rows = box_of(i >= 0, pi);
+      box_union<64>(rows);
+    }
+    unsigned long long near = ~0ull;     // column groups of the next four tiles that the wave's rows reach
     double acc = 0.0;
-    for (int base = c0; base < c1; base += kTile) {
+    for (int base = c0; base < c1; base += kTile, near >>= kGroups) {
       const int nc = min(kTile, c1 - base);
+      if (CULL && ((base - c0) & (4 * kTile - 1)) == 0) {
+        const float4 *box = d.cbox + 2 * (size_t)(S.blk0 * kGroups + (base - S.a0) / kBoxCols + (int)(threadIdx.x & 63));
+        bool reach = false;
+        if (base + (int)(threadIdx.x & 63) * kBoxCols < c1) {
+          const float4 lo = box[0], hi = box[1];
+          reach = !(box_gap2(rows, lo, hi) * (lo.w * lo.w) > kFarCoord * kFarCoord);
+        }
+        near = __ballot(reach);
+      }
+      unsigned groups = (unsigned)near & ((1u << kGroups) - 1u);
+      if (CULL && groups == 0) continue;   // (its sum would be an exact zero)
       float tacc = 0.f;
       // every lane runs the loop (a padding row, i < 0, at the origin: its sum
       // is dropped), so the column index stays wave-uniform.  Only a tile
@@ -98,19 +119,27 @@ __global__ __launch_bounds__(ROWS) void k_descreen(Dev d, const float4 *__restri
           // the same FMA either way: a pair's term does not depend on its tile's test
           tacc = fmaf(q, (decltype(self)::value && j == i) ? 0.f : w.x, tacc);
         };
-        int c = 0;
-        for (; c + 4 <= nc; c += 4) {                   // four columns' records in two scalar loads
-          float4 pj[4];
-          float2 w[4];
+        auto columns = [&](int c, int ce) {
+          for (; c + 4 <= ce; c += 4) {                 // four columns' records in two scalar loads
+            float4 pj[4];
+            float2 w[4];
 #pragma unroll
-          for (int u = 0; u < 4; u++) {
-            pj[u] = ccol[base + c + u];
-            w[u] = cwt[base + c + u];
+            for (int u = 0; u < 4; u++) {
+              pj[u] = ccol[base + c + u];
+              w[u] = cwt[base + c + u];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) column(base + c + u, pj[u], w[u]);   // sums stay in column order
           }
-#pragma unroll
-          for (int u = 0; u < 4; u++) column(base + c + u, pj[u], w[u]);   // sums stay in column order
-        }
-        for (; c < nc; c++) column(base + c, ccol[base + c], cwt[base + c]);
+          for (; c < ce; c++) column(base + c, ccol[base + c], cwt[base + c]);
+        };
+        if (!CULL) columns(0, nc);
+        else
+          while (groups) {                              // runs of near groups, in column order
+            const int g = __builtin_ctz(groups), run = __builtin_ctz(~(groups >> g));
+            groups &= ~(((1u << run) - 1u) << g);
+            columns(g * kBoxCols, min(nc, (g + run) * kBoxCols));
+          }
       };
       if (__ballot(i >= base && i < base + nc) != 0ull) tile(std::true_type{});
       else tile(std::false_type{});
@@ -128,15 +157,13 @@ void launch_descreen(const Dev &d, const Tuning &t, hipStream_t s) {
   if (d.sg_on) grid = std::min(grid, kSgPersistentGrid);   // calls where every block leaves at once
   const float4 *ccol = d.dcol;
   const float2 *cwt = d.dcw;
-  if (gtab) {
-    if (d.rows == 64) hipLaunchKernelGGL((k_descreen<64, true>), dim3(grid), dim3(64), 0, s, d, ccol, cwt);
-    else if (d.rows == 128) hipLaunchKernelGGL((k_descreen<128, true>), dim3(grid), dim3(128), 0, s, d, ccol, cwt);
-    else hipLaunchKernelGGL((k_descreen<256, true>), dim3(grid), dim3(256), 0, s, d, ccol, cwt);
-  } else {
-    if (d.rows == 64) hipLaunchKernelGGL((k_descreen<64, false>), dim3(grid), dim3(64), lds, s, d, ccol, cwt);
-    else if (d.rows == 128) hipLaunchKernelGGL((k_descreen<128, false>), dim3(grid), dim3(128), lds, s, d, ccol, cwt);
-    else hipLaunchKernelGGL((k_descreen<256, false>), dim3(grid), dim3(256), lds, s, d, ccol, cwt);
-  }
+  const int m = gtab ? 0 : (d.cull_desc ? 2 : 1);
+  const auto pick = [&](auto g, auto plain, auto cull) { return m == 0 ? g : (m == 1 ? plain : cull); };
+  const auto k = d.rows == 64 ? pick(k_descreen<64, true, false>, k_descreen<64, false, false>, k_descreen<64, false, true>)
+               : d.rows == 128
+                   ? pick(k_descreen<128, true, false>, k_descreen<128, false, false>, k_descreen<128, false, true>)
+                   : pick(k_descreen<256, true, false>, k_descreen<256, false, false>, k_descreen<256, false, true>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(d.rows), lds, s, d, ccol, cwt);
 }
 
 // ------------------------------------------------------------- GB pairs
@@ -414,7 +441,7 @@ __device__ __forceinline__ void chain_poly(const float4 &c, const float4 &e, flo
   dqx = fmaf(fmaf(e.z, u, e.y), u, e.x);
 }
 
-enum : int { CM_PLAIN = 0, CM_GROUP = 1 };
+enum : int { CM_PLAIN = 0, CM_GROUP = 1, CM_CULL = 2 };
 
 // per 64-column chunk: the columns' records, and once every wave is past the
 // chunk, in the same bytes, its column sums [gb xyz, vw xyz, U, V][column]
@@ -428,6 +455,7 @@ struct ChainChunk {
   };
 };
 
+// CM_CULL (large solutes): a wave passes over the chunks past the tables' end.
 // CM_GROUP: where a CU holds one item at a time (one wave per SIMD), the pairs of
 // a column step (two steps with one row per lane) are met first, tested for
 // the band with one wave-uniform branch, and read the tables together: a
@@ -499,6 +527,19 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
   for (int k = 0; k < NR; k++) {
     rg[k][0] = rg[k][1] = rg[k][2] = rv[k][0] = rv[k][1] = rv[k][2] = rU[k] = rV[k] = 0.f;
   }
+  // pairs past the tables' end add nothing: a wave passes over the chunks whose
+  // box lies that far from its rows'
+  unsigned reach = 15u;
+  if (MODE == CM_CULL) {
+    const float4 *b = d.chbox + 2 * (4 * item.x + (NR == 2 ? 2 * rh : rh)), *q = d.chbox + 2 * (4 * item.y + (lane & 3));
+    Box rows{{b[0].x, b[0].y, b[0].z}, {b[1].x, b[1].y, b[1].z}};
+    if (NR == 2) {
+      rows.lo[0] = fminf(rows.lo[0], b[2].x); rows.lo[1] = fminf(rows.lo[1], b[2].y); rows.lo[2] = fminf(rows.lo[2], b[2].z);
+      rows.hi[0] = fmaxf(rows.hi[0], b[3].x); rows.hi[1] = fmaxf(rows.hi[1], b[3].y); rows.hi[2] = fmaxf(rows.hi[2], b[3].z);
+    }
+    const float far = kFarCoord / fminf(cQ, kOne ? cQ : cP);
+    reach = (unsigned)__ballot(!(box_gap2(rows, q[0], q[1]) > far * far)) & 15u;     // lane c: chunk c
+  }
   // the item's 64-column chunks of block Q; waves of chunk parity cp take
   // chunks cbeg + cp, cbeg + cp + NR, ...
   const int cbeg = item.w & 15, cend = item.w >> 4;
@@ -506,7 +547,7 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
   for (int ci = 0; ci < niter; ci++) {
     const int c = cbeg + cp + NR * ci;
     float ca[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (c < cend) {
+    if (c < cend && ((reach >> c) & 1u)) {
       struct Pair {
         float ex, ey, ez, id, x1, x2, u1, u2;
         int k1, k2;
@@ -811,6 +852,7 @@ void launch_chain(const Dev &d, const Tuning &t, hipStream_t s) {
   const bool fixed = (d.options & 2) != 0;
   auto k = fixed ? k_chain<false, CM_PLAIN> : k_chain<true, CM_PLAIN>;
   if (d.nchain_items <= kChainGroupItems) k = fixed ? k_chain<false, CM_GROUP> : k_chain<true, CM_GROUP>;
+  else if (d.cull_chain) k = fixed ? k_chain<false, CM_CULL> : k_chain<true, CM_CULL>;
   hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, d);
   if (d.ncblk) hipLaunchKernelGGL(k_chain_sum, dim3(d.ncblk, 8), dim3(256), 0, s, d);
 }
@@ -827,9 +869,12 @@ hipError_t prepare_pairs(int ntypes) {
   auto set = [&](const void *f, int bytes) {
     if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   };
-  set((const void *)k_descreen<64, false>, d1);
-  set((const void *)k_descreen<128, false>, d1);
-  set((const void *)k_descreen<256, false>, d1);
+  set((const void *)k_descreen<64, false, false>, d1);
+  set((const void *)k_descreen<128, false, false>, d1);
+  set((const void *)k_descreen<256, false, false>, d1);
+  set((const void *)k_descreen<64, false, true>, d1);
+  set((const void *)k_descreen<128, false, true>, d1);
+  set((const void *)k_descreen<256, false, true>, d1);
   if (e == hipSuccess) limit = d1;
   return e;
 }
