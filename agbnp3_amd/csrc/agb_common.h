@@ -181,7 +181,7 @@ struct Dev {
   const int *asys;       // system of each atom
   const int *hrow;       // atom of each heavy row
   // static inputs (pack order)
-  const int *int2ext;    // pack order -> caller order (concatenated per system)
+  const int *ext2int;    // caller order (concatenated per system) -> pack order
   const float *R;        // r + 0.5
   const float *q;
   const int *rtype;
@@ -250,6 +250,7 @@ struct Dev {
   long long *acc_beta;                 // descreening sums [n]
   long long *acc_gbA, *acc_gbg;        // GB pairs: A_i [n], gradient [n][3]
   long long *acc_ch;                   // chain rule [n][8]: gb xyz, vdw xyz, U, V
+  unsigned long long *hstat;           // pinned host memory (may be null): the call's status word and counters 0..3
   unsigned long long *counters;        // [0] kept overlaps [1] evaluated [2] nbl entries [3] max row
                                        // [4] roots queued for the second breadth-first tier (pass A; pass B
                                        //     takes the same list), [5] unused

@@ -231,9 +231,11 @@ struct Pack {
   void *call_block = nullptr;
   int call_nchain = 0;                 // chain-rule items the block's partial sums hold
   size_t call_dpart = 0;               // descreening tile sums it holds
-  double *dx = nullptr, *dy = nullptr, *dz = nullptr;      // coordinate staging (device)
   double *dout = nullptr;                                  // outputs: 15n + 7 nsys
-  double *hstage = nullptr;                                // pinned host staging
+  // pinned host staging, which the first and last kernels of a host-API call
+  // read and write themselves: outputs, coordinates, status and counters (5)
+  double *hstage = nullptr;
+  bool host_status = false;            // the last call put its status there
   // timing mode: one event set per recorded call, averaged when read back
   std::vector<std::vector<hipEvent_t>> ev_sets;
   std::vector<std::string> ev_names;
@@ -786,23 +788,23 @@ int ensure_call_state(Pack &P) {
   }
   const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
   const size_t nn = std::max(P.n, 1);
-  const size_t stage = (18 * nn + 7 * (size_t)P.nsys + 8) * sizeof(double);   // outputs, inputs, status
+  const size_t outs = 15 * nn + 7 * (size_t)P.nsys, stage = (outs + 3 * nn + 8) * sizeof(double);
   char *blk = nullptr;
-  if (hipMalloc((void **)&blk, bytes + stage) != hipSuccess) {
-    errprint("agbnp3: device allocation of %zu bytes failed\n", bytes + stage);
+  if (hipMalloc((void **)&blk, bytes + outs * sizeof(double)) != hipSuccess) {
+    errprint("agbnp3: device allocation of %zu bytes failed\n", bytes + outs * sizeof(double));
     return AGBNP_ERR;
   }
   P.call_block = blk;
   P.call_nchain = d.nchain_items;
   P.call_dpart = P.call_ndpart();
   carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
-  double *st = reinterpret_cast<double *>(blk + bytes);
-  P.dx = st;
-  P.dy = st + nn;
-  P.dz = st + 2 * nn;
-  P.dout = st + 3 * nn;
+  P.dout = reinterpret_cast<double *>(blk + bytes);
   HIPCHK(hipMemset(d.ws_part, 0, sizeof(double) * std::max(d.nws, 1)));
-  if (!P.hstage) HIPCHK(hipHostMalloc((void **)&P.hstage, stage, hipHostMallocDefault));
+  if (!P.hstage) {
+    HIPCHK(hipHostMalloc((void **)&P.hstage, stage, hipHostMallocDefault));
+    memset(P.hstage, 0, stage);
+  }
+  d.hstat = reinterpret_cast<unsigned long long *>(P.hstage + 15 * (size_t)P.n + 7 * (size_t)P.nsys + 3 * (size_t)P.n);
   // (a pack that is only copied into a batch, or called through
   // agbnp3_ener_static, never comes here: no stream for it)
   if (!P.side && P.n >= kSideAtoms && make_side(P) != AGBNP_OK) return AGBNP_ERR;
@@ -828,7 +830,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
       lmap[b].push_back(g);
     }
   P.ntypes = (int)P.radii.size();
-  std::vector<int> int2ext, asys, hrow, ws_stale0;
+  std::vector<int> ext2int, asys, hrow, ws_stale0;
   std::vector<float> R, q, galpha, igamma, sgamma, ialpha, salpha, hbcorr;
   std::vector<double> vols;
   std::vector<int2> ablk;
@@ -852,7 +854,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
     S.rmax_heavy = rmax;
     P.sinfo.push_back(S);
     for (int i = 0; i < m.natoms; i++) {
-      int2ext.push_back(a0 + m.int2ext[i]);
+      ext2int.push_back(a0 + m.ext2int[i]);
       asys.push_back(b);
       P.rtype.push_back(lmap[b][m.rtype[i]]);
       P.heavy.push_back(i < m.nheavy);
@@ -910,7 +912,7 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
   chain_tables(ty, ty2, P.ntypes * P.ntypes, d.tdx, ctab);
   auto &L = P.allocs;
   if (upload(L, &d.sys, P.sinfo) || upload(L, &d.asys, asys) || upload(L, &d.hrow, hrow) ||
-      upload(L, &d.int2ext, int2ext) || upload(L, &d.R, R) || upload(L, &d.q, q) || upload(L, &d.rtype, P.rtype) ||
+      upload(L, &d.ext2int, ext2int) || upload(L, &d.R, R) || upload(L, &d.q, q) || upload(L, &d.rtype, P.rtype) ||
       upload(L, &d.galpha, galpha) || upload(L, &d.igamma, igamma) || upload(L, &d.sgamma, sgamma) ||
       upload(L, &d.ialpha, ialpha) || upload(L, &d.salpha, salpha) || upload(L, &d.hbcorr_f, hbcorr) ||
       upload(L, &d.vols, vols) || upload(L, &d.tbl, tb) || upload(L, &d.ctab, ctab) || upload(L, &d.ablk, ablk) ||
@@ -1033,6 +1035,7 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   mark("tree_derivs");
   launch_final(d, sp, br, sa, dgbdr, dvwdr, decav, dehb, energies, s);
   mark("final");
+  if (!capturing) P.host_status = d.hstat != nullptr;
   HIPCHK(hipGetLastError());
   return AGBNP_OK;
 }
@@ -1051,6 +1054,12 @@ int run_pipeline(Pack &P, const double *x, const double *y, const double *z, dou
 
 // status word and largest neighbour-list row of the last call (waits)
 int read_status(Pack &P, int *status, int *maxrow) {
+  if (P.host_status) {                  // k_final has written it to host memory
+    HIPCHK(hipStreamSynchronize(P.stream));
+    *status = (int)(P.d.hstat[0] & 0xffffffffull);
+    if (maxrow) *maxrow = (int)P.d.hstat[1 + 3];
+    return AGBNP_OK;
+  }
   int st = 0;
   unsigned long long c[4] = {0, 0, 0, 0};
   HIPCHK(hipMemcpyAsync(&st, P.d.status, sizeof(int), hipMemcpyDeviceToHost, P.stream));
@@ -1112,22 +1121,16 @@ int pack_ener_host(Pack &P, const double *x, const double *y, const double *z, d
   memcpy(hin, x, n * sizeof(double));
   memcpy(hin + n, y, n * sizeof(double));
   memcpy(hin + 2 * n, z, n * sizeof(double));
-  hipStream_t s = P.stream;
-  HIPCHK(hipMemcpyAsync(P.dx, hin, n * sizeof(double), hipMemcpyHostToDevice, s));
-  HIPCHK(hipMemcpyAsync(P.dy, hin + n, n * sizeof(double), hipMemcpyHostToDevice, s));
-  HIPCHK(hipMemcpyAsync(P.dz, hin + 2 * n, n * sizeof(double), hipMemcpyHostToDevice, s));
-  double *o = P.dout;
-  // outputs and status word come back together: one wait per call (the
-  // outputs of a call that overflowed are discarded and the call re-run)
-  unsigned long long *hst = reinterpret_cast<unsigned long long *>(hin + 3 * n);
+  // the kernels read the coordinates and write outputs and status in place
+  // (copies would be five launches of their own, 30 us of a small call): one
+  // wait per call; the outputs of a call that overflowed are discarded and
+  // the call re-run
   for (int attempt = 0; attempt < 3; attempt++) {
-    if (run_pipeline(P, P.dx, P.dy, P.dz, o, o + n, o + 2 * n, o + 3 * n, o + 6 * n, o + 9 * n, o + 12 * n,
-                     o + 15 * n, false) != AGBNP_OK)
+    if (run_pipeline(P, hin, hin + n, hin + 2 * n, h, h + n, h + 2 * n, h + 3 * n, h + 6 * n, h + 9 * n, h + 12 * n,
+                     h + 15 * n, false) != AGBNP_OK)
       return AGBNP_ERR;
-    HIPCHK(hipMemcpyAsync(h, o, (15 * n + 7 * (size_t)P.nsys) * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(hst, P.d.status, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(hst + 1, P.d.counters, 4 * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(hipStreamSynchronize(P.stream));
+    const unsigned long long *hst = P.d.hstat;
     const int st = (int)(hst[0] & 0xffffffffull), maxrow = (int)hst[1 + 3];
     if (st == 0) {
       adapt_cap(P, maxrow);
@@ -1691,8 +1694,8 @@ int agbnp3_ener_static(int tag, const double *x, const double *y, const double *
              "holds %zu (use agbnp3_ener_device).\n", tag, P.n, need, (size_t)AGBNP3_STATIC_SCRATCH_BYTES);
     return AGBNP_ERR;
   }
-  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items,
-                                       P.call_ndpart());
+  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items, P.call_ndpart());
+  d.hstat = nullptr;
   // no per-kernel timing events here (creating them allocates)
   const int saved = P.options;
   P.options &= ~AGBNP3_OPT_TIMING;
@@ -2118,6 +2121,7 @@ int agbnp3_batch_graph_launch(int batch) {
     return AGBNP_ERR;
   }
   HIPCHK(hipGraphLaunch(B->p.gexec, B->p.stream));
+  B->p.host_status = true;
   return AGBNP_OK;
 }
 

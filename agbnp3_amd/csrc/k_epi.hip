@@ -288,45 +288,58 @@ __device__ __forceinline__ void system_energies(const Dev &d, int sys, double *e
 
 // ----------------------------------------------------------- final output
 // gradients: GB = 332 (pair + chain + tree), vdW = chain + tree,
-// cavity = tree, HB = direct + tree (agbnp3.c:1718-1786); caller order
+// cavity = tree, HB = direct + tree (agbnp3.c:1718-1786); caller order.  The
+// outputs may lie in host memory, so a block's gradients go through LDS and
+// leave as whole lines; the call's status goes there too (hstat), which saves
+// the host three copies of their own launch and wait each.
 __global__ __launch_bounds__(kEpi) void k_final(Dev d, double *sp, double *br, double *sa, double *dgbdr,
                                                 double *dvwdr, double *decav, double *dehb, double *energies) {
+  __shared__ double out[4][3 * kEpi];
   if ((int)blockIdx.x < d.nsys) {                    // the first blocks: a system's energies each
+    if (blockIdx.x == 0 && d.hstat && threadIdx.x < 5)
+      d.hstat[threadIdx.x] = threadIdx.x == 0 ? (unsigned long long)(unsigned)*d.status : d.counters[threadIdx.x - 1];
     system_energies(d, blockIdx.x, energies);
     return;
   }
-  const int i = (blockIdx.x - d.nsys) * kEpi + threadIdx.x;
-  if (i >= d.n) return;
-  const int e = d.int2ext[i];
-  const SysInfo &S = d.sys[d.asys[i]];
-  const bool heavy = i < S.a0 + S.nh;
-  const double df = S.df64;
-  double g_gb[3], g_vw[3];
-  const double f4 = 1.0 / (4.0 * kPi);
-  for (int q = 0; q < 3; q++) {
-    g_gb[q] = 2.0 * df * fix_get(d.acc_gbg[3 * (size_t)i + q]) + df * f4 * fix_get(d.acc_ch[8 * (size_t)i + q]);
-    g_vw[q] = f4 * fix_get(d.acc_ch[8 * (size_t)i + 3 + q]);
-  }
-  double g_cav[3] = {0, 0, 0}, g_hb[3];
-  for (int q = 0; q < 3; q++) g_hb[q] = fix_get(d.acc_hb[3 * (size_t)i + q]);
-  if (heavy) {
-    const long long *t = d.acc_grad + (size_t)i * TG_N;
+  const int e0 = (blockIdx.x - d.nsys) * kEpi, e = e0 + threadIdx.x;
+  if (e < d.n) {
+    const int i = d.ext2int[e];
+    const SysInfo &S = d.sys[d.asys[i]];
+    const bool heavy = i < S.a0 + S.nh;
+    const double df = S.df64;
+    double g_gb[3], g_vw[3];
+    const double f4 = 1.0 / (4.0 * kPi);
     for (int q = 0; q < 3; q++) {
-      g_gb[q] += fix_get(t[TG_GB + q]);
-      g_vw[q] += fix_get(t[TG_VW + q]);
-      g_cav[q] = fix_get(t[TG_CAV + q]);
-      g_hb[q] += fix_get(t[TG_HB + q]);
+      g_gb[q] = 2.0 * df * fix_get(d.acc_gbg[3 * (size_t)i + q]) + df * f4 * fix_get(d.acc_ch[8 * (size_t)i + q]);
+      g_vw[q] = f4 * fix_get(d.acc_ch[8 * (size_t)i + 3 + q]);
     }
+    double g_cav[3] = {0, 0, 0}, g_hb[3];
+    for (int q = 0; q < 3; q++) g_hb[q] = fix_get(d.acc_hb[3 * (size_t)i + q]);
+    if (heavy) {
+      const long long *t = d.acc_grad + (size_t)i * TG_N;
+      for (int q = 0; q < 3; q++) {
+        g_gb[q] += fix_get(t[TG_GB + q]);
+        g_vw[q] += fix_get(t[TG_VW + q]);
+        g_cav[q] = fix_get(t[TG_CAV + q]);
+        g_hb[q] += fix_get(t[TG_HB + q]);
+      }
+    }
+    for (int q = 0; q < 3; q++) {
+      out[0][3 * threadIdx.x + q] = kTokcal * g_gb[q];
+      out[1][3 * threadIdx.x + q] = g_vw[q];
+      out[2][3 * threadIdx.x + q] = g_cav[q];
+      out[3][3 * threadIdx.x + q] = g_hb[q];
+    }
+    sp[e] = heavy ? d.sp[i] : 1.0;
+    br[e] = d.br[i];
+    sa[e] = heavy ? d.sa_f[i] : 0.0;
   }
-  for (int q = 0; q < 3; q++) {
-    dgbdr[3 * (size_t)e + q] = kTokcal * g_gb[q];
-    dvwdr[3 * (size_t)e + q] = g_vw[q];
-    decav[3 * (size_t)e + q] = g_cav[q];
-    dehb[3 * (size_t)e + q] = g_hb[q];
-  }
-  sp[e] = heavy ? d.sp[i] : 1.0;
-  br[e] = d.br[i];
-  sa[e] = heavy ? d.sa_f[i] : 0.0;
+  __syncthreads();
+  double *const dst[4] = {dgbdr, dvwdr, decav, dehb};
+  const int m = 3 * min(kEpi, d.n - e0);
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    for (int q = threadIdx.x; q < m; q += kEpi) dst[k][3 * (size_t)e0 + q] = out[k][q];
 }
 
 void launch_final(const Dev &d, double *sp, double *br, double *sa, double *dgbdr, double *dvwdr, double *decav,

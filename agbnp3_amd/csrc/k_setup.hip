@@ -13,7 +13,9 @@ namespace agb {
 
 // ---------------------------------------------------------------- ingest
 // caller-order FP64 coordinates -> internal FP32 (x, y, z, R); clears the
-// scatter accumulators and work-queue heads of the call
+// scatter accumulators and work-queue heads of the call.  A thread takes its
+// caller's atom (the coordinates may lie in host memory, which is read in
+// whole lines) and clears its internal one.
 __global__ __launch_bounds__(256) void k_ingest(Dev d, const double *__restrict__ x,
                                                 const double *__restrict__ y,
                                                 const double *__restrict__ z) {
@@ -21,8 +23,8 @@ __global__ __launch_bounds__(256) void k_ingest(Dev d, const double *__restrict_
   if (d.sg_on && i < d.nsys) d.sg_state[4 * i + 3] = 0;   // surrogate: out-of-range flag of the call
   if (d.sg_on && i == 0) *d.sg_any_plain = 0;
   if (i < d.n) {
-    const int e = d.int2ext[i];
-    d.pos[i] = make_float4((float)x[e], (float)y[e], (float)z[e], d.R[i]);
+    const int a = d.ext2int[i];
+    d.pos[a] = make_float4((float)x[i], (float)y[i], (float)z[i], d.R[a]);
     const SysInfo &S = d.sys[d.asys[i]];
     if (i < S.a0 + S.nh) {
       d.acc_vol[i] = 0;
