@@ -44,6 +44,11 @@ constexpr float kCullDesc = 1.85f, kCullChain = 2.6f;
 constexpr int kDtItems = 2048;
 // most items of a chain-rule launch whose lookups are grouped: four per CU
 constexpr int kChainGroupItems = 1024;
+// most chain-rule items of a launch that takes them longest first, by their
+// kinds' times (k_chain at 25,000 atoms, 3,800 items for 1,280 places: 270 us
+// by pair count alone, 237 by time; the order does not touch the sums).  At
+// 40,000 atoms, 9,700 items, no difference is left to gain
+constexpr size_t kChainByTime = 8192;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;

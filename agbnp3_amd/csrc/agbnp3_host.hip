@@ -613,7 +613,7 @@ int build_items(Pack &P) {
   // kinds (k_chain): both blocks heavy atoms only; hydrogen rows against heavy
   // columns (the hydrogen block is made the row block); anything else
   // (diagonal blocks, blocks mixing heavy atoms and hydrogens)
-  std::vector<std::pair<int4, long long>> cit;
+  std::vector<std::pair<int4, int>> cit;     // with its relative time
   for (const auto &fe : csys)
     for (int p = fe.first; p < fe.second; p++)
       for (int q = p; q < fe.second; q++) {
@@ -626,15 +626,21 @@ int build_items(Pack &P) {
         // columns in chunks of chain_chunk (64 or 128; 0: the whole block)
         const int step = P.tune.chain_chunk > 0 && P.tune.chain_chunk < 256 ? P.tune.chain_chunk / 64 : 4;
         const int ncol = csize[it.y], nch = (ncol + 63) / 64;
+        // relative time of a pair by kind: general, heavy x heavy of two types or of one, hydrogen rows with and without vdW terms
+        const int cost = it.z == 0 ? 9 : it.z == 1 ? (cblk[p].x == cblk[q].x ? 5 : 8) : (it.z == 2 ? 5 : 4);
         for (int c0 = 0; c0 < nch; c0 += step) {
           const int c1 = std::min(nch, c0 + step);
           int4 ci = it;
           ci.w = c0 | (c1 << 4);
-          cit.push_back({ci, (long long)csize[it.x] * std::min(ncol - 64 * c0, 64 * (c1 - c0))});
+          cit.push_back({ci, cost * (c1 - c0)});
         }
       }
-  std::stable_sort(cit.begin(), cit.end(), [](const std::pair<int4, long long> &a, const std::pair<int4, long long> &b) {
-    return a.second > b.second;
+  // longest first where the launch's end counts; in long launches only full
+  // items before cut ones, so that those in flight together share their row blocks
+  const bool by_time = cit.size() <= kChainByTime;
+  std::stable_sort(cit.begin(), cit.end(), [&](const std::pair<int4, int> &a, const std::pair<int4, int> &b) {
+    if (by_time) return a.second > b.second;
+    return (a.first.w >> 4) - (a.first.w & 15) > (b.first.w >> 4) - (b.first.w & 15);
   });
   std::vector<int4> chain(cit.size());
   for (size_t k = 0; k < cit.size(); k++) chain[k] = cit[k].first;
