@@ -774,10 +774,9 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
 // the second stream and its events
 int make_side(Pack &P) {
   HIPCHK(hipStreamCreateWithFlags(&P.side, hipStreamNonBlocking));
-  HIPCHK(hipEventCreateWithFlags(&P.ev_fork, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&P.ev_join, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&P.ev_fork2, hipEventDisableTiming));
-  HIPCHK(hipEventCreateWithFlags(&P.ev_join2, hipEventDisableTiming));
+  // (the streams are one device's: no fence towards the host)
+  for (hipEvent_t *e : {&P.ev_fork, &P.ev_join, &P.ev_fork2, &P.ev_join2})
+    HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming | hipEventDisableSystemFence));
   return AGBNP_OK;
 }
 
