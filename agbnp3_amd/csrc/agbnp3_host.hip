@@ -235,6 +235,8 @@ struct Pack {
   // pinned host staging, which the first and last kernels of a host-API call
   // read and write themselves: outputs, coordinates, status and counters (5)
   double *hstage = nullptr;
+  unsigned long long *hstat = nullptr; // pinned: status word and counters 0..3 of the last call
+  std::vector<void *> pinned;          // what the two lie in
   bool host_status = false;            // the last call put its status there
   // timing mode: one event set per recorded call, averaged when read back
   std::vector<std::vector<hipEvent_t>> ev_sets;
@@ -407,8 +409,10 @@ void free_pack(Pack &P) {
   P.allocs.clear();
   P.item_allocs.clear();
   P.sg_allocs.clear();
-  if (P.hstage) (void)hipHostFree(P.hstage);
+  for (void *p : P.pinned) (void)hipHostFree(p);
+  P.pinned.clear();
   P.hstage = nullptr;
+  P.hstat = nullptr;
   for (auto &set : P.ev_sets)
     for (hipEvent_t e : set) (void)hipEventDestroy(e);
   P.ev_sets.clear();
@@ -782,8 +786,21 @@ int make_side(Pack &P) {
 
 // the pack's own per-call state and host-API staging, on first use (calls
 // from agbnp3_ener_static use the library's static scratch instead)
-int ensure_call_state(Pack &P) {
+constexpr size_t kHstatBytes = 256;    // (the staging behind it starts on a line)
+int ensure_call_state(Pack &P, bool host_api = false) {
   Dev &d = P.d;
+  // pinned memory: the call's status and counters, and the host API's staging
+  // behind them (calls on device pointers do without those megabytes)
+  if (host_api ? !P.hstage : !P.hstat) {
+    const size_t stage = host_api ? (18 * (size_t)P.n + 7 * (size_t)P.nsys) * sizeof(double) : 0;
+    char *blk = nullptr;
+    HIPCHK(hipHostMalloc((void **)&blk, kHstatBytes + stage, hipHostMallocDefault));
+    P.pinned.push_back(blk);
+    memset(blk, 0, kHstatBytes);
+    if (!P.hstat) P.hstat = reinterpret_cast<unsigned long long *>(blk);
+    if (host_api) P.hstage = reinterpret_cast<double *>(blk + kHstatBytes);
+  }
+  d.hstat = P.hstat;
   if (P.call_block && d.nchain_items <= P.call_nchain && P.call_ndpart() <= P.call_dpart) return AGBNP_OK;
   if (P.call_block) {            // more items than the block holds (another launch shape)
     HIPCHK(hipStreamSynchronize(P.stream));
@@ -793,7 +810,7 @@ int ensure_call_state(Pack &P) {
   }
   const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
   const size_t nn = std::max(P.n, 1);
-  const size_t outs = 15 * nn + 7 * (size_t)P.nsys, stage = (outs + 3 * nn + 8) * sizeof(double);
+  const size_t outs = 15 * nn + 7 * (size_t)P.nsys;
   char *blk = nullptr;
   if (hipMalloc((void **)&blk, bytes + outs * sizeof(double)) != hipSuccess) {
     errprint("agbnp3: device allocation of %zu bytes failed\n", bytes + outs * sizeof(double));
@@ -805,11 +822,6 @@ int ensure_call_state(Pack &P) {
   carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
   P.dout = reinterpret_cast<double *>(blk + bytes);
   HIPCHK(hipMemset(d.ws_part, 0, sizeof(double) * std::max(d.nws, 1)));
-  if (!P.hstage) {
-    HIPCHK(hipHostMalloc((void **)&P.hstage, stage, hipHostMallocDefault));
-    memset(P.hstage, 0, stage);
-  }
-  d.hstat = reinterpret_cast<unsigned long long *>(P.hstage + 15 * (size_t)P.n + 7 * (size_t)P.nsys + 3 * (size_t)P.n);
   // (a pack that is only copied into a batch, or called through
   // agbnp3_ener_static, never comes here: no stream for it)
   if (!P.side && P.n >= kSideAtoms && make_side(P) != AGBNP_OK) return AGBNP_ERR;
@@ -1119,7 +1131,7 @@ void adapt_cap(Pack &P, int maxrow) {
 // overflowed, copy the outputs back.
 int pack_ener_host(Pack &P, const double *x, const double *y, const double *z, double *out /* 15n + 7 nsys */,
                    const char *who) {
-  if (ensure_call_state(P) != AGBNP_OK) return AGBNP_ERR;
+  if (ensure_call_state(P, true) != AGBNP_OK) return AGBNP_ERR;
   const size_t n = P.n;
   double *h = P.hstage;
   double *hin = h + 15 * n + 7 * (size_t)P.nsys;
@@ -1738,7 +1750,7 @@ int agbnp3_ener(int tag, int init, float_i *x, float_i *y, float_i *z, float_i *
   // library (agbnp3.h); the engine's boundary arrays are double either way
   std::vector<double> xin, yin, zin;
   const double *xd = as_double(x, n, xin), *yd = as_double(y, n, yin), *zd = as_double(z, n, zin);
-  if (ensure_call_state(I->p) != AGBNP_OK) return AGBNP_ERR;
+  if (ensure_call_state(I->p, true) != AGBNP_OK) return AGBNP_ERR;
   double *h = I->p.hstage;    // outputs land at the start of the staging area
   if (pack_ener_host(I->p, xd, yd, zd, h, "agbnp3_ener()") != AGBNP_OK) {
     errprint("agbnp3_ener(): error in agbnp3_total_energy().\n");
