@@ -169,10 +169,15 @@ __device__ __forceinline__ void block_bbox(const float4 *pos, int a0, int count,
                                            float *hi) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   float l[3] = {INFINITY, INFINITY, INFINITY}, h[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (int k = t; k < count; k += 1024) {
-    const float4 p = pos[a0 + k];
-    l[0] = fminf(l[0], p.x); l[1] = fminf(l[1], p.y); l[2] = fminf(l[2], p.z);
-    h[0] = fmaxf(h[0], p.x); h[1] = fmaxf(h[1], p.y); h[2] = fmaxf(h[2], p.z);
+  for (int k0 = t; k0 < count; k0 += 4 * 1024) {     // (four loads in flight; an atom met twice changes nothing)
+    float4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) p[u] = pos[a0 + min(k0 + 1024 * u, count - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      l[0] = fminf(l[0], p[u].x); l[1] = fminf(l[1], p[u].y); l[2] = fminf(l[2], p[u].z);
+      h[0] = fmaxf(h[0], p[u].x); h[1] = fmaxf(h[1], p[u].y); h[2] = fmaxf(h[2], p[u].z);
+    }
   }
 #pragma unroll
   for (int k = 0; k < 3; k++) {
@@ -226,11 +231,17 @@ __device__ __forceinline__ void bin_atoms(const GridParams &g, const float4 *pos
   const int ncell = g.ncell;
   for (int c = t; c < ncell; c += 1024) cnt[c] = 0;
   __syncthreads();
-  for (int k = t; k < count; k += 1024) {
-    const float4 p = pos[a0 + k];
-    const int c = cell_index(g, p.x, p.y, p.z);
-    cell_of[a0 + k] = c;
-    atomicAdd(&cnt[c], 1);
+  for (int k0 = t; k0 < count; k0 += 4 * 1024) {     // four loads in flight
+    float4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) p[u] = pos[a0 + min(k0 + 1024 * u, count - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (k0 + 1024 * u < count) {
+        const int c = cell_index(g, p[u].x, p[u].y, p[u].z);
+        cell_of[a0 + k0 + 1024 * u] = c;
+        atomicAdd(&cnt[c], 1);
+      }
   }
   __syncthreads();
   // exclusive scan of cnt over the cells, contiguous cells per thread
@@ -261,10 +272,13 @@ __device__ __forceinline__ void bin_atoms(const GridParams &g, const float4 *pos
   }
   if (t == 0) start[ncell] = a0 + count;
   __syncthreads();
-  for (int k = t; k < count; k += 1024) {
-    const int c = cell_of[a0 + k];
-    const int slot = atomicAdd(&cnt[c], 1);
-    out[slot] = a0 + k;
+  for (int k0 = t; k0 < count; k0 += 4 * 1024) {
+    int c[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) c[u] = cell_of[a0 + min(k0 + 1024 * u, count - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (k0 + 1024 * u < count) out[atomicAdd(&cnt[c[u]], 1)] = a0 + k0 + 1024 * u;
   }
   if (!sorted) return;
   __syncthreads();

@@ -112,25 +112,29 @@ void launch_cells(const Dev &d, hipStream_t s) {
 // cutoff is among those candidates, so later calls re-test and re-sort just
 // the candidates with the same FP32 arithmetic and get the same list as a
 // full rebuild.  k_guard decides on the device (graph replays included).
-constexpr int kNbWaves = 4;
+// Bound: a row's chain of dependent loads (atom of a cell slot, its position)
+// and, in the sort, of LDS reads.  Four steps' loads in flight and one 64-bit
+// key per entry, its reads eight ahead: 2,000 atoms 12.2 -> 7.0 us, 6,000 21.0
+// -> 9.2, 25,000 22.1 -> 15.1, 24 x 6000 89 -> 63.  (Positions kept in cell
+// order by k_cells: 8.4 us at 6,000, but k_cells, one block, 7.8 -> 12.2.)
+constexpr int kNbWaves = 4, kNbAhead = 4;
 
 template <int CAP>
 __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
 #pragma clang fp contract(off)
-  __shared__ float sd2[kNbWaves][CAP];
-  __shared__ int sj[kNbWaves][CAP];
+  // a row's entries as one key: d2 >= 0, so its bits order as the number
+  __shared__ unsigned long long key[kNbWaves][CAP];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int h = blockIdx.x * kNbWaves + w;
-  const bool active = h < d.nh;             // wave-uniform
-  const int i = active ? d.hrow[h] : 0;
+  if (h >= d.nh) return;                    // wave-uniform (no block barrier follows)
+  const int i = d.hrow[h];
   const int sys = d.asys[i];
   const float4 pi = d.pos[i];
   const bool reuse = d.skin > 0.f;
   const bool rebuild = !reuse || d.nbl_state[2] != 0;
   int cnt = 0;
   // exact test of pair (i, j); the candidate test (reuse) on the same d2
-  auto test = [&](int j, bool want_cand, bool &pass, bool &cpass, float &d2) {
-    const float4 pj = d.pos[j];
+  auto test = [&](const float4 &pj, bool want_cand, bool &pass, bool &cpass, float &d2) {
     const float ex = __fsub_rn(pj.x, pi.x), ey = __fsub_rn(pj.y, pi.y), ez = __fsub_rn(pj.z, pi.z);
     d2 = __fadd_rn(__fadd_rn(__fmul_rn(ex, ex), __fmul_rn(ey, ey)), __fmul_rn(ez, ez));
     const float u = __fmul_rn(__fadd_rn(pi.w, pj.w), kNbOffset);
@@ -144,38 +148,43 @@ __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
     const unsigned long long m = __ballot(pass);
     if (pass) {
       const int slot = cnt + __popcll(m & ((1ull << lane) - 1ull));
-      if (slot < CAP) { sd2[w][slot] = d2; sj[w][slot] = j; }
+      if (slot < CAP) key[w][slot] = (unsigned long long)__float_as_uint(d2) << 32 | (unsigned)j;
     }
     cnt += __popcll(m);
   };
-  if (active && rebuild) {
+  if (rebuild) {
     const GridParams g = d.grid[sys];
     const int *cstart = d.cell_start + (size_t)sys * (kMaxCells + 1);
     int *cand = reuse ? d.cand_nbr + (size_t)h * kCandCap : nullptr;
     int ccnt = 0;
     int cx, cy, cz;
     cell_coords(g, pi.x, pi.y, pi.z, cx, cy, cz);
-    // candidates gathered 64 at a time over the whole stencil; the (d2, j)
-    // sort below makes the list independent of the order of enumeration
+    // candidates over the whole stencil, kNbAhead steps of 64 in flight; the
+    // (d2, j) sort below makes the list independent of the order of enumeration
     int start[9], off[9];
     const int total = stencil_segments(g, cstart, cx, cy, cz, start, off);
-    for (int base = 0; base < total; base += 64) {
-      const int k = base + lane;
-      bool pass = false, cpass = false;
-      int j = -1;
-      float d2 = 0.f;
-      if (k < total) {
-        j = d.cell_atoms[stencil_slot(start, off, k)];
-        if (j > i) test(j, reuse, pass, cpass, d2);
-      }
-      keep(pass, j, d2);
-      if (reuse) {
-        const unsigned long long mc = __ballot(cpass);
-        if (cpass) {
-          const int slot = ccnt + __popcll(mc & ((1ull << lane) - 1ull));
-          if (slot < kCandCap) cand[slot] = j;
+    for (int base = 0; base < total; base += 64 * kNbAhead) {
+      int j[kNbAhead];
+      float4 pj[kNbAhead];
+#pragma unroll
+      for (int u = 0; u < kNbAhead; u++) j[u] = d.cell_atoms[stencil_slot(start, off, min(base + 64 * u + lane, total - 1))];
+#pragma unroll
+      for (int u = 0; u < kNbAhead; u++) pj[u] = d.pos[j[u]];
+#pragma unroll
+      for (int u = 0; u < kNbAhead; u++) {
+        if (base + 64 * u >= total) break;             // wave-uniform
+        bool pass = false, cpass = false;
+        float d2 = 0.f;
+        if (base + 64 * u + lane < total && j[u] > i) test(pj[u], reuse, pass, cpass, d2);
+        keep(pass, j[u], d2);
+        if (reuse) {
+          const unsigned long long mc = __ballot(cpass);
+          if (cpass) {
+            const int slot = ccnt + __popcll(mc & ((1ull << lane) - 1ull));
+            if (slot < kCandCap) cand[slot] = j[u];
+          }
+          ccnt += __popcll(mc);
         }
-        ccnt += __popcll(mc);
       }
     }
     if (reuse && lane == 0) {
@@ -187,7 +196,7 @@ __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
         d.nbl_state[3] += 1;       // rebuilds since reuse was set
       }
     }
-  } else if (active) {
+  } else {
     const int nc = d.cand_nne[h];
     const int *cand = d.cand_nbr + (size_t)h * kCandCap;
     for (int base = 0; base < nc; base += 64) {
@@ -197,7 +206,7 @@ __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
       float d2 = 0.f;
       if (k < nc) {
         j = cand[k];
-        test(j, false, pass, cpass, d2);
+        test(d.pos[j], false, pass, cpass, d2);
       }
       keep(pass, j, d2);
     }
@@ -207,17 +216,13 @@ __global__ __launch_bounds__(64 * kNbWaves) void k_nblist(Dev d) {
     if (lane == 0) atomicOr(d.status, ST_NBLIST_OVERFLOW);
     m = CAP;
   }
-  __syncthreads();
-  if (!active) return;
+  wave_sync();
   for (int e = lane; e < m; e += 64) {
-    const float de = sd2[w][e];
-    const int je = sj[w][e];
+    const unsigned long long ke = key[w][e];
     int rank = 0;
-    for (int f = 0; f < m; f++) {
-      const float df = sd2[w][f];
-      rank += (df < de) || (df == de && sj[w][f] < je);
-    }
-    d.nbr[(size_t)h * d.cap + rank] = je;
+#pragma unroll 8
+    for (int f = 0; f < m; f++) rank += key[w][f] < ke;
+    d.nbr[(size_t)h * d.cap + rank] = (int)(unsigned)ke;
   }
   if (lane == 0) d.nne[h] = m;
 }
