@@ -458,10 +458,10 @@ struct ChainChunk {
 
 // CM_CULL (large solutes): a wave passes over the chunks past the tables' end.
 // CM_GROUP: where a CU holds one item at a time (one wave per SIMD), the pairs of
-// a column step (two steps with one row per lane) are met first, tested for
+// two column steps (four with one row per lane) are met first, tested for
 // the band with one wave-uniform branch, and read the tables together: a
 // divergent branch per lookup serialises the lookups' LDS reads (2,000 atoms:
-// 76 -> 66 us).  With several items per CU their waves fill those waits, and
+// 76 -> 60 us; half as many steps 66, twice as many 64).  With several items per CU their waves fill those waits, and
 // taking the lookups one by one is as fast or faster (150,000 atoms: 7.1 ms
 // against 7.3).
 template <int KIND, bool QUIRK, int MODE>
@@ -474,7 +474,7 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
   constexpr int NW = 4 / NR;           // waves on one chunk
   constexpr int kUnroll = 3 - NR;      // column steps unrolled: 2 with one row, 1 with two
   constexpr bool GROUP = MODE == CM_GROUP;
-  constexpr int NS = GROUP ? kUnroll : 1;                  // column steps of a group
+  constexpr int NS = GROUP ? 2 * kUnroll : 1;              // column steps of a group
   constexpr bool kOne = KIND == CK_HX || KIND == CK_HX0;   // one direction: k (hydrogen) <- j
   constexpr bool kTwo = KIND == CK_HH || KIND == CK_GEN;   // two lookups (CK_HHS: one serves both directions)
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
