@@ -49,6 +49,10 @@ constexpr int kChainGroupItems = 1024;
 // by pair count alone, 237 by time; the order does not touch the sums).  At
 // 40,000 atoms, 9,700 items, no difference is left to gain
 constexpr size_t kChainByTime = 8192;
+// most items of a chain rule by row groups (k_chain_split; a call of 4,000
+// atoms, 155 items, 302 -> 268 us; with up to 512, 6,000 atoms 315 -> 327), and
+// most of its blocks for which a front takes four pairs at a time
+constexpr int kSplitItems = 256, kSplitSets = 6, kSplitFour = 256;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;
@@ -218,6 +222,13 @@ struct Dev {
   // quantities x 256 atoms (FP32 tile sums, [item][side][q][256]); per block
   // the (item, side) slots holding its atoms' sums, in a fixed order
   float *chpart;
+  // the chain rule by row groups (split_on): blocks (item << 2 | row group, or
+  // chunk parity << 1 | half of the rows), and per item kSplitSets sets of 8
+  // quantities x 256 atoms: its column sums by row group, then (4, 5) its row
+  // sums by parity; chain_sets: column sets, + 8 with a second parity
+  int split_on, nchain_sub;
+  const int *chain_sub, *chain_sets;
+  float *chsplit;
   int *ch_done;          // [nchain]: item evaluated this call (hybrid surrogate calls skip items)
   int *ch_flag;          // [4 ncblk]: 64-atom chunk holds an out-of-range atom (hybrid calls)
   const int *ch_cstart;  // [8][ncblk + 1]: per summed quantity, each block's run of ch_contrib

@@ -225,11 +225,14 @@ struct Pack {
   bool dt = false;                     // descreening by tiles (unless a surrogate is attached)
   long long ndpart = 0;                // its tile sums
   size_t call_ndpart() const { return dt ? (size_t)ndpart : 0; }
+  bool split = false;                  // chain rule by row groups (unless a surrogate is attached)
+  size_t call_nsplit() const { return split ? (size_t)d.nchain_items * kSplitSets * 2048 : 0; }
   // per-call working state (carve_call_state) and the host-API staging,
   // allocated by the first call that needs them (ensure_call_state), so an
   // instance evaluated only through agbnp3_ener_static never holds them
   void *call_block = nullptr;
   int call_nchain = 0;                 // chain-rule items the block's partial sums hold
+  size_t call_split = 0;               // numbers of their sums by row groups
   size_t call_dpart = 0;               // descreening tile sums it holds
   double *dout = nullptr;                                  // outputs: 15n + 7 nsys
   // pinned host staging, which the first and last kernels of a host-API call
@@ -648,6 +651,19 @@ int build_items(Pack &P) {
   });
   std::vector<int4> chain(cit.size());
   for (size_t k = 0; k < cit.size(); k++) chain[k] = cit[k].first;
+  // the same by row groups, where the items are few and no shape was asked for
+  // (whole blocks only: every chunk of an item's columns is then written)
+  P.split = P.tune.chain_chunk == 0 && (int)chain.size() <= kSplitItems;
+  std::vector<int> sub, sets;
+  for (int k = 0; P.split && k < (int)chain.size(); k++) {
+    const int4 &it = chain[k];
+    const bool one_row = it.z == 0 || (it.z == 1 && cblk[it.x].x != cblk[it.y].x);     // rows per lane (k_chain)
+    const int groups = (csize[it.x] + (one_row ? 63 : 127)) / (one_row ? 64 : 128), nch = it.w >> 4;
+    const int parities = one_row || nch == 1 ? 1 : 2;
+    for (int p = 0; p < parities; p++)
+      for (int g = 0; g < groups; g++) sub.push_back(k << 2 | p << 1 | g);
+    sets.push_back(groups | (parities == 2 ? 8 : 0));
+  }
   // where each block's chain-rule sums are: (item, side) slots ordered by the
   // other block's place in its system, row side first, so that a batch member
   // adds its partial sums in the order its own instance does
@@ -707,6 +723,7 @@ int build_items(Pack &P) {
       upload(P.item_allocs, &d.desc_items, desc) || upload(P.item_allocs, &d.dt_items, dt) || upload(P.item_allocs, &d.chain_items, chain) ||
       upload(P.item_allocs, &d.cperm, cperm) || upload(P.item_allocs, &d.cblk, cblk) ||
       upload(P.item_allocs, &d.ch_cstart, ch_cstart) || upload(P.item_allocs, &d.ch_contrib, ch_contrib) ||
+      upload(P.item_allocs, &d.chain_sub, sub) || upload(P.item_allocs, &d.chain_sets, sets) ||
       upload(P.item_allocs, &d.gb_items, gbi) || upload(P.item_allocs, &d.gb_eslot, gbs))
     return AGBNP_ERR;
   d.rows = rows;
@@ -715,6 +732,7 @@ int build_items(Pack &P) {
   d.ndt_items = (int)dt.size();
   d.dt_run = desc_cols / 256;
   d.nchain_items = (int)chain.size();
+  d.nchain_sub = (int)sub.size();
   d.ncblk = (int)cblk.size();
   d.ngb_items = (int)gbi.size();
   return AGBNP_OK;
@@ -727,7 +745,7 @@ int build_items(Pack &P) {
 // on a 256-byte boundary of one block; with base == nullptr only the size is
 // computed.  The neighbour-list rows are `cap` wide.
 size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_, int nablk, int ntile, int cap,
-                        int nchain, size_t ndpart) {
+                        int nchain, size_t nsplit, size_t ndpart) {
   const size_t n = std::max(n_, 1), nh = std::max(nh_, 1), nws = std::max(nws_, 1);
   size_t off = 0;
   auto take = [&](auto *&ptr, size_t count) {
@@ -770,6 +788,7 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   take(d.epart, (size_t)EP_COUNT * std::max(nablk, 1));
   take(d.dpart, ndpart);
   take(d.chpart, (size_t)nchain * 2 * 8 * 256);
+  take(d.chsplit, nsplit);
   take(d.ch_done, (size_t)nchain);
   take(d.ch_flag, 4 * (size_t)std::max(d.ncblk, 1));
   return (off + 255) & ~(size_t)255;
@@ -801,14 +820,16 @@ int ensure_call_state(Pack &P, bool host_api = false) {
     if (host_api) P.hstage = reinterpret_cast<double *>(blk + kHstatBytes);
   }
   d.hstat = P.hstat;
-  if (P.call_block && d.nchain_items <= P.call_nchain && P.call_ndpart() <= P.call_dpart) return AGBNP_OK;
+  if (P.call_block && d.nchain_items <= P.call_nchain && P.call_nsplit() <= P.call_split &&
+      P.call_ndpart() <= P.call_dpart) return AGBNP_OK;
   if (P.call_block) {            // more items than the block holds (another launch shape)
     HIPCHK(hipStreamSynchronize(P.stream));
     if (P.side) HIPCHK(hipStreamSynchronize(P.side));
     (void)hipFree(P.call_block);
     P.call_block = nullptr;
   }
-  const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
+  const size_t bytes = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_nsplit(),
+                                       P.call_ndpart());
   const size_t nn = std::max(P.n, 1);
   const size_t outs = 15 * nn + 7 * (size_t)P.nsys;
   char *blk = nullptr;
@@ -818,8 +839,10 @@ int ensure_call_state(Pack &P, bool host_api = false) {
   }
   P.call_block = blk;
   P.call_nchain = d.nchain_items;
+  P.call_split = P.call_nsplit();
   P.call_dpart = P.call_ndpart();
-  carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_ndpart());
+  carve_call_state(d, blk, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, 256, d.nchain_items, P.call_nsplit(),
+                                       P.call_ndpart());
   P.dout = reinterpret_cast<double *>(blk + bytes);
   HIPCHK(hipMemset(d.ws_part, 0, sizeof(double) * std::max(d.nws, 1)));
   // (a pack that is only copied into a batch, or called through
@@ -968,6 +991,7 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   d.skin = P.skin;
   d.reuse_every = P.reuse_every;
   d.dt_on = P.dt && !d.sg_on;
+  d.split_on = P.split && !d.sg_on;
   hipStream_t s = P.stream;
   const bool timed = !capturing && (P.options & AGBNP3_OPT_TIMING) != 0;
   int k = 0;
@@ -1705,13 +1729,14 @@ int agbnp3_ener_static(int tag, const double *x, const double *y, const double *
   if (scratch_base(dev, &base) != AGBNP_OK) return AGBNP_ERR;
   Dev d = P.d;
   const size_t need = carve_call_state(d, nullptr, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items,
-                                       P.call_ndpart());
+                                       P.call_nsplit(), P.call_ndpart());
   if (need > (size_t)AGBNP3_STATIC_SCRATCH_BYTES) {
     errprint("agbnp3_ener_static(): tag %d (%d atoms) needs %zu bytes of per-call state; the static scratch "
              "holds %zu (use agbnp3_ener_device).\n", tag, P.n, need, (size_t)AGBNP3_STATIC_SCRATCH_BYTES);
     return AGBNP_ERR;
   }
-  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items, P.call_ndpart());
+  carve_call_state(d, base, P.n, P.nh, P.nsys, d.nws, d.nablk, P.ntile, P.cap, d.nchain_items, P.call_nsplit(),
+                                       P.call_ndpart());
   d.hstat = nullptr;
   // no per-kernel timing events here (creating them allocates)
   const int saved = P.options;

@@ -442,6 +442,63 @@ __device__ __forceinline__ void chain_poly(const float4 &c, const float4 &e, flo
   dqx = fmaf(fmaf(e.z, u, e.y), u, e.x);
 }
 
+// one pair of a row atom k and a column atom j: x_j - x_k, 1 / d, and the table
+// coordinates (as computed, interval, fraction) of k <- j and, with two
+// lookups, j <- k
+struct ChainPair {
+  float ex, ey, ez, id, x1, x2, u1, u2;
+  int k1, k2;
+};
+template <int KIND>
+__device__ __forceinline__ ChainPair chain_meet(const float4 &pk, const float4 &pj, float cP, float cQ, bool pair) {
+  ChainPair m;
+  m.ex = pj.x - pk.x; m.ey = pj.y - pk.y; m.ez = pj.z - pk.z;
+  const float d2 = m.ex * m.ex + m.ey * m.ey + m.ez * m.ez;
+  m.id = __builtin_amdgcn_rsqf(d2);               // hardware reciprocal square root (1 ulp)
+  float dist = d2 * m.id;
+  if (KIND == CK_GEN) {
+    m.id = pair ? m.id : 0.f;
+    dist = pair ? dist : 1e6f;
+  }
+  m.x1 = dist * cQ;
+  chain_coord(m.x1, m.k1, m.u1);
+  if (KIND == CK_HH || KIND == CK_GEN) {
+    m.x2 = dist * cP;
+    chain_coord(m.x2, m.k2, m.u2);
+  }
+  return m;
+}
+// its terms: hgb and hvw (along x_j - x_k), Q4(k <- j) and Q4(j <- k), from
+// the interval records c1 and c2 (one direction: c2 the derivative record)
+template <int KIND, bool QUIRK>
+__device__ __forceinline__ void chain_terms(const ChainPair &m, const float4 &pj, const float4 &pp, float wk, float q2k,
+                                            float abk, bool kheavy, const float4 &c1, const float4 &c2, float &hgb,
+                                            float &hvw, float &q1, float &q2) {
+  float dq1, dq2;
+  if (KIND == CK_HX || KIND == CK_HX0) {
+    chain_poly(c1, c2, m.u1, q1, dq1);
+    const float t1 = pj.w * dq1 * m.id;
+    hgb = q2k * t1;
+    hvw = KIND == CK_HX ? abk * t1 : 0.f;
+    q2 = 0.f;
+    return;
+  }
+  chain_poly<QUIRK>(c1, m.u1, q1, dq1);           // k <- j (weight 0 unless j heavy)
+  if (KIND == CK_HH || KIND == CK_GEN) {
+    chain_poly<QUIRK>(c2, m.u2, q2, dq2);         // j <- k
+  } else {
+    q2 = q1;
+    dq2 = dq1;
+  }
+  if (KIND == CK_GEN) {
+    q2 = kheavy ? q2 : 0.f;
+    q1 = pp.z != 0.f ? q1 : 0.f;
+  }
+  const float t1 = pj.w * dq1 * m.id, t2 = wk * dq2 * m.id;
+  hgb = fmaf(q2k, t1, pp.x * t2);
+  hvw = fmaf(abk, t1, pp.y * t2);
+}
+
 enum : int { CM_PLAIN = 0, CM_GROUP = 1, CM_CULL = 2 };
 
 // per 64-column chunk: the columns' records, and once every wave is past the
@@ -552,60 +609,24 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
     const int c = cbeg + cp + NR * ci;
     float ca[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (c < cend && ((reach >> c) & 1u)) {
-      struct Pair {
-        float ex, ey, ez, id, x1, x2, u1, u2;
-        int k1, k2;
-      };
       auto meet = [&](int k, int col, const float4 &pj, const float4 &pp) {
-        Pair m;
-        m.ex = pj.x - pk[k].x; m.ey = pj.y - pk[k].y; m.ez = pj.z - pk[k].z;
-        const float d2 = m.ex * m.ex + m.ey * m.ey + m.ez * m.ez;
-        m.id = __builtin_amdgcn_rsqf(d2);               // hardware reciprocal square root (1 ulp)
-        float dist = d2 * m.id;
-        if (KIND == CK_GEN) {
-          // the self pair of a diagonal block, padding rows, hydrogen-hydrogen
-          // pairs: no weight, and a distance past the tables (zero interval)
-          const bool pair = kok[k] && (kheavy[k] || pp.z != 0.f) && !(diag && c * 64 + col == rr[k]);
-          m.id = pair ? m.id : 0.f;
-          dist = pair ? dist : 1e6f;
-        }
-        m.x1 = dist * cQ;
-        chain_coord(m.x1, m.k1, m.u1);
-        if (!GROUP) chain_fix(m.x1, pk[k], pj, RQ, dxinv, m.k1, m.u1);
-        if (kTwo) {
-          m.x2 = dist * cP;
-          chain_coord(m.x2, m.k2, m.u2);
-          if (!GROUP) chain_fix(m.x2, pj, pk[k], RP, dxinv, m.k2, m.u2);
+        // the self pair of a diagonal block, padding rows, hydrogen-hydrogen
+        // pairs: no weight, and a distance past the tables (zero interval)
+        const bool pair = KIND != CK_GEN || (kok[k] && (kheavy[k] || pp.z != 0.f) && !(diag && c * 64 + col == rr[k]));
+        ChainPair m = chain_meet<KIND>(pk[k], pj, cP, cQ, pair);
+        if (!GROUP) {
+          chain_fix(m.x1, pk[k], pj, RQ, dxinv, m.k1, m.u1);
+          if (kTwo) chain_fix(m.x2, pj, pk[k], RP, dxinv, m.k2, m.u2);
         }
         return m;
       };
-      auto add = [&](int k, const Pair &m, const float4 &pj, const float4 &pp, const float4 &c1, const float4 &c2) {
-        float hgb, hvw = 0.f, q1, dq1;
+      auto add = [&](int k, const ChainPair &m, const float4 &pj, const float4 &pp, const float4 &c1, const float4 &c2) {
+        float hgb, hvw, q1, q2;
+        chain_terms<KIND, QUIRK>(m, pj, pp, wk[k], q2k[k], abk[k], kheavy[k], c1, c2, hgb, hvw, q1, q2);
         if (kOne) {
-          chain_poly(c1, c2, m.u1, q1, dq1);            // tab_cr holds tab_rc's derivatives
-          const float t1 = pj.w * dq1 * m.id;
-          hgb = q2k[k] * t1;
           ca[6] = fmaf(q2k[k], q1, ca[6]);
-          if (KIND == CK_HX) {
-            hvw = abk[k] * t1;
-            ca[7] = fmaf(abk[k], q1, ca[7]);
-          }
+          if (KIND == CK_HX) ca[7] = fmaf(abk[k], q1, ca[7]);
         } else {
-          float q2, dq2;
-          chain_poly<QUIRK>(c1, m.u1, q1, dq1);         // k <- j (weight 0 unless j heavy)
-          if (kTwo) {
-            chain_poly<QUIRK>(c2, m.u2, q2, dq2);       // j <- k
-          } else {
-            q2 = q1;
-            dq2 = dq1;
-          }
-          if (KIND == CK_GEN) {
-            q2 = kheavy[k] ? q2 : 0.f;
-            q1 = pp.z != 0.f ? q1 : 0.f;
-          }
-          const float t1 = pj.w * dq1 * m.id, t2 = wk[k] * dq2 * m.id;
-          hgb = fmaf(q2k[k], t1, pp.x * t2);
-          hvw = fmaf(abk[k], t1, pp.y * t2);
           rU[k] = fmaf(pp.x, q2, rU[k]);
           rV[k] = fmaf(pp.y, q2, rV[k]);
           ca[6] = fmaf(q2k[k], q1, ca[6]);
@@ -627,7 +648,7 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
 #pragma unroll 1
         for (int s = 0; s < 64; s += NS) {
           float4 pj[NS], pp[NS], c1[NS][NR], c2[NS][NR];
-          Pair m[NS][NR];
+          ChainPair m[NS][NR];
           float band = 0.f;
 #pragma unroll
           for (int t = 0; t < NS; t++) {
@@ -671,7 +692,7 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
           const float4 pj = ch[c].col.pos[col], pp = ch[c].col.par[col];
 #pragma unroll
           for (int k = 0; k < NR; k++) {
-            const Pair m = meet(k, col, pj, pp);
+            const ChainPair m = meet(k, col, pj, pp);
             float4 c2;
             if (kTwo || kOne) c2 = tab_cr[kTwo ? m.k2 : m.k1];
             add(k, m, pj, pp, tab_rc[m.k1], c2);
@@ -744,6 +765,215 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
   }
 }
 
+// ------------------------------------- chain rule of small calls, by row groups
+// The same sums (k_chain), where its items are fewer than the CUs and one
+// wave's 256 steps through its 64 rows (or 128 steps of two rows) are the
+// launch.  Those rows and the steps of a column through them fix the order of
+// every sum, so they are not cut; the work on a pair is spread over waves
+// instead.  A block takes one wave's share of an item: four waves (fronts) form
+// the terms of a batch of pairs, EACH of them each, and pass them through LDS
+// to a fifth that adds the rows' sums and a sixth that adds the columns' (its
+// lanes are columns, so nothing rotates), one batch behind.  Column sums of an
+// item's row groups, and row sums of its two chunk parities, leave apart and
+// k_chain_sum adds them in the order k_chain does.
+// Bound: a front's chain from the column's LDS read over the table reads to
+// its terms, once per batch.  Against k_chain: 61 atoms 20 -> 13 us, 613 57 ->
+// 24, 2,000 60 -> 26 (eight waves as fronts 30).
+constexpr int kSplitFronts = 4, kSplitWaves = kSplitFronts + 2;
+template <int REC>
+struct SplitLds {
+  float4 cpos[256], cpar[256];           // the columns (ChainChunk's records)
+  float4 rpos[2][64];                    // the rows: position,
+  float2 rpar[2][64];                    // q2ab and abrw
+  float4 ring[2][REC][64];               // per pair: hgb, hvw, Q4(k <- j), Q4(j <- k)
+};
+
+template <int KIND, bool QUIRK, int EACH>
+__device__ __forceinline__ void chain_split_item(const Dev &d, int it, int part, const int4 &item,
+                                                 const float4 *__restrict__ tab_rc, const float4 *__restrict__ tab_cr,
+                                                 SplitLds<kSplitFronts * EACH> &L) {
+  constexpr int NR = (KIND == CK_HH || KIND == CK_GEN) ? 1 : 2;      // rows per lane, as k_chain has them
+  constexpr bool kOne = KIND == CK_HX || KIND == CK_HX0;
+  constexpr bool kTwo = KIND == CK_HH || KIND == CK_GEN;
+  constexpr int kRec = kSplitFronts * EACH, kSteps = kRec / NR, kBatches = 64 / kSteps;     // of a batch, of a chunk
+  const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
+  const int rh = NR == 2 ? part & 1 : part, cp = NR == 2 ? part >> 1 : 0;
+  const int4 bp = d.cblk[item.x];
+  const bool diag = item.x == item.y;
+  const float dxinv = d.tdxinv;
+  const SysInfo &S = d.sys[bp.y];
+  const int hend = S.a0 + S.nh;
+  const float RP = d.pos[d.cperm[item.x * 256]].w, RQ = d.pos[d.cperm[item.y * 256]].w;
+  const float iRP = 1.0f / RP, iRQ = 1.0f / RQ;
+  const float cP = iRP * dxinv, cQ = iRQ * dxinv;
+  if (threadIdx.x < 256) {
+    const int j = d.cperm[item.y * 256 + threadIdx.x];
+    float4 p = make_float4(1e6f, 1e6f, 1e6f, 0.f);
+    float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (j >= 0) {
+      const float4 pj = d.pos[j];
+      const float hv = j < hend ? 1.f : 0.f;
+      p = make_float4(pj.x, pj.y, pj.z, hv != 0.f ? d.sp_f[j] * iRQ * iRQ * dxinv : 0.f);
+      q = make_float4(d.q2ab_f[j], d.abrw_f[j], hv, 0.f);
+    }
+    L.cpos[threadIdx.x] = p;
+    L.cpar[threadIdx.x] = q;
+  }
+  int rr[NR];
+  float4 pk[NR];
+  float wk[NR], q2k[NR], abk[NR];
+  bool kok[NR], kheavy[NR];
+#pragma unroll
+  for (int k = 0; k < NR; k++) {
+    rr[k] = NR == 2 ? rh * 128 + lane + 64 * k : rh * 64 + lane;
+    const int kr = d.cperm[item.x * 256 + rr[k]];
+    pk[k] = make_float4(-1e6f, -1e6f, -1e6f, 1.f);
+    wk[k] = 0.f; q2k[k] = 0.f; abk[k] = 0.f;
+    kok[k] = kr >= 0;
+    kheavy[k] = false;
+    if (kr >= 0) {
+      pk[k] = d.pos[kr];
+      q2k[k] = d.q2ab_f[kr];
+      abk[k] = d.abrw_f[kr];
+      kheavy[k] = kr < hend;
+      wk[k] = kheavy[k] ? d.sp_f[kr] * iRP * iRP * dxinv : 0.f;
+    }
+    if (role == 0) {
+      L.rpos[k][lane] = pk[k];
+      L.rpar[k][lane] = make_float2(q2k[k], abk[k]);
+    }
+  }
+  __syncthreads();
+  const int cbeg = (item.w & 15) + cp, cend = item.w >> 4;
+  const int nbatch = (cend - cbeg + NR - 1) / NR * kBatches;
+  float rg[NR][3], rv[NR][3], rU[NR], rV[NR];            // the fifth wave's row sums
+#pragma unroll
+  for (int k = 0; k < NR; k++)
+    rg[k][0] = rg[k][1] = rg[k][2] = rv[k][0] = rv[k][1] = rv[k][2] = rU[k] = rV[k] = 0.f;
+  float ca[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // the sixth wave's column sums
+#pragma unroll 1
+  for (int t = 0; t <= nbatch; t++) {
+    if (role < kSplitFronts) {
+      if (t < nbatch) {
+        const int c = cbeg + NR * (t / kBatches), s0 = t % kBatches * kSteps;
+        float4 pj[EACH], pp[EACH], c1[EACH], c2[EACH];
+        ChainPair m[EACH];
+        float band = 0.f;
+#pragma unroll
+        for (int r = 0; r < EACH; r++) {
+          const int k = NR == 2 ? r & 1 : 0, col = (lane - s0 - (EACH * role + r) / NR) & 63;
+          pj[r] = L.cpos[c * 64 + col];
+          pp[r] = L.cpar[c * 64 + col];
+          const bool pair = KIND != CK_GEN || (kok[k] && (kheavy[k] || pp[r].z != 0.f) && !(diag && c * 64 + col == rr[k]));
+          m[r] = chain_meet<KIND>(pk[k], pj[r], cP, cQ, pair);
+          band = fmaxf(band, fabsf(m[r].u1 - 0.5f));
+          if (kTwo) band = fmaxf(band, fabsf(m[r].u2 - 0.5f));
+        }
+        if (__builtin_expect(__ballot(band > kChainBand) != 0ull, 0)) {
+#pragma unroll
+          for (int r = 0; r < EACH; r++) {
+            const int k = NR == 2 ? r & 1 : 0;
+            chain_fix(m[r].x1, pk[k], pj[r], RQ, dxinv, m[r].k1, m[r].u1);
+            if (kTwo) chain_fix(m[r].x2, pj[r], pk[k], RP, dxinv, m[r].k2, m[r].u2);
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < EACH; r++) {
+          c1[r] = tab_rc[m[r].k1];
+          if (kTwo || kOne) c2[r] = tab_cr[kTwo ? m[r].k2 : m[r].k1];
+        }
+#pragma unroll
+        for (int r = 0; r < EACH; r++) {
+          const int k = NR == 2 ? r & 1 : 0;
+          float hgb, hvw, q1, q2;
+          chain_terms<KIND, QUIRK>(m[r], pj[r], pp[r], wk[k], q2k[k], abk[k], kheavy[k], c1[r], c2[r], hgb, hvw, q1, q2);
+          L.ring[t & 1][EACH * role + r][lane] = make_float4(hgb, hvw, q1, q2);
+        }
+      }
+    } else if (t > 0) {
+      const int c = cbeg + NR * ((t - 1) / kBatches), s0 = (t - 1) % kBatches * kSteps;
+      const float4 (*ring)[64] = L.ring[(t - 1) & 1];
+      if (role == kSplitFronts) {
+#pragma unroll
+        for (int r = 0; r < kRec; r++) {
+          const int k = NR == 2 ? r & 1 : 0, col = (lane - s0 - r / NR) & 63;
+          const float4 pj = L.cpos[c * 64 + col], h = ring[r][lane];
+          const float ex = pj.x - pk[k].x, ey = pj.y - pk[k].y, ez = pj.z - pk[k].z;
+          rg[k][0] = fmaf(h.x, ex, rg[k][0]); rg[k][1] = fmaf(h.x, ey, rg[k][1]); rg[k][2] = fmaf(h.x, ez, rg[k][2]);
+          if (KIND != CK_HX0) {
+            rv[k][0] = fmaf(h.y, ex, rv[k][0]); rv[k][1] = fmaf(h.y, ey, rv[k][1]); rv[k][2] = fmaf(h.y, ez, rv[k][2]);
+          }
+          if (!kOne) {
+            const float4 pp = L.cpar[c * 64 + col];
+            rU[k] = fmaf(pp.x, h.w, rU[k]);
+            rV[k] = fmaf(pp.y, h.w, rV[k]);
+          }
+        }
+      } else if (!diag) {
+        const float4 pj = L.cpos[c * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < kRec; r++) {
+          const int k = NR == 2 ? r & 1 : 0, row = (lane + s0 + r / NR) & 63;
+          const float4 pr = L.rpos[k][row], h = ring[r][row];
+          const float2 qa = L.rpar[k][row];
+          const float ex = pj.x - pr.x, ey = pj.y - pr.y, ez = pj.z - pr.z;
+          ca[0] = fmaf(-h.x, ex, ca[0]); ca[1] = fmaf(-h.x, ey, ca[1]); ca[2] = fmaf(-h.x, ez, ca[2]);
+          if (KIND != CK_HX0) {
+            ca[3] = fmaf(-h.y, ex, ca[3]); ca[4] = fmaf(-h.y, ey, ca[4]); ca[5] = fmaf(-h.y, ez, ca[5]);
+          }
+          ca[6] = fmaf(qa.x, h.z, ca[6]);
+          if (KIND != CK_HX0) ca[7] = fmaf(qa.y, h.z, ca[7]);
+        }
+        if (t % kBatches == 0) {                          // the chunk's last batch
+          float *o = d.chsplit + ((size_t)it * kSplitSets + rh) * 2048 + c * 64 + lane;
+#pragma unroll
+          for (int q = 0; q < 8; q++) {
+            if (KIND != CK_HX0 || q < 3 || q == 6) o[q * 256] = ca[q];
+            ca[q] = 0.f;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (role == kSplitFronts) {
+    float *pr = d.chsplit + ((size_t)it * kSplitSets + 4 + cp) * 2048;
+#pragma unroll
+    for (int k = 0; k < NR; k++) {
+      float *o = pr + rr[k];
+      o[0 * 256] = rg[k][0]; o[1 * 256] = rg[k][1]; o[2 * 256] = rg[k][2];
+      if (KIND != CK_HX0) {
+        o[3 * 256] = rv[k][0]; o[4 * 256] = rv[k][1]; o[5 * 256] = rv[k][2];
+      }
+      if (!kOne) {
+        o[6 * 256] = kheavy[k] ? rU[k] : 0.f;
+        o[7 * 256] = kheavy[k] ? rV[k] : 0.f;
+      }
+    }
+  }
+}
+
+template <bool QUIRK, int EACH>
+__global__ __launch_bounds__(64 * kSplitWaves) void k_chain_split(Dev d) {
+  __shared__ float4 tab_rc[kTblN], tab_cr[kTblN];
+  __shared__ SplitLds<kSplitFronts * EACH> L;
+  const int sub = d.chain_sub[blockIdx.x], it = sub >> 2, part = sub & 3;
+  const int4 item = d.chain_items[it];
+  const int4 bp = d.cblk[item.x], bq = d.cblk[item.y];
+  const int trc = bp.x * d.ntypes + bq.x, tcr = bq.x * d.ntypes + bp.x;
+  const bool one = item.z == CK_HX || item.z == CK_HX0;
+  for (int k = threadIdx.x; k < kTblN; k += 64 * kSplitWaves) {
+    const float4 v = d.ctab[(size_t)trc * kTblN + k];
+    tab_rc[k] = v;
+    tab_cr[k] = one ? chain_dpoly<QUIRK>(v) : d.ctab[(size_t)tcr * kTblN + k];
+  }
+  if (item.z == CK_HH && bp.x == bq.x) chain_split_item<CK_HHS, QUIRK, EACH>(d, it, part, item, tab_rc, tab_cr, L);
+  else if (item.z == CK_HH) chain_split_item<CK_HH, QUIRK, EACH>(d, it, part, item, tab_rc, tab_cr, L);
+  else if (item.z == CK_HX0) chain_split_item<CK_HX0, QUIRK, EACH>(d, it, part, item, tab_rc, tab_cr, L);
+  else if (item.z == CK_HX) chain_split_item<CK_HX, QUIRK, EACH>(d, it, part, item, tab_rc, tab_cr, L);
+  else chain_split_item<CK_GEN, QUIRK, EACH>(d, it, part, item, tab_rc, tab_cr, L);
+}
+
 // Chain-rule sums per atom: the partial sums of every item holding its block,
 // in the block's fixed slot order, added in FP64 and stored as the call's
 // fixed-point accumulators (no atomics; systems on the surrogate this call
@@ -762,7 +992,32 @@ __global__ __launch_bounds__(256) void k_chain_sum(Dev d) {
   const int *cs = d.ch_cstart + (size_t)q * (d.ncblk + 1);     // the slots that hold quantity q
   const int c0 = cs[b], c1 = cs[b + 1];
   double acc = 0.0;
-  if (mode == 2) {
+  if (d.split_on) {
+    // an item's column sums by row groups and its row sums by chunk parities
+    // first, in FP32 in k_chain's order
+    const float *set = d.chsplit + q * 256 + threadIdx.x;
+    for (int c = c0; c < c1; c += 4) {
+      float v[4][4];
+      int m[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int e = d.ch_contrib[min(c + u, c1 - 1)], it = e >> 1, col = e & 1, n = d.chain_sets[it];
+        // sets 0 .. of a column, 4 and 5 of a row (the loads have no branches,
+        // so that all are in flight; what is past the count is left out)
+        const size_t at = ((size_t)it * kSplitSets + (col ? 0 : 4)) * 2048;
+        m[u] = c + u < c1 ? (col ? n & 7 : 1 + (n >> 3)) : 0;
+#pragma unroll
+        for (int g = 0; g < 4; g++) v[u][g] = set[at + (g < 2 ? g : (col ? g : 1)) * 2048];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        float t = m[u] > 0 ? v[u][0] : 0.f;
+#pragma unroll
+        for (int g = 1; g < 4; g++) t += m[u] > g ? v[u][g] : 0.f;
+        acc += (double)t;
+      }
+    }
+  } else if (mode == 2) {
     // only the items k_chain evaluated this call (the others hold another
     // call's sums)
     for (int c = c0; c < c1; c++) {
@@ -854,6 +1109,15 @@ void launch_chain(const Dev &d, const Tuning &t, hipStream_t s) {
     if (d.ncblk) hipLaunchKernelGGL(k_chain_flags, dim3(d.ncblk), dim3(256), 0, s, d);
   }
   const bool fixed = (d.options & 2) != 0;
+  if (d.split_on) {
+    // four pairs per front while every block has a CU to itself (half
+    // as many batches; 2,000 atoms, 190 blocks, call 224 -> 214 us; 4,000, 450 blocks, 268 -> 274)
+    const auto k = d.nchain_sub <= kSplitFour ? (fixed ? k_chain_split<false, 4> : k_chain_split<true, 4>)
+                                              : (fixed ? k_chain_split<false, 2> : k_chain_split<true, 2>);
+    hipLaunchKernelGGL(k, dim3(d.nchain_sub), dim3(64 * kSplitWaves), 0, s, d);
+    hipLaunchKernelGGL(k_chain_sum, dim3(d.ncblk, 8), dim3(256), 0, s, d);
+    return;
+  }
   auto k = fixed ? k_chain<false, CM_PLAIN> : k_chain<true, CM_PLAIN>;
   if (d.nchain_items <= kChainGroupItems) k = fixed ? k_chain<false, CM_GROUP> : k_chain<true, CM_GROUP>;
   else if (d.cull_chain) k = fixed ? k_chain<false, CM_CULL> : k_chain<true, CM_CULL>;

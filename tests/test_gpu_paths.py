@@ -1,8 +1,9 @@
 """Calls that a rule on sizes sends another way give the same results.
 
 Bitwise, the two routes of one call against each other: descreening by tiles
-(few work items) against the plain kernel; far columns skipped by boxes
-against none skipped.  Against the FP64 oracle: two atoms in one place, which
+(few work items) against the plain kernel; the chain rule by row groups (few
+work items) against the plain kernel; far columns skipped by boxes against
+none skipped.  Against the FP64 oracle: two atoms in one place, which
 the GB kernel's off-diagonal tiles meet without the pair mask, and water sites
 with more than 64 candidate atoms.
 """
@@ -48,6 +49,28 @@ def test_descreening_by_tiles_equals_the_plain_kernel(natoms, rows):
         tiles = inst.ener()
         inst.set_tuning(rows=rows, desc_chunk=512)
         assert_same(tiles, inst.ener(), natoms)
+    finally:
+        inst.delete()
+
+
+@pytest.mark.parametrize("natoms,mixed,fixed", [(8, False, False), (61, False, True), (300, True, False),
+                                                (513, False, False), (1777, True, True), (2000, False, False),
+                                                (4100, True, False), (4700, False, True)])
+def test_chain_rule_by_row_groups_equals_the_plain_kernel(natoms, mixed, fixed):
+    """256 columns per item are what both routes use; asked for, they are the plain kernel's.  mixed: hydrogens with
+    vdW terms, and some with a heavy atom's radius."""
+    s = synth.generate(20260400 + natoms, natoms)
+    if mixed:
+        r, salpha = s.r.copy(), s.salpha.copy()
+        salpha[s.ihydrogen[::2]] = -0.1
+        heavy = np.setdiff1d(np.arange(natoms), s.ihydrogen)
+        r[s.ihydrogen[::5]] = r[heavy[0]]
+        s = dataclasses.replace(s, r=r, salpha=salpha)
+    inst = api.Instance(s, api.OPT_HB_FIXED | api.OPT_SPLINE_FIXED if fixed else 0)
+    try:
+        groups = inst.ener()
+        inst.set_tuning(chain_chunk=256)
+        assert_same(groups, inst.ener(), natoms)
     finally:
         inst.delete()
 
