@@ -111,6 +111,20 @@ __device__ __forceinline__ void slot_add(double *p, double v) { atomicAdd(p, v);
 __device__ __forceinline__ void slot_add(long long *p, double v) {
   atomicAdd((unsigned long long *)p, (unsigned long long)__double2ll_rn(v * kFix));
 }
+// The same for |v| < kSmall: at 1.5 x 2^20 a double's last place is 2^-32, so
+// an addition there rounds v to the fixed point, and the sum's bits less the
+// constant's are the integer: one addition and one subtraction instead of the
+// conversion's seven FP64 instructions, 12 times per member of every overlap.
+// 2,000 atoms: call 219 -> 216 us, 25,000 984 -> 977, 64 poses 800 -> 786.
+constexpr float kSmall = 524288.f;
+__device__ __forceinline__ void slot_add_small(double *p, double v) { atomicAdd(p, v); }
+__device__ __forceinline__ void slot_add_small(long long *p, double v) {
+  constexpr double c = 1572864.0;
+  atomicAdd((unsigned long long *)p,
+            (unsigned long long)(__builtin_bit_cast(long long, v + c) - __builtin_bit_cast(long long, c)));
+}
+// whether every active lane may add numbers of this sum of sizes as above
+__device__ __forceinline__ bool all_small(float big) { return __builtin_expect(__ballot(!(big < kSmall)) == 0ull, 1); }
 
 // Pass-B terms of one kept overlap of order N for each member k: the
 // derivatives of its self-volume and surface contributions with respect to
@@ -193,10 +207,21 @@ __device__ __forceinline__ void add_contrib(Lds &S, const OvlOut &o, const int (
       const float4 pk = S.p[mem[k]];
       sa[k] = sa_term(o, sign, pk.w, pk.x, pk.y, pk.z, S.r[mem[k]]);
     }
+    float big = o.Vp;
 #pragma unroll
-    for (int k = 1; k < N; k++) {
-      slot_add(&S.acc[0][mem[k]], wv);
-      slot_add(&S.acc[1][mem[k]], (double)sa[k]);
+    for (int k = 1; k < N; k++) big += fabsf(sa[k]);
+    if (all_small(big)) {
+#pragma unroll
+      for (int k = 1; k < N; k++) {
+        slot_add_small(&S.acc[0][mem[k]], wv);
+        slot_add_small(&S.acc[1][mem[k]], (double)sa[k]);
+      }
+    } else {
+#pragma unroll
+      for (int k = 1; k < N; k++) {
+        slot_add(&S.acc[0][mem[k]], wv);
+        slot_add(&S.acc[1][mem[k]], (double)sa[k]);
+      }
     }
   } else {
     float A_[N], X_[N], Y_[N], Z_[N], R_[N], WC[N], WV[N], WG[N];
@@ -213,8 +238,16 @@ __device__ __forceinline__ void add_contrib(Lds &S, const OvlOut &o, const int (
 #pragma unroll
         for (int v = 0; v < TG_N; v++) root[v] += (RT)out[v];
       } else {
+        float big = 0.f;
 #pragma unroll
-        for (int v = 0; v < TG_N; v++) slot_add(&S.acc[v][mem[k]], out[v]);
+        for (int v = 0; v < TG_N; v++) big += fabsf(out[v]);
+        if (all_small(big)) {
+#pragma unroll
+          for (int v = 0; v < TG_N; v++) slot_add_small(&S.acc[v][mem[k]], out[v]);
+        } else {
+#pragma unroll
+          for (int v = 0; v < TG_N; v++) slot_add(&S.acc[v][mem[k]], out[v]);
+        }
       }
     });
   }

@@ -4,8 +4,9 @@ Bitwise, the two routes of one call against each other: descreening by tiles
 (few work items) against the plain kernel; the chain rule by row groups (few
 work items) against the plain kernel; far columns skipped by boxes against
 none skipped.  Against the FP64 oracle: two atoms in one place, which
-the GB kernel's off-diagonal tiles meet without the pair mask, and water sites
-with more than 64 candidate atoms.
+the GB kernel's off-diagonal tiles meet without the pair mask, water sites
+with more than 64 candidate atoms, and overlap terms past the range of the
+tree's fast fixed-point conversion.
 """
 import dataclasses
 
@@ -117,5 +118,25 @@ def test_water_sites_with_more_than_64_candidates():
         out, ref = inst.ener(), oracle.Oracle(t).ener()
         assert abs(out["ehb"] - ref["ehb"]) <= 1e-5 * abs(ref["ehb"])
         assert rms(out["dehb"] - ref["dehb"]) <= G_RMS
+    finally:
+        inst.delete()
+
+
+@pytest.mark.parametrize("natoms", [61, 700])
+def test_overlap_terms_past_the_fast_conversion(natoms):
+    """Surface tensions that take some atoms' cavity terms past 2^19, and leave others' below it in the same waves.
+    FP32 terms: 1e-5 of the gradients' size, as the energies' bound."""
+    s = synth.generate(20260320 + natoms, natoms)
+    igamma = s.igamma.copy()
+    heavy = np.setdiff1d(np.arange(natoms), s.ihydrogen)
+    igamma[heavy[::3]] *= 1e7
+    s = dataclasses.replace(s, igamma=igamma)
+    inst = api.Instance(s)
+    try:
+        out, ref = inst.ener(), oracle.Oracle(s).ener()
+        assert np.abs(ref["decav"]).max() > 2.0 ** 20
+        assert rms(out["decav"] - ref["decav"]) <= 1e-5 * rms(ref["decav"])
+        for k in ("dgbdr", "dehb"):
+            assert rms(out[k] - ref[k]) <= G_RMS, k
     finally:
         inst.delete()
