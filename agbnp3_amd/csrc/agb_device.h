@@ -128,7 +128,10 @@ __device__ __forceinline__ unsigned *queue_head(unsigned *queue, int which) {
   return queue + which * kQueueSpread * kQueueStride;
 }
 __device__ __forceinline__ int first_item() { return (int)blockIdx.x; }
-__device__ __forceinline__ int next_item(unsigned *head, int *slot) {
+// (A grid with a block per item asks no head: the answer, a microsecond away
+// behind the block's own scatter, would only hold its place on the CU.)
+__device__ __forceinline__ int next_item(unsigned *head, int *slot, int count) {
+  if ((int)gridDim.x >= count) return count;
   __syncthreads();                       // the previous item is finished by all waves
   if (threadIdx.x == 0) {
     const unsigned S = min((unsigned)kQueueSpread, gridDim.x), x = blockIdx.x % S;
@@ -139,7 +142,8 @@ __device__ __forceinline__ int next_item(unsigned *head, int *slot) {
 }
 // the same in runs of `n` consecutive items (run u = items u n .. u n + n - 1)
 __device__ __forceinline__ int first_item_n(int n) { return (int)blockIdx.x * n; }
-__device__ __forceinline__ int next_item_n(unsigned *head, int *slot, int n) {
+__device__ __forceinline__ int next_item_n(unsigned *head, int *slot, int n, int count) {
+  if ((int)gridDim.x * n >= count) return count;
   __syncthreads();
   if (threadIdx.x == 0) {
     const unsigned S = min((unsigned)kQueueSpread, gridDim.x), x = blockIdx.x % S;

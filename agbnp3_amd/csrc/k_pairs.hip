@@ -62,7 +62,7 @@ __global__ __launch_bounds__(ROWS) void k_descreen(Dev d, const float4 *__restri
   // scalar arithmetic
   int staged = -1;
   for (int it0 = first_item(); it0 < d.ndesc_items;
-       it0 = next_item(queue_head(d.queue, Q_DESC), &slot)) {
+       it0 = next_item(queue_head(d.queue, Q_DESC), &slot, d.ndesc_items)) {
     const int it = __builtin_amdgcn_readfirstlane(it0);
     const int4 item = d.desc_items[it];
     const int i = d.row_perm[item.x * ROWS + threadIdx.x];
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(256, 4) void k_gbpair(Dev d) {
   __shared__ double ered[4];
   __shared__ int slot;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;   // wave w: every row, column chunk w
-  for (int it = first_item(); it < d.ngb_items; it = next_item(queue_head(d.queue, Q_GB), &slot)) {
+  for (int it = first_item(); it < d.ngb_items; it = next_item(queue_head(d.queue, Q_GB), &slot, d.ngb_items)) {
     const int4 tp = d.gb_items[it];      // rows [x, y), columns [z, w)
     const bool diag = tp.x == tp.z;
     const int nch = (tp.w - tp.z + 63) >> 6;
@@ -1061,7 +1061,7 @@ __global__ __launch_bounds__(256) void k_chain(Dev d) {
   if (d.sg_on && !*d.sg_any_plain) return;   // every system on the surrogate this call (grid-uniform)
   int staged_rc = -1, staged_cr = INT_MIN;     // nothing staged (keys are tables >= 0 or -1 - table)
   for (int it = first_item(); it < d.nchain_items;
-       it = next_item(queue_head(d.queue, Q_CHAIN), &slot)) {
+       it = next_item(queue_head(d.queue, Q_CHAIN), &slot, d.nchain_items)) {
     const int4 item = d.chain_items[it];
     const int4 bp = d.cblk[item.x], bq = d.cblk[item.y];
     if (d.sg_on) {

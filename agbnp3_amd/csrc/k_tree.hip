@@ -588,9 +588,14 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
   // pass B's first tier leaves the roots pass A queued to the second tier,
   // which takes pass A's list: both passes walk the same tree, so they
   // outgrow the same buffers
-  if (PB && list == 0 && d.tree_tier[h]) return true;  // block-uniform
-  const int i = d.hrow[h];
-  const int m = d.nne[h];
+  // (its header and row are loaded together, and then all that hangs on them:
+  // one by one, seven loads deep, they were a fifth of an average root's time)
+  int i = d.hrow[h], m = d.nne[h], tier = PB && list == 0 ? d.tree_tier[h] : 0, nb = 0;
+  if (tid > 0 && tid <= d.cap) nb = d.nbr[(size_t)h * d.cap + tid - 1];
+  asm volatile("" : "+v"(i), "+v"(m), "+v"(tier), "+v"(nb));
+  i = __builtin_amdgcn_readfirstlane(i);
+  m = __builtin_amdgcn_readfirstlane(m);
+  if (PB && list == 0 && __builtin_amdgcn_readfirstlane(tier)) return true;  // block-uniform
   // a root that outgrows these buffers: pass A's first tier queues it for the
   // second (and records that); past the second tier it is walked depth first,
   // in pass A by the caller, in pass B from a list
@@ -608,27 +613,35 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
     return false;
   }
   const float4 pr = d.pos[i];
-  for (int s = tid; s <= m; s += NT) {
-    const int at = s == 0 ? i : d.nbr[(size_t)h * d.cap + s - 1];
+  const int sys = PB ? d.asys[i] : 0;
+  auto stage = [&](int s, int at) {
     const float4 p = d.pos[at];
-    S.idx[s] = at;
-    S.p[s] = make_float4(p.x - pr.x, p.y - pr.y, p.z - pr.z, d.galpha[at]);   // root frame
+    const float ga = d.galpha[at];
+    float c[6];
     if (PB) {
-      S.q[s] = make_float4(p.w, d.deru_f[at], d.derv_f[at], d.derh_f[at]);
-      S.w[s] = make_float4(d.gammap_f[at], d.dervs_f[at], d.derus_f[at], 0.f);
+      c[0] = d.deru_f[at]; c[1] = d.derv_f[at]; c[2] = d.derh_f[at];
+      c[3] = d.gammap_f[at]; c[4] = d.dervs_f[at]; c[5] = d.derus_f[at];
+    }
+    S.idx[s] = at;
+    S.p[s] = make_float4(p.x - pr.x, p.y - pr.y, p.z - pr.z, ga);   // root frame
+    if (PB) {
+      S.q[s] = make_float4(p.w, c[0], c[1], c[2]);
+      S.w[s] = make_float4(c[3], c[4], c[5], 0.f);
     } else {
       S.r[s] = p.w;
     }
 #pragma unroll
     for (int v = 0; v < (PB ? TG_N : 2); v++) S.acc[v][s] = 0;
-  }
+  };
+  if (tid <= m) stage(tid, tid == 0 ? i : nb);
+  for (int s = tid + NT; s <= m; s += NT) stage(s, d.nbr[(size_t)h * d.cap + s - 1]);
+  const float df = PB ? d.sys[sys].df : 0.f;
   __syncthreads();
   using RT = typename std::conditional<PB, float, double>::type;
   RT root[TG_N];
 #pragma unroll
   for (int v = 0; v < TG_N; v++) root[v] = 0;
   unsigned nkept = 0, neval = 0;
-  const float df = d.sys[d.asys[i]].df;
   bool ovf = false;
   // order 2: the root with every list entry, one sibling group
   int n = 0;
@@ -753,7 +766,7 @@ __global__ __launch_bounds__(64 * kFirstWaves, PB ? 4 : 7) void k_tree_bfs(Dev d
   // their fixed-point scatters rarely meet on one atom
   const long long P = d.nh % 7919 ? 7919 : (d.nh % 7927 ? 7927 : 7933);
   unsigned long long tk = 0, te = 0;
-  for (int k0 = first_item_n(run); k0 < d.nh; k0 = next_item_n(head, &slot, run))
+  for (int k0 = first_item_n(run); k0 < d.nh; k0 = next_item_n(head, &slot, run, d.nh))
     for (int k = k0; k < min(k0 + run, d.nh); k++)
       tree_bfs_root<CAP, PB, kLevelCap, kFirstWaves>(d, S, (int)(((long long)k * P) % d.nh), 0, tk, te);
   add_tree_counts(d, PB, tk, te);
@@ -779,7 +792,7 @@ __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
   const int count = (int)d.counters[4];
   unsigned *head = queue_head(d.queue, PB ? Q_TREE_BB : Q_TREE_BA);
   unsigned long long tk = 0, te = 0;
-  for (int k = first_item(); k < count; k = next_item(head, &slot)) {
+  for (int k = first_item(); k < count; k = next_item(head, &slot, count)) {
     const int h = d.tree_ovf[k];
     const bool done = tree_bfs_root<CAP, PB, kLevelCapBig, kBigWaves>(d, S, h, 1, tk, te);
     if constexpr (!PB) {
