@@ -272,6 +272,7 @@ struct Dev {
                                        //     takes the same list), [5] unused
                                        // [6], [7] roots walked depth first (pass A, B)
   int *tree_ovf;                       // [2][nh] heavy rows of the roots queued for the second tier, for pass B's depth-first walk
+  uint2 *tree_cnt;                     // [nh] overlaps kept and evaluated by pass A's first tier (in A's memory, until k_q2ab)
   unsigned char *tree_tier;            // [nh] pass A's first tier: 0 walked there, 1 queued for the next
   double *volumep_raw, *sa_raw, *sa_f, *sp, *spe, *psvol, *gammap;   // [n]
   float *sp_f, *spe_f;                 // FP32 copies for pair kernels
@@ -345,7 +346,7 @@ struct Tuning {
   int desc_grid = 0;       // persistent blocks (0: one per item)
   int gb_grid = 0;
   int chain_grid = 0;
-  int tree_grid = 0;       // persistent blocks of the first overlap-tree tier (0: 16 per CU)
+  int tree_grid = 0;       // persistent blocks of the first overlap-tree tier (0: one per root)
 };
 
 // ---- launchers (kernel translation units) ------------------------------

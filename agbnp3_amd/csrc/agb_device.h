@@ -140,18 +140,6 @@ __device__ __forceinline__ int next_item(unsigned *head, int *slot, int count) {
   __syncthreads();
   return *slot;
 }
-// the same in runs of `n` consecutive items (run u = items u n .. u n + n - 1)
-__device__ __forceinline__ int first_item_n(int n) { return (int)blockIdx.x * n; }
-__device__ __forceinline__ int next_item_n(unsigned *head, int *slot, int n, int count) {
-  if ((int)gridDim.x * n >= count) return count;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned S = min((unsigned)kQueueSpread, gridDim.x), x = blockIdx.x % S;
-    *slot = (int)((gridDim.x + S * atomicAdd(head + x * kQueueStride, 1u) + x) * (unsigned)n);
-  }
-  __syncthreads();
-  return *slot;
-}
 
 // ------------------------------------------------------------------ cells
 __device__ __forceinline__ void cell_coords(const GridParams &g, float x, float y, float z, int &cx, int &cy,

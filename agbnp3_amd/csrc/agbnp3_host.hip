@@ -775,6 +775,7 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   for (double **q : {&d.volumep_raw, &d.sa_raw, &d.sa_f, &d.sp, &d.spe, &d.psvol, &d.gammap, &d.beta, &d.br,
                      &d.brw, &d.swf, &d.A, &d.q2ab, &d.abrw, &d.deru, &d.derv, &d.derus, &d.dervs, &d.derh})
     take(*q, n);
+  d.tree_cnt = reinterpret_cast<uint2 *>(d.A);
   for (float **q : {&d.sp_f, &d.spe_f, &d.br_f, &d.q2ab_f, &d.abrw_f, &d.deru_f, &d.derv_f, &d.derus_f,
                     &d.dervs_f, &d.derh_f, &d.gammap_f})
     take(*q, n);

@@ -25,27 +25,38 @@ __device__ void block_partials(const Dev &d, const int *slots, const double *v, 
   }
 }
 
-// near-pair total and longest row (counters 2, 3): one add and one max per
-// block rather than per row (same-address atomics serialise in L2).  The
-// grid has at least one block per 256 heavy rows.
-__device__ __forceinline__ void nbl_counts(const Dev &d) {
-  __shared__ unsigned ssum[kEpi / 64], smax[kEpi / 64];
+// near-pair total and longest row (counters 2, 3) and the first tree tier's
+// counts: one add or max per block rather than per row (same-address atomics
+// serialise in L2).  The grid has at least one block per 256 heavy rows.
+__device__ __forceinline__ void row_counts(const Dev &d) {
+  __shared__ unsigned red[4][kEpi / 64];
   const int h = blockIdx.x * kEpi + threadIdx.x;
   if (blockIdx.x * kEpi >= d.nh) return;             // block-uniform
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  unsigned sum = h < d.nh ? (unsigned)d.nne[h] : 0u, mx = sum;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sum += __shfl_xor((int)sum, o, 64);
-    mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
+  unsigned v[4] = {0u, 0u, 0u, 0u};                  // pairs, longest row, overlaps kept, evaluated
+  if (h < d.nh) {
+    const uint2 c = d.tree_cnt[h];
+    v[0] = v[1] = (unsigned)d.nne[h];
+    v[2] = c.x;
+    v[3] = c.y;
   }
-  if (lane == 0) { ssum[w] = sum; smax[w] = mx; }
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const unsigned t = (unsigned)__shfl_xor((int)v[k], o, 64);
+      v[k] = k == 1 ? max(v[k], t) : v[k] + t;
+    }
+    if (lane == 0) red[k][w] = v[k];
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned t = 0, m = 0;
-    for (int q = 0; q < kEpi / 64; q++) { t += ssum[q]; m = max(m, smax[q]); }
-    if (t) atomicAdd(&d.counters[2], (unsigned long long)t);
-    if (m) atomicMax(&d.counters[3], (unsigned long long)m);
+  if (threadIdx.x < 4) {
+    const int k = threadIdx.x;
+    unsigned long long t = 0;
+    for (int q = 0; q < kEpi / 64; q++) t = k == 1 ? max(t, (unsigned long long)red[k][q]) : t + red[k][q];
+    unsigned long long *c = d.counters + kCountBase + 8 * (blockIdx.x % kCountSlots);
+    if (k == 1) atomicMax(&d.counters[3], t);
+    else if (t) atomicAdd(k == 0 ? &d.counters[2] : c + (k - 2), t);
   }
 }
 
@@ -54,7 +65,7 @@ __device__ __forceinline__ void nbl_counts(const Dev &d) {
 // (agbnp3.c:1104-1117); E_cav, E_corr_cav, molecular volume
 // (agbnp3.c:1390-1411)
 __global__ __launch_bounds__(kEpi) void k_scale(Dev d) {
-  nbl_counts(d);
+  row_counts(d);
   const int2 blk = d.ablk[blockIdx.x];
   const int i = blk.x + threadIdx.x;
   double ecav = 0.0, ecorr = 0.0, mv = 0.0;

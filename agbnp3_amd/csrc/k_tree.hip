@@ -604,7 +604,10 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
       const bool first = !PB && list == 0;
       const unsigned k = atomicAdd(&d.counters[first ? 4 : 6 + (PB ? 1 : 0)], 1ull);
       if (first || PB) d.tree_ovf[(PB ? (size_t)d.nh : 0) + k] = h;
-      if (first) d.tree_tier[h] = 1;
+      if (first) {
+        d.tree_tier[h] = 1;
+        d.tree_cnt[h] = make_uint2(0, 0);
+      }
     }
     __syncthreads();
   };
@@ -701,7 +704,14 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
     rsum[v] = wave_sum((double)root[v]);
     if (W > 1 && lane == 0) slot_add(&S.acc[v][0], rsum[v]);
   }
+  if (W > 1 && lane == 0) S.wcnt[0][tid >> 6] = (int)neval;
   if (W > 1) __syncthreads();
+  if (!PB && list == 0 && tid == 0) {     // pass A's first tier: its counts, which k_scale adds up
+    unsigned ev = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) ev += (unsigned)S.wcnt[0][w];
+    d.tree_cnt[h] = make_uint2(nkept, ev);
+  }
   if (W == 1 && tid == 0) {
     const int at = S.idx[0];
     if (!PB) {
@@ -729,7 +739,8 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
 }
 
 // overlaps kept (block totals) and evaluated (per wave) by one persistent
-// block (pass A only)
+// block of pass A's second tier (the first stores them per root: three atomics
+// of each block at exit cost it 1 % of a call)
 __device__ __forceinline__ void add_tree_counts(const Dev &d, bool pass_b, unsigned long long tk,
                                                 unsigned long long te) {
   if (pass_b || (threadIdx.x & 63) != 0) return;
@@ -739,8 +750,11 @@ __device__ __forceinline__ void add_tree_counts(const Dev &d, bool pass_b, unsig
 }
 
 
-// persistent: each block takes roots from a queue until none are left;
-// overflowing roots go to the second tier's list.  Two waves per root share
+// A block per root (or, tuned, a persistent grid that takes roots from a
+// queue): the dispatcher hands them out with less delay than a queue head, and
+// evenly where the trees are not (11,000 atoms, call 445 -> 424 us, 90 ragged
+// systems 1454 -> 1403, against 4,096 blocks that took two roots at a time).
+// Overflowing roots go to the second tier's list.  Two waves per root share
 // every order's candidates (slot sums in fixed point): at one wave per root
 // the LDS of a root (13-27 KB) left a SIMD one or two waves to hide the
 // walk's LDS and memory latency.
@@ -756,20 +770,13 @@ __global__ __launch_bounds__(64 * kFirstWaves, PB ? 4 : 7) void k_tree_bfs(Dev d
   __shared__ BfsLds<CAP, PB, kLevelCap, kFirstWaves> S;
   __shared__ int slot;
   unsigned *head = queue_head(d.queue, PB ? Q_TREE_B : Q_TREE_A);
-  // roots in runs of `run` per queue grab (one returning atomic on the queue
-  // head per grab; at least two: the grabs serialise on that one address),
-  // one by one where the grid has a block for each: half the blocks would
-  // otherwise walk two in a row beside an idle half
-  const int run = (int)gridDim.x >= d.nh ? 1 : max(2, min(8, d.nh / (int)(gridDim.x * 8)));
   // queue position k takes root (k * P) mod nh, P a prime that does not
   // divide nh: roots in flight together lie far apart in the atom order, so
   // their fixed-point scatters rarely meet on one atom
   const long long P = d.nh % 7919 ? 7919 : (d.nh % 7927 ? 7927 : 7933);
   unsigned long long tk = 0, te = 0;
-  for (int k0 = first_item_n(run); k0 < d.nh; k0 = next_item_n(head, &slot, run, d.nh))
-    for (int k = k0; k < min(k0 + run, d.nh); k++)
-      tree_bfs_root<CAP, PB, kLevelCap, kFirstWaves>(d, S, (int)(((long long)k * P) % d.nh), 0, tk, te);
-  add_tree_counts(d, PB, tk, te);
+  for (int k = first_item(); k < d.nh; k = next_item(head, &slot, d.nh))
+    tree_bfs_root<CAP, PB, kLevelCap, kFirstWaves>(d, S, (int)(((long long)k * P) % d.nh), 0, tk, te);
 }
 
 // second tier: the roots pass A's first tier queued (in both passes), with
@@ -835,7 +842,7 @@ hipError_t prepare_tree() {
 // for the second tier
 template <int CAP>
 static void launch_tree_cap(const Dev &d, const Tuning &t, int pass, int tier, hipStream_t s) {
-  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : 256 * 16), gf = std::min(d.nh, 64);
+  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : d.nh), gf = std::min(d.nh, 64);
   const int gb = std::min(d.nh, 512);
   const size_t la = big_lds<CAP, false>(), lb = big_lds<CAP, true>();
   if (pass == 0) {
