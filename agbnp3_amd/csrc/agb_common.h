@@ -30,6 +30,12 @@ constexpr float kHbSwA = 0.65f, kHbSwB = 1.0f, kHbSwA0 = 0.6f;
 // from which the second tier of the derivative pass has that stream
 constexpr int kForkAtoms = 16384;
 constexpr int kSideAtoms = 512;
+// heavy atoms from which the derivative pass's second tier is launched first:
+// its blocks, two to a CU, otherwise find no room before the first tier ends
+// (40,000 atoms, 19,000 of them heavy, call 1994 -> 1966 us, 12 x 6000 1245 ->
+// 1224; 25,000 no change, 11,000 429 -> 437; in a replayed graph of 64 or 90
+// systems 1 % slower)
+constexpr int kBigFirst = 16384;
 // columns of a descreening group with a box of its own
 constexpr int kBoxCols = 16;
 // extents of a solute, in units of the longest table's reach (46 A for heavy

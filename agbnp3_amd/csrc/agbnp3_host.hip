@@ -1067,9 +1067,10 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   if (fork2) {
     HIPCHK(hipEventRecord(P.ev_fork2, s));
     HIPCHK(hipStreamWaitEvent(P.side, P.ev_fork2, 0));
-    launch_tree_tier(d, t, 1, 1, P.side);
+    const int there = d.nh > kBigFirst && !capturing ? 0 : 1;    // the tier on the second stream
+    launch_tree_tier(d, t, 1, there, P.side);
     HIPCHK(hipEventRecord(P.ev_join2, P.side));
-    launch_tree_tier(d, t, 1, 0, s);
+    launch_tree_tier(d, t, 1, 1 - there, s);
     HIPCHK(hipStreamWaitEvent(s, P.ev_join2, 0));
   } else {
     launch_tree(d, t, 1, s);
