@@ -267,6 +267,7 @@ __device__ void ws_place_site(const Dev &d, const WsDef &def, int which, WSite &
 // site with more than 1024 candidates fails the call.
 constexpr int kWsWaves = 4;
 constexpr int kWsCap = 128, kWsCapBig = 1024;
+constexpr int kWsAhead = 4;
 
 template <int WAVES, int CAP>
 struct WsLds {
@@ -317,28 +318,34 @@ __device__ bool ws_free_site(const Dev &d, WsLds<WAVES, CAP> &L, int site, int w
   if (active) {
     int cx, cy, cz;
     cell_coords(g, wpos[0], wpos[1], wpos[2], cx, cy, cz);
-    // the stencil's candidates 64 at a time; sorted by atom index below
+    // the stencil's candidates, kWsAhead steps of 64 in flight; sorted by atom
+    // index below
     int start[9], off[9];
     const int total = stencil_segments(g, cstart, cx, cy, cz, start, off);
-    for (int base = 0; base < total; base += 64) {
-      const int k = base + lane;
-      bool pass = false;
-      int j = -1;
-      if (k < total) {
-        j = d.cell_atoms[stencil_slot(start, off, k)];
-        const float4 pj = d.pos[j];
-        const float ex = __fsub_rn(pj.x, wpos[0]), ey = __fsub_rn(pj.y, wpos[1]),
-                    ez = __fsub_rn(pj.z, wpos[2]);
-        const float d2 = __fadd_rn(__fadd_rn(__fmul_rn(ex, ex), __fmul_rn(ey, ey)), __fmul_rn(ez, ez));
-        const float u = __fmul_rn(__fadd_rn(pj.w, kHbRadius), kNbOffset);
-        pass = d2 < __fmul_rn(u, u);
+    for (int base = 0; base < total; base += 64 * kWsAhead) {
+      int j[kWsAhead];
+      float4 pj[kWsAhead];
+#pragma unroll
+      for (int u = 0; u < kWsAhead; u++) j[u] = d.cell_atoms[stencil_slot(start, off, min(base + 64 * u + lane, total - 1))];
+#pragma unroll
+      for (int u = 0; u < kWsAhead; u++) pj[u] = d.pos[j[u]];
+#pragma unroll
+      for (int u = 0; u < kWsAhead; u++) {
+        if (base + 64 * u >= total) break;             // wave-uniform
+        bool pass = false;
+        if (base + 64 * u + lane < total) {
+          const float ex = __fsub_rn(pj[u].x, wpos[0]), ey = __fsub_rn(pj[u].y, wpos[1]), ez = __fsub_rn(pj[u].z, wpos[2]);
+          const float d2 = __fadd_rn(__fadd_rn(__fmul_rn(ex, ex), __fmul_rn(ey, ey)), __fmul_rn(ez, ez));
+          const float t = __fmul_rn(__fadd_rn(pj[u].w, kHbRadius), kNbOffset);
+          pass = d2 < __fmul_rn(t, t);
+        }
+        const unsigned long long m = __ballot(pass);
+        if (pass) {
+          const int slot = cnt + __popcll(m & ((1ull << lane) - 1ull));
+          if (slot < CAP) L.cj[w][slot] = j[u];
+        }
+        cnt += __popcll(m);
       }
-      const unsigned long long m = __ballot(pass);
-      if (pass) {
-        const int slot = cnt + __popcll(m & ((1ull << lane) - 1ull));
-        if (slot < CAP) L.cj[w][slot] = j;
-      }
-      cnt += __popcll(m);
     }
   }
   // a site past these buffers adds nothing here
