@@ -59,6 +59,10 @@ constexpr size_t kChainByTime = 8192;
 // atoms, 155 items, 302 -> 268 us; with up to 512, 6,000 atoms 315 -> 327), and
 // most of its blocks for which a front takes four pairs at a time
 constexpr int kSplitItems = 256, kSplitSets = 6, kSplitFour = 256;
+// most items of the GB pairs by chunks (k_gb_split; a call of 2,000 atoms, 36
+// items, 215 -> 208 us, of 2,700, 66 items, 233 -> 234, of 4,000, 136 items, 259 -> 271),
+// and sets of 4 x 256 numbers that an item's sums take there
+constexpr int kGbSplitItems = 48, kGbSets = 5;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;
@@ -292,6 +296,9 @@ struct Dev {
   float4 *chbox;
   double *beta, *br, *brw, *swf;       // [n]
   float *br_f;
+  int gbs_on;                          // GB pairs by chunks:
+  float *gbsplit;                      // per GB energy slot its row sums by chunk and its column sums
+  double *gbener;                      // and its energy by chunk
   double *gb_epart;                    // per GB energy slot: sum of q_i q_j / f
   double *A, *q2ab, *abrw;             // [n]
   float *q2ab_f, *abrw_f;

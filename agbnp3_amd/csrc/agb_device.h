@@ -340,6 +340,24 @@ __device__ __forceinline__ void fix_add(long long *p, double v) {
 }
 __device__ __forceinline__ double fix_get(long long v) { return (double)v * kFixInv; }
 
+// ----------------------------------------------------- chain-rule factors
+// q2ab = (q^2 + A B) swf', abrw = alpha brw swf' (kernels.c:433-450).  The
+// FP32 copies are the chain rule's weights: on a surrogate call with
+// out-of-range atoms (mode 2) only those atoms' radii come from the
+// descreening, so every other atom's chain-rule weight is zero (the
+// surrogate's gradient pass weighs them from the FP64 values)
+__device__ __forceinline__ void chain_factors(const Dev &d, int i, double A) {
+  const double q = d.q[i];
+  const double q2ab = (q * q + A * d.br[i]) * d.swf[i];
+  const double abrw = ((double)d.ialpha[i] + (double)d.salpha[i]) * d.brw[i] * d.swf[i];
+  d.A[i] = A;
+  d.q2ab[i] = q2ab;
+  d.abrw[i] = abrw;
+  const bool chain = !d.sg_on || d.sg_state[4 * d.asys[i] + 2] != 2 || d.sg_oor[i];
+  d.q2ab_f[i] = chain ? (float)q2ab : 0.f;
+  d.abrw_f[i] = chain ? (float)abrw : 0.f;
+}
+
 // ------------------------------------------------- U, V coefficients
 // deru = U/V_i, derus = df/(4pi) psvol deru, dervs = psvol derv/(4pi)
 // (kernels.c:861-875), from the chain rule's sums (which = 0: U, and H_i of

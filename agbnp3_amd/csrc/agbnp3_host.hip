@@ -784,6 +784,9 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   take(d.cbox, 2 * (size_t)std::max(nablk, 1) * (256 / kBoxCols));
   take(d.chbox, 8 * (size_t)std::max(d.ncblk, 1));
   take(d.gb_epart, (size_t)std::max(ntile, 1));
+  const size_t ngbs = ntile <= kGbSplitItems ? ntile : 0;
+  take(d.gbsplit, ngbs * kGbSets * 1024);
+  take(d.gbener, ngbs * 4);
   take(d.ws_part, nws);
   take(d.ws_ovf, nws);
   take(d.epart, (size_t)EP_COUNT * std::max(nablk, 1));
@@ -993,6 +996,7 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   d.reuse_every = P.reuse_every;
   d.dt_on = P.dt && !d.sg_on;
   d.split_on = P.split && !d.sg_on;
+  d.gbs_on = d.ngb_items <= kGbSplitItems && P.tune.gb_grid == 0 && d.nchain_items <= kChainGroupItems && !d.sg_on;
   hipStream_t s = P.stream;
   const bool timed = !capturing && (P.options & AGBNP3_OPT_TIMING) != 0;
   int k = 0;

@@ -205,11 +205,7 @@ void launch_born(const Dev &d, hipStream_t s) {
 }
 
 // -------------------------------------------------- chain-rule factors
-// q2ab = (q^2 + A B) swf', abrw = alpha brw swf' (kernels.c:433-450).  The
-// FP32 copies are the chain rule's weights: on a surrogate call with
-// out-of-range atoms (mode 2) only those atoms' radii come from the
-// descreening, so every other atom's chain-rule weight is zero (the
-// surrogate's gradient pass weighs them from the FP64 values)
+// (chain_factors), after the GB pairs
 __global__ __launch_bounds__(kEpi) void k_q2ab(Dev d) {
   const int nblk = (d.n + kEpi - 1) / kEpi;
   if ((int)blockIdx.x >= nblk) {        // further blocks: the boxes of the chain rule's chunks
@@ -225,19 +221,11 @@ __global__ __launch_bounds__(kEpi) void k_q2ab(Dev d) {
     return;
   }
   const int i = blockIdx.x * kEpi + threadIdx.x;
-  if (i < d.n) {
-    const double A = fix_get(d.acc_gbA[i]);
-    const double q = d.q[i];
-    d.A[i] = A;
-    d.q2ab[i] = (q * q + A * d.br[i]) * d.swf[i];
-    d.abrw[i] = ((double)d.ialpha[i] + (double)d.salpha[i]) * d.brw[i] * d.swf[i];
-    const bool chain = !d.sg_on || d.sg_state[4 * d.asys[i] + 2] != 2 || d.sg_oor[i];
-    d.q2ab_f[i] = chain ? (float)d.q2ab[i] : 0.f;
-    d.abrw_f[i] = chain ? (float)d.abrw[i] : 0.f;
-  }
+  if (i < d.n) chain_factors(d, i, fix_get(d.acc_gbA[i]));
 }
 
 void launch_q2ab(const Dev &d, hipStream_t s) {
+  if (d.gbs_on) return;                 // (k_gb_sum's; no boxes at its sizes)
   const int boxes = d.cull_chain && d.nchain_items > kChainGroupItems ? d.ncblk : 0;
   hipLaunchKernelGGL(k_q2ab, dim3((d.n + kEpi - 1) / kEpi + boxes), dim3(kEpi), 0, s, d);
 }

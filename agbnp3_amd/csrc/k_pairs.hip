@@ -205,29 +205,38 @@ __device__ __forceinline__ float lds_rot(float v, int from) {
 struct GbRow {
   float x, y, z, q, b, qib;     // position, charge, Born radius, -log2(e) / (4 B)
 };
-// MASK: the reference's mask (kernels.c:107), d2 > 0, which also drops the
-// self pair; without it the smallest d2 is kept instead
+// its terms: q_i q_j and 1/f, x_j - x_i, the gradient's, and A's two factors.  MASK: the
+// reference's mask (kernels.c:107), d2 > 0, which also drops the self pair;
+// without it the smallest d2 is kept instead
+struct GbTerm {
+  float qq, fgb, ex, ey, ez, mw, h, bd;
+};
+template <bool MASK>
+__device__ __forceinline__ void gb_term(const GbRow &r, const float4 &cp, const float2 &cb, float &d2min, GbTerm &g) {
+  g.ex = cp.x - r.x; g.ey = cp.y - r.y; g.ez = cp.z - r.z;
+  const float d2 = g.ex * g.ex + g.ey * g.ey + g.ez * g.ez;
+  g.qq = r.q * cp.w;
+  if (MASK) g.qq = d2 > 0.f ? g.qq : 0.f;
+  else d2min = fminf(d2min, d2);
+  const float bb = r.b * cb.x;
+  const float et = __builtin_amdgcn_exp2f(d2 * (r.qib * cb.y));     // exp(-d2 / (4 B_i B_j))
+  g.fgb = __builtin_amdgcn_rsqf(d2 + bb * et);
+  const float qf3 = g.qq * g.fgb * g.fgb * g.fgb;
+  g.h = qf3 * et;
+  g.mw = fmaf(-0.25f, g.h, qf3);               // qf3 (1 - et/4)
+  g.bd = fmaf(0.25f, d2, bb);                  // (A's term: qf3 et (bb + d2/4))
+}
 template <bool MASK>
 __device__ __forceinline__ void gb_pair(const GbRow &r, const float4 &cp, const float2 &cb, float &d2min, float &re,
                                         float &rA, float &rx, float &ry, float &rz, float &cA, float &cgx, float &cgy,
                                         float &cgz) {
-  const float ex = cp.x - r.x, ey = cp.y - r.y, ez = cp.z - r.z;
-  const float d2 = ex * ex + ey * ey + ez * ez;
-  float qq = r.q * cp.w;
-  if (MASK) qq = d2 > 0.f ? qq : 0.f;
-  else d2min = fminf(d2min, d2);
-  const float bb = r.b * cb.x;
-  const float et = __builtin_amdgcn_exp2f(d2 * (r.qib * cb.y));     // exp(-d2 / (4 B_i B_j))
-  const float fgb = __builtin_amdgcn_rsqf(d2 + bb * et);
-  const float qf3 = qq * fgb * fgb * fgb;
-  re += qq * fgb;
-  const float g = qf3 * et;
-  const float mw = fmaf(-0.25f, g, qf3);                 // qf3 (1 - et/4)
-  const float at = g * fmaf(0.25f, d2, bb);              // qf3 et (bb + d2/4)
-  rx += mw * ex; ry += mw * ey; rz += mw * ez;
-  rA += at;
-  cA += at;
-  cgx = fmaf(mw, ex, cgx); cgy = fmaf(mw, ey, cgy); cgz = fmaf(mw, ez, cgz);     // (negated)
+  GbTerm g;
+  gb_term<MASK>(r, cp, cb, d2min, g);
+  re += g.qq * g.fgb;
+  rx += g.mw * g.ex; ry += g.mw * g.ey; rz += g.mw * g.ez;
+  rA = fmaf(g.h, g.bd, rA);
+  cA = fmaf(g.h, g.bd, cA);
+  cgx = fmaf(g.mw, g.ex, cgx); cgy = fmaf(g.mw, g.ey, cgy); cgz = fmaf(g.mw, g.ez, cgz);     // (negated)
 }
 
 __global__ __launch_bounds__(256, 4) void k_gbpair(Dev d) {
@@ -340,8 +349,185 @@ __global__ __launch_bounds__(256, 4) void k_gbpair(Dev d) {
   }
 }
 
+// ------------------------------------------- GB pairs of small calls
+// The same sums (k_gbpair) where its items are fewer than the CUs and one
+// wave's 64 steps of four rows are the launch.  A block takes one item's
+// 64-column chunk, and six waves share the work of k_gbpair's one: four form
+// the pairs' terms, each for 64 of the tile's rows with their sums, and pass
+// them through LDS, batch by batch, to one that adds the column sums (its lanes
+// are columns, so nothing rotates) and one that adds the energy, in the order
+// k_gbpair's lanes do.  The sums leave apart; k_gb_sum adds them in k_gbpair's
+// order, per atom, and does k_q2ab's work with them.
+// Bound: the column wave's LDS reads, one batch of them per barrier.  Against
+// k_gbpair (with k_q2ab): 61 atoms 21 + 4.2 -> 8.1 + 3.1 us, 613 22 + 4.3 ->
+// 12.7 + 5.1, 2,000 22 + 4.7 -> 13.0 + 5.0.
+constexpr int kGbSteps = 4;              // steps of a batch
+constexpr int kGbWaves = 6;
+__global__ __launch_bounds__(64 * kGbWaves) void k_gb_split(Dev d) {
+  // columns and rows twice in a row (k_gbpair): x, y, z, charge; Born radius, its reciprocal
+  __shared__ float4 cxq[128], rx4[4][128];
+  __shared__ float2 cbr[128];
+  __shared__ float4 grad[2][kGbSteps][4][64];              // the terms: gradient, A's factors
+  __shared__ float2 ener[2][kGbSteps][4][64];              // charges, 1/f
+  const int lane = threadIdx.x & 63, role = threadIdx.x >> 6;
+  const int it = blockIdx.x >> 2, w = blockIdx.x & 3;
+  const int4 tp = d.gb_items[it];        // rows [x, y), columns [z, w)
+  if (w * 64 >= tp.w - tp.z) return;     // no such chunk (block-uniform)
+  const bool diag = tp.x == tp.z;
+  const int nrow = (tp.y - tp.x + 63) >> 6;                // row groups with an atom
+  if (role == 4) {
+    const int j = tp.z + 64 * w + lane;
+    float4 c = make_float4(-1e6f - (float)(64 * w + lane), 0.f, 0.f, 0.f);
+    float2 b = make_float2(1.f, 1.f);
+    if (j < tp.w) {
+      const float4 p = d.pos[j];
+      const float bj = d.br_f[j];
+      c = make_float4(p.x, p.y, p.z, d.q[j]);
+      b = make_float2(bj, __builtin_amdgcn_rcpf(bj));
+    }
+    cxq[lane] = c;
+    cxq[lane + 64] = c;
+    cbr[lane] = b;
+    cbr[lane + 64] = b;
+  }
+  GbRow row{1e6f + (float)(64 * role + lane), 0.f, 0.f, 0.f, 1.f, 0.f};
+  if (role < 4) {
+    const int i = tp.x + 64 * role + lane;
+    if (i < tp.y) {
+      const float4 p = d.pos[i];
+      row.x = p.x; row.y = p.y; row.z = p.z;
+      row.q = d.q[i];
+      row.b = d.br_f[i];
+    }
+    row.qib = -0.25f * 1.44269504088896341f * __builtin_amdgcn_rcpf(row.b);
+    rx4[role][lane] = rx4[role][lane + 64] = make_float4(row.x, row.y, row.z, 0.f);
+  }
+  __syncthreads();
+  float rA = 0.f, rx = 0.f, ry = 0.f, rz = 0.f;            // a row's sums (the first four waves)
+  float cA = 0.f, cgx = 0.f, cgy = 0.f, cgz = 0.f, re = 0.f;   // a column's (the fifth), the energy (the sixth)
+  float d2min = 1.f;
+  auto sweep = [&](auto rows) {
+    constexpr int NROW = decltype(rows)::value;
+#pragma unroll 1
+    for (int t = 0; t <= 64 / kGbSteps; t++) {
+      if (role < NROW) {
+        if (t < 64 / kGbSteps) {
+#pragma unroll
+          for (int u = 0; u < kGbSteps; u++) {
+            const int s = t * kGbSteps + u;
+            GbTerm g;
+            gb_term<true>(row, cxq[lane + 64 - s], cbr[lane + 64 - s], d2min, g);
+            rx += g.mw * g.ex; ry += g.mw * g.ey; rz += g.mw * g.ez;
+            rA = fmaf(g.h, g.bd, rA);
+            grad[t & 1][u][role][lane] = make_float4(g.mw, g.h, g.bd, 0.f);
+            ener[t & 1][u][role][lane] = make_float2(g.qq, g.fgb);
+          }
+        }
+      } else if (t > 0 && role >= 4) {
+        const int b = (t - 1) & 1, s0 = (t - 1) * kGbSteps;
+        if (role == 5) {
+          float2 e[kGbSteps][NROW];
+#pragma unroll
+          for (int u = 0; u < kGbSteps; u++)
+#pragma unroll
+            for (int k = 0; k < NROW; k++) e[u][k] = ener[b][u][k][lane];
+#pragma unroll
+          for (int u = 0; u < kGbSteps; u++)
+#pragma unroll
+            for (int k = 0; k < NROW; k++) re += e[u][k].x * e[u][k].y;
+        } else if (!diag) {
+          const float4 c = cxq[lane];
+#pragma unroll
+          for (int u = 0; u < kGbSteps; u++) {
+            float4 g[NROW], r[NROW];
+#pragma unroll
+            for (int k = 0; k < NROW; k++) {
+              g[k] = grad[b][u][k][(lane + s0 + u) & 63];
+              r[k] = rx4[k][lane + s0 + u];
+            }
+#pragma unroll
+            for (int k = 0; k < NROW; k++) {
+              const float ex = c.x - r[k].x, ey = c.y - r[k].y, ez = c.z - r[k].z;
+              cA = fmaf(g[k].y, g[k].z, cA);
+              cgx = fmaf(g[k].x, ex, cgx); cgy = fmaf(g[k].x, ey, cgy); cgz = fmaf(g[k].x, ez, cgz);
+            }
+          }
+        }
+      }
+      __syncthreads();
+    }
+  };
+  // (row groups without an atom add nothing)
+  if (nrow == 4) sweep(std::integral_constant<int, 4>{});
+  else if (nrow == 3) sweep(std::integral_constant<int, 3>{});
+  else if (nrow == 2) sweep(std::integral_constant<int, 2>{});
+  else sweep(std::integral_constant<int, 1>{});
+  // sets of 4 quantities x 256 atoms of the item's slot: 0..3 its rows by chunk, 4 its columns
+  float *o = d.gbsplit + (size_t)d.gb_eslot[it] * kGbSets * 1024;
+  if (role < 4) {
+    float *p = o + w * 1024 + 64 * role + lane;
+    p[0] = rA; p[256] = rx; p[512] = ry; p[768] = rz;
+  } else if (role == 4) {
+    float *p = o + 4 * 1024 + 64 * w + lane;
+    p[0] = cA; p[256] = cgx; p[512] = cgy; p[768] = cgz;
+  } else {
+    const double e = wave_sum((double)re * (diag ? 0.5 : 1.0));
+    if (lane == 0) d.gbener[4 * (size_t)d.gb_eslot[it] + w] = e;
+  }
+}
+
+// one quantity (A, gradient x, y, z) of one tile's atoms from every item that
+// holds the tile; A's threads form the chain-rule factors at once, and the
+// first gradient's the items' energies.  Grid (tiles, 4).
+__global__ __launch_bounds__(256) void k_gb_sum(Dev d) {
+  const int b = blockIdx.x, q = blockIdx.y, t = threadIdx.x;
+  const int2 blk = d.ablk[b];
+  const SysInfo &S = d.sys[d.asys[blk.x]];
+  const int T = b - S.blk0, nb = S.nblk;
+  auto slot = [&](int I, int J) { return S.tile0 + I * nb - I * (I - 1) / 2 + J - I; };
+  const int i = blk.x + t;
+  if (q == 1)
+    for (int J = T + t; J < nb; J += 256) {
+      const int nch = (min(256, S.n - 256 * J) + 63) >> 6;
+      const double *e = d.gbener + 4 * (size_t)slot(T, J);
+      double v = e[0] + (nch > 1 ? e[1] : 0.0);
+      v += nch > 2 ? e[2] : 0.0;
+      v += nch > 3 ? e[3] : 0.0;
+      d.gb_epart[slot(T, J)] = v;
+    }
+  if (i >= blk.y) return;
+  const float *base = d.gbsplit + q * 256 + t;
+  long long sum = 0;
+#pragma unroll 2
+  for (int J = T; J < nb; J++) {          // the tile as rows: by chunks, in FP32
+    const int nch = (min(256, S.n - 256 * J) + 63) >> 6;
+    const float *s = base + (size_t)slot(T, J) * kGbSets * 1024;
+    const float v0 = s[0], v1 = s[1024], v2 = s[2048], v3 = s[3072];
+    float v = v0 + (nch > 1 ? v1 : 0.f);
+    v += nch > 2 ? v2 : 0.f;
+    v += nch > 3 ? v3 : 0.f;
+    sum += __double2ll_rn((double)v * kFix);
+  }
+#pragma unroll 4
+  for (int I = 0; I < T; I++) {
+    const double v = (double)base[(size_t)slot(I, T) * kGbSets * 1024 + 4 * 1024];
+    sum += __double2ll_rn((q == 0 ? v : -v) * kFix);
+  }
+  if (q == 0) {
+    d.acc_gbA[i] = sum;
+    chain_factors(d, i, fix_get(sum));
+  } else {
+    d.acc_gbg[3 * (size_t)i + q - 1] = sum;
+  }
+}
+
 void launch_gbpair(const Dev &d, const Tuning &t, hipStream_t s) {
   if (!d.ngb_items) return;
+  if (d.gbs_on) {
+    hipLaunchKernelGGL(k_gb_split, dim3(4 * d.ngb_items), dim3(64 * kGbWaves), 0, s, d);
+    hipLaunchKernelGGL(k_gb_sum, dim3(d.nablk, 4), dim3(256), 0, s, d);
+    return;
+  }
   const int grid = t.gb_grid > 0 ? std::min(t.gb_grid, d.ngb_items) : d.ngb_items;
   hipLaunchKernelGGL(k_gbpair, dim3(grid), dim3(256), 0, s, d);
 }

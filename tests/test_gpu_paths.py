@@ -1,8 +1,8 @@
 """Calls that a rule on sizes sends another way give the same results.
 
 Bitwise, the two routes of one call against each other: descreening by tiles
-(few work items) against the plain kernel; the chain rule by row groups (few
-work items) against the plain kernel; far columns skipped by boxes against
+(few work items) against the plain kernel; the chain rule by row groups and
+the GB pairs by chunks (few work items) against the plain kernels; far columns skipped by boxes against
 none skipped.  Against the FP64 oracle: two atoms in one place, which
 the GB kernel's off-diagonal tiles meet without the pair mask, water sites
 with more than 64 candidate atoms, and overlap terms past the range of the
@@ -72,6 +72,25 @@ def test_chain_rule_by_row_groups_equals_the_plain_kernel(natoms, mixed, fixed):
         groups = inst.ener()
         inst.set_tuning(chain_chunk=256)
         assert_same(groups, inst.ener(), natoms)
+    finally:
+        inst.delete()
+
+
+@pytest.mark.parametrize("natoms", [8, 61, 64, 130, 257, 513, 700, 2000, 2304])
+def test_gb_pairs_by_chunks_equal_the_plain_kernel(natoms):
+    """A grid asked for is the plain kernel's; two atoms of different tiles in one place as well."""
+    s = synth.generate(20260500 + natoms, natoms)
+    h = s.ihydrogen
+    x, y, z = s.x.copy(), s.y.copy(), s.z.copy()
+    if natoms > 512:
+        i, j = int(h[0]), int(h[-1])
+        x[j], y[j], z[j] = x[i], y[i], z[i]
+    inst = api.Instance(s)
+    try:
+        chunks = inst.ener(), inst.ener(x, y, z)
+        inst.set_tuning(gb_grid=4096)
+        assert_same(chunks[0], inst.ener(), natoms)
+        assert_same(chunks[1], inst.ener(x, y, z), natoms)
     finally:
         inst.delete()
 
