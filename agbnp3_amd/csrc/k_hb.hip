@@ -505,8 +505,24 @@ void launch_ws_free(const Dev &d, hipStream_t s) {
 // table's).  Past kDtItems items the plain kernel's scalar loads are the
 // better form: 25,000 atoms 169 us against 239 here.
 constexpr int kDtCols = 256, kDtUnroll = 4;
+// most blocks, sites' and rows', for that: its LDS leaves a CU to each (1,500 atoms,
+// call 206 -> 198 us; 2,000, 330 blocks, 208 either way; 4,000, 900 blocks, 258 -> 284)
+constexpr int kDtFew = 320;
 constexpr size_t dt_lds(int ntypes) {
   return (size_t)ntypes * kTblN * sizeof(float2) + kDtCols * (sizeof(float4) + sizeof(float2));
+}
+
+// one column's Q4 for a row at pi (q4_value without its branch)
+__device__ __forceinline__ float desc_value(const float2 *tab, const float4 &pj, const float2 &cw, const float4 &pi) {
+  const float ex = pj.x - pi.x, ey = pj.y - pi.y, ez = pj.z - pi.z;
+  const float xh = __builtin_amdgcn_sqrtf(fmaf(ez, ez, fmaf(ex, ex, ey * ey))) * pj.w;
+  const unsigned k = (unsigned)(int)xh;
+  const float2 *n = tab + __float_as_int(cw.y) * kTblN + min(k, (unsigned)(kTblN - 2));
+  const float2 n0 = n[0], n1 = n[1];
+  const float B = __builtin_amdgcn_fractf(xh), A = 1.f - B;
+  const float s = fmaf(B, n1.y, fmaf(A, n0.y, n0.y + n1.y));
+  const float v = fmaf(-(A * B), s, fmaf(A, n0.x, B * n1.x));
+  return k <= (unsigned)(kTblN - 2) ? v : 0.f;
 }
 
 __device__ __forceinline__ void desc_tile(const Dev &d, char *lds, int item) {
@@ -541,18 +557,8 @@ __device__ __forceinline__ void desc_tile(const Dev &d, char *lds, int item) {
       float q[N], w[N];
 #pragma unroll
       for (int u = 0; u < N; u++) {
-        const float4 pj = col[c + u];
         const float2 cw = cwt[c + u];
-        const float ex = pj.x - pi.x, ey = pj.y - pi.y, ez = pj.z - pi.z;
-        const float xh = __builtin_amdgcn_sqrtf(fmaf(ez, ez, fmaf(ex, ex, ey * ey))) * pj.w;
-        // q4_value without its branch
-        const unsigned k = (unsigned)(int)xh;
-        const float2 *n = tab + __float_as_int(cw.y) * kTblN + min(k, (unsigned)(kTblN - 2));
-        const float2 n0 = n[0], n1 = n[1];
-        const float B = __builtin_amdgcn_fractf(xh), A = 1.f - B;
-        const float s = fmaf(B, n1.y, fmaf(A, n0.y, n0.y + n1.y));
-        const float v = fmaf(-(A * B), s, fmaf(A, n0.x, B * n1.x));
-        q[u] = k <= (unsigned)(kTblN - 2) ? v : 0.f;
+        q[u] = desc_value(tab, col[c + u], cw, pi);
         w[u] = decltype(self)::value && it.y + c + u == i ? 0.f : cw.x;
       }
 #pragma unroll
@@ -569,10 +575,63 @@ __device__ __forceinline__ void desc_tile(const Dev &d, char *lds, int item) {
   if (i >= 0) d.dpart[it.w + i] = acc;
 }
 
+// The same for calls of so few items that a wave's 256 columns are the launch:
+// a block takes 64 of an item's rows, its four waves look up 64 columns each and
+// leave the values in LDS, and one adds them up in column order.
+// Bound: the sites beside it (12 us).  k_desc_sites at 613 atoms 22.1 -> 14.4 us.
+__device__ __forceinline__ void desc_tile_few(const Dev &d, char *lds, int sub) {
+  float2 *tab = reinterpret_cast<float2 *>(lds);
+  float4 *col = reinterpret_cast<float4 *>(tab + d.ntypes * kTblN);
+  float2 *cwt = reinterpret_cast<float2 *>(col + kDtCols);
+  float4 *val = reinterpret_cast<float4 *>(cwt + kDtCols);       // [four columns][lane]
+  const int groups = d.rows / 64, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int4 it = d.dt_items[sub / groups];
+  const int nc = it.z - it.y;
+  const int i = d.row_perm[it.x * d.rows + (sub % groups) * 64 + lane];
+  if (__ballot(i >= 0) == 0ull) return;             // padding rows (the same in every wave)
+  const float dp2 = d.tdx * (d.tdx / 6.0f);
+  const float2 *src = d.tbl + (size_t)d.rblk[it.x].x * d.ntypes * kTblN;
+  float4 pi = make_float4(0.f, 0.f, 0.f, 0.f), pc = pi;
+  float2 wc = make_float2(0.f, 0.f);                // (columns past the range: no weight, tables of type 0)
+  if ((int)threadIdx.x < nc) {
+    pc = d.dcol[it.y + threadIdx.x];
+    wc = d.dcw[it.y + threadIdx.x];
+  }
+  if (i >= 0) pi = d.pos[i];
+#pragma unroll 10
+  for (int k = threadIdx.x; k < d.ntypes * kTblN; k += 256) {
+    const float2 v = src[k];
+    tab[k] = make_float2(v.x, v.y * dp2);
+  }
+  col[threadIdx.x] = pc;
+  cwt[threadIdx.x] = wc;
+  __syncthreads();
+#pragma unroll 2
+  for (int c = 64 * w; c < min(64 * w + 64, nc); c += 4) {
+    float q[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) q[u] = desc_value(tab, col[c + u], cwt[c + u], pi);
+    val[c / 4 * 64 + lane] = make_float4(q[0], q[1], q[2], q[3]);
+  }
+  __syncthreads();
+  if (w != 0) return;                               // (no barrier follows)
+  float acc = 0.f;
+#pragma unroll 4
+  for (int c = 0; c < nc; c += 4) {
+    const float4 v = val[c / 4 * 64 + lane];
+    const float q[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int u = 0; u < 4; u++) acc = fmaf(q[u], it.y + c + u == i ? 0.f : cwt[c + u].x, acc);
+  }
+  if (i >= 0) d.dpart[it.w + i] = acc;
+}
+
+template <bool FEW>
 __global__ __launch_bounds__(256) void k_desc_sites(Dev d, int nsite_blocks) {
   extern __shared__ __align__(16) char lds[];
   if ((int)blockIdx.x >= nsite_blocks) {
-    desc_tile(d, lds, (int)blockIdx.x - nsite_blocks);
+    if constexpr (FEW) desc_tile_few(d, lds, (int)blockIdx.x - nsite_blocks);
+    else desc_tile(d, lds, (int)blockIdx.x - nsite_blocks);
     return;
   }
   // four sites, then those with more candidates than 128 one by one
@@ -590,25 +649,32 @@ __global__ __launch_bounds__(256) void k_desc_sites(Dev d, int nsite_blocks) {
   }
 }
 
-static size_t desc_sites_lds(const Dev &d) {
-  return std::max(dt_lds(d.ntypes), std::max(sizeof(WsLds<kWsWaves, kWsCap>), sizeof(WsLds<1, kWsCapBig>)));
+static size_t desc_sites_lds(int ntypes, bool few) {
+  const size_t tile = dt_lds(ntypes) + (few ? (size_t)kDtCols * 64 * sizeof(float) : 0);
+  return std::max(tile, std::max(sizeof(WsLds<kWsWaves, kWsCap>), sizeof(WsLds<1, kWsCapBig>)));
 }
 
 hipError_t prepare_sites(int ntypes) {
   static int limit = 0;                             // raised to the largest any pack has needed
-  Dev d{};
-  d.ntypes = std::min(ntypes, kLdsTypes);
-  const int need = (int)desc_sites_lds(d);
-  if (need <= limit) return hipSuccess;
-  const hipError_t e = hipFuncSetAttribute((const void *)k_desc_sites, hipFuncAttributeMaxDynamicSharedMemorySize, need);
-  if (e == hipSuccess) limit = need;
+  const int t = std::min(ntypes, kLdsTypes);
+  if (t <= limit) return hipSuccess;
+  const auto set = [&](const void *f, bool few) {
+    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)desc_sites_lds(t, few));
+  };
+  hipError_t e = set((const void *)k_desc_sites<false>, false);
+  if (e == hipSuccess) e = set((const void *)k_desc_sites<true>, true);
+  if (e == hipSuccess) limit = t;
   return e;
 }
 
 void launch_desc_sites(const Dev &d, hipStream_t s) {
-  const int ns = (d.nws + kWsWaves - 1) / kWsWaves;
-  if (ns + d.ndt_items)
-    hipLaunchKernelGGL(k_desc_sites, dim3(ns + d.ndt_items), dim3(256), desc_sites_lds(d), s, d, ns);
+  const int ns = (d.nws + kWsWaves - 1) / kWsWaves, subs = d.ndt_items * (d.rows / 64);
+  // few: about a block per CU, which is what its LDS allows
+  const bool few = ns + subs <= kDtFew;
+  const int nb = ns + (few ? subs : d.ndt_items);
+  if (nb)
+    hipLaunchKernelGGL(few ? k_desc_sites<true> : k_desc_sites<false>, dim3(nb), dim3(256), desc_sites_lds(d.ntypes, few), s,
+                       d, ns);
 }
 
 }  // namespace agb

@@ -54,6 +54,20 @@ def test_descreening_by_tiles_equals_the_plain_kernel(natoms, rows):
         inst.delete()
 
 
+@pytest.mark.parametrize("natoms,rows", [(64, 128), (300, 128), (700, 64), (1200, 256), (1500, 128)])
+def test_descreening_of_few_tiles_equals_the_plain_kernel(natoms, rows):
+    # (64 rows per block there, each wave's columns looked up apart)
+    s = synth.generate(20260600 + natoms, natoms)
+    inst = api.Instance(s)
+    try:
+        inst.set_tuning(rows=rows)
+        tiles = inst.ener()
+        inst.set_tuning(rows=rows, desc_chunk=512)
+        assert_same(tiles, inst.ener(), natoms)
+    finally:
+        inst.delete()
+
+
 @pytest.mark.parametrize("natoms,mixed,fixed", [(8, False, False), (61, False, True), (300, True, False),
                                                 (513, False, False), (1777, True, True), (2000, False, False),
                                                 (4100, True, False), (4700, False, True)])
