@@ -149,11 +149,26 @@ __global__ __launch_bounds__(kEpi) void k_born(Dev d) {
       const SysInfo &S = d.sys[d.asys[i]];
       const int nt = (S.nh + 255) / 256;
       const float *p = d.dpart + S.dp0 + (i - S.a0);
+      // (eight tiles' loads in flight: 6,000 atoms 7.2 -> 5.2 us, 11,000, 21 tiles, 11.9 -> 6.5)
       long long sum = 0;
-      for (int t0 = 0; t0 < nt; t0 += d.dt_run) {
-        double a = 0.0;
-        for (int t = t0; t < min(t0 + d.dt_run, nt); t++) a += (double)p[(size_t)t * S.n];
-        sum += __double2ll_rn(a * kFix);
+      double a = 0.0;
+      int left = d.dt_run;                   // tiles of the run still to come
+      for (int t0 = 0; t0 < nt; t0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = p[(size_t)min(t0 + u, nt - 1) * S.n];
+        // (here, not each behind its test below)
+        asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          if (t0 + u >= nt) break;
+          a += (double)v[u];
+          if (--left == 0 || t0 + u == nt - 1) {
+            sum += __double2ll_rn(a * kFix);
+            a = 0.0;
+            left = d.dt_run;
+          }
+        }
       }
       s = fix_get(sum);
     } else {
