@@ -55,10 +55,11 @@ constexpr int kChainGroupItems = 1024;
 // by pair count alone, 237 by time; the order does not touch the sums).  At
 // 40,000 atoms, 9,700 items, no difference is left to gain
 constexpr size_t kChainByTime = 8192;
-// most items of a chain rule by row groups (k_chain_split; a call of 4,000
-// atoms, 155 items, 302 -> 268 us; with up to 512, 6,000 atoms 315 -> 327), and
-// most of its blocks for which a front takes four pairs at a time
-constexpr int kSplitItems = 256, kSplitSets = 6, kSplitFour = 256;
+// most items of a chain rule by row groups (k_chain_split; calls of 4,000, 5,300
+// and 6,000 atoms, 155, 250 and 300 items, 302 -> 264, 310 -> 277 and 309 ->
+// 300 us; 6,600, 360 items, 323 -> 320), and most of its blocks for which a
+// front takes four pairs at a time
+constexpr int kSplitItems = 384, kSplitSets = 6, kSplitFour = 256;
 // most items of the GB pairs by chunks (k_gb_split; a call of 2,000 atoms, 36
 // items, 215 -> 208 us, of 2,700, 66 items, 233 -> 234, of 4,000, 136 items, 259 -> 271),
 // and sets of 4 x 256 numbers that an item's sums take there

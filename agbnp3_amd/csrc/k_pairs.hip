@@ -952,26 +952,27 @@ __device__ __forceinline__ void chain_item(const Dev &d, int it, const int4 &ite
 }
 
 // ------------------------------------- chain rule of small calls, by row groups
-// The same sums (k_chain), where its items are fewer than the CUs and one
+// The same sums (k_chain), where its items are about as few as the CUs and one
 // wave's 256 steps through its 64 rows (or 128 steps of two rows) are the
 // launch.  Those rows and the steps of a column through them fix the order of
 // every sum, so they are not cut; the work on a pair is spread over waves
 // instead.  A block takes one wave's share of an item: four waves (fronts) form
 // the terms of a batch of pairs, EACH of them each, and pass them through LDS
-// to a fifth that adds the rows' sums and a sixth that adds the columns' (its
-// lanes are columns, so nothing rotates), one batch behind.  Column sums of an
+// to four that add the GB and vdW sums of the rows and of the columns (lanes
+// are columns there, so nothing rotates), one batch behind.  Column sums of an
 // item's row groups, and row sums of its two chunk parities, leave apart and
 // k_chain_sum adds them in the order k_chain does.
 // Bound: a front's chain from the column's LDS read over the table reads to
 // its terms, once per batch.  Against k_chain: 61 atoms 20 -> 13 us, 613 57 ->
-// 24, 2,000 60 -> 26 (eight waves as fronts 30).
-constexpr int kSplitFronts = 4, kSplitWaves = kSplitFronts + 2;
+// 24, 2,000 60 -> 26 (eight waves as fronts 30); with two waves instead of four
+// behind the fronts no change there, but 5,000 atoms' call 267 -> 279 us.
+constexpr int kSplitFronts = 4, kSplitWaves = kSplitFronts + 4;
 template <int REC>
 struct SplitLds {
   float4 cpos[256], cpar[256];           // the columns (ChainChunk's records)
   float4 rpos[2][64];                    // the rows: position,
-  float2 rpar[2][64];                    // q2ab and abrw
-  float4 ring[2][REC][64];               // per pair: hgb, hvw, Q4(k <- j), Q4(j <- k)
+  float rw[2][2][64], cw[2][256];        // [0] q2ab and [1] abrw of the rows and the columns
+  float ring[2][REC][4][64];             // per pair: hgb, hvw, Q4(k <- j), Q4(j <- k)
 };
 
 template <int KIND, bool QUIRK, int EACH>
@@ -1004,6 +1005,8 @@ __device__ __forceinline__ void chain_split_item(const Dev &d, int it, int part,
     }
     L.cpos[threadIdx.x] = p;
     L.cpar[threadIdx.x] = q;
+    L.cw[0][threadIdx.x] = q.x;
+    L.cw[1][threadIdx.x] = q.y;
   }
   int rr[NR];
   float4 pk[NR];
@@ -1026,17 +1029,20 @@ __device__ __forceinline__ void chain_split_item(const Dev &d, int it, int part,
     }
     if (role == 0) {
       L.rpos[k][lane] = pk[k];
-      L.rpar[k][lane] = make_float2(q2k[k], abk[k]);
+      L.rw[0][k][lane] = q2k[k];
+      L.rw[1][k][lane] = abk[k];
     }
   }
   __syncthreads();
   const int cbeg = (item.w & 15) + cp, cend = item.w >> 4;
   const int nbatch = (cend - cbeg + NR - 1) / NR * kBatches;
-  float rg[NR][3], rv[NR][3], rU[NR], rV[NR];            // the fifth wave's row sums
+  // of the four waves behind the fronts, two add the GB sums (x, y, z and U) and
+  // two the vdW ones (and V); of each two, one the rows' and one the columns'
+  const int part2 = (role - kSplitFronts) >> 1;
+  const bool rows = ((role - kSplitFronts) & 1) == 0;
+  float g[NR][3], uv[NR];
 #pragma unroll
-  for (int k = 0; k < NR; k++)
-    rg[k][0] = rg[k][1] = rg[k][2] = rv[k][0] = rv[k][1] = rv[k][2] = rU[k] = rV[k] = 0.f;
-  float ca[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};   // the sixth wave's column sums
+  for (int k = 0; k < NR; k++) g[k][0] = g[k][1] = g[k][2] = uv[k] = 0.f;
 #pragma unroll 1
   for (int t = 0; t <= nbatch; t++) {
     if (role < kSplitFronts) {
@@ -1073,68 +1079,59 @@ __device__ __forceinline__ void chain_split_item(const Dev &d, int it, int part,
           const int k = NR == 2 ? r & 1 : 0;
           float hgb, hvw, q1, q2;
           chain_terms<KIND, QUIRK>(m[r], pj[r], pp[r], wk[k], q2k[k], abk[k], kheavy[k], c1[r], c2[r], hgb, hvw, q1, q2);
-          L.ring[t & 1][EACH * role + r][lane] = make_float4(hgb, hvw, q1, q2);
+          float (*rec)[64] = L.ring[t & 1][EACH * role + r];
+          rec[0][lane] = hgb;
+          if (KIND != CK_HX0) rec[1][lane] = hvw;
+          rec[2][lane] = q1;
+          if (!kOne) rec[3][lane] = q2;
         }
       }
-    } else if (t > 0) {
+    } else if (t > 0 && (KIND != CK_HX0 || part2 == 0)) {
       const int c = cbeg + NR * ((t - 1) / kBatches), s0 = (t - 1) % kBatches * kSteps;
-      const float4 (*ring)[64] = L.ring[(t - 1) & 1];
-      if (role == kSplitFronts) {
+      const float (*ring)[4][64] = L.ring[(t - 1) & 1];
+      if (rows) {
 #pragma unroll
         for (int r = 0; r < kRec; r++) {
           const int k = NR == 2 ? r & 1 : 0, col = (lane - s0 - r / NR) & 63;
-          const float4 pj = L.cpos[c * 64 + col], h = ring[r][lane];
+          const float4 pj = L.cpos[c * 64 + col];
+          const float h = ring[r][part2][lane];
           const float ex = pj.x - pk[k].x, ey = pj.y - pk[k].y, ez = pj.z - pk[k].z;
-          rg[k][0] = fmaf(h.x, ex, rg[k][0]); rg[k][1] = fmaf(h.x, ey, rg[k][1]); rg[k][2] = fmaf(h.x, ez, rg[k][2]);
-          if (KIND != CK_HX0) {
-            rv[k][0] = fmaf(h.y, ex, rv[k][0]); rv[k][1] = fmaf(h.y, ey, rv[k][1]); rv[k][2] = fmaf(h.y, ez, rv[k][2]);
-          }
-          if (!kOne) {
-            const float4 pp = L.cpar[c * 64 + col];
-            rU[k] = fmaf(pp.x, h.w, rU[k]);
-            rV[k] = fmaf(pp.y, h.w, rV[k]);
-          }
+          g[k][0] = fmaf(h, ex, g[k][0]); g[k][1] = fmaf(h, ey, g[k][1]); g[k][2] = fmaf(h, ez, g[k][2]);
+          if (!kOne) uv[k] = fmaf(L.cw[part2][c * 64 + col], ring[r][3][lane], uv[k]);
         }
       } else if (!diag) {
         const float4 pj = L.cpos[c * 64 + lane];
 #pragma unroll
         for (int r = 0; r < kRec; r++) {
           const int k = NR == 2 ? r & 1 : 0, row = (lane + s0 + r / NR) & 63;
-          const float4 pr = L.rpos[k][row], h = ring[r][row];
-          const float2 qa = L.rpar[k][row];
+          const float4 pr = L.rpos[k][row];
+          const float h = ring[r][part2][row];
           const float ex = pj.x - pr.x, ey = pj.y - pr.y, ez = pj.z - pr.z;
-          ca[0] = fmaf(-h.x, ex, ca[0]); ca[1] = fmaf(-h.x, ey, ca[1]); ca[2] = fmaf(-h.x, ez, ca[2]);
-          if (KIND != CK_HX0) {
-            ca[3] = fmaf(-h.y, ex, ca[3]); ca[4] = fmaf(-h.y, ey, ca[4]); ca[5] = fmaf(-h.y, ez, ca[5]);
-          }
-          ca[6] = fmaf(qa.x, h.z, ca[6]);
-          if (KIND != CK_HX0) ca[7] = fmaf(qa.y, h.z, ca[7]);
+          g[0][0] = fmaf(-h, ex, g[0][0]); g[0][1] = fmaf(-h, ey, g[0][1]); g[0][2] = fmaf(-h, ez, g[0][2]);
+          uv[0] = fmaf(L.rw[part2][k][row], ring[r][2][row], uv[0]);
         }
         if (t % kBatches == 0) {                          // the chunk's last batch
           float *o = d.chsplit + ((size_t)it * kSplitSets + rh) * 2048 + c * 64 + lane;
 #pragma unroll
-          for (int q = 0; q < 8; q++) {
-            if (KIND != CK_HX0 || q < 3 || q == 6) o[q * 256] = ca[q];
-            ca[q] = 0.f;
+          for (int q = 0; q < 3; q++) {
+            o[(3 * part2 + q) * 256] = g[0][q];
+            g[0][q] = 0.f;
           }
+          o[(6 + part2) * 256] = uv[0];
+          uv[0] = 0.f;
         }
       }
     }
     __syncthreads();
   }
-  if (role == kSplitFronts) {
+  if (role >= kSplitFronts && rows && (KIND != CK_HX0 || part2 == 0)) {
     float *pr = d.chsplit + ((size_t)it * kSplitSets + 4 + cp) * 2048;
 #pragma unroll
     for (int k = 0; k < NR; k++) {
       float *o = pr + rr[k];
-      o[0 * 256] = rg[k][0]; o[1 * 256] = rg[k][1]; o[2 * 256] = rg[k][2];
-      if (KIND != CK_HX0) {
-        o[3 * 256] = rv[k][0]; o[4 * 256] = rv[k][1]; o[5 * 256] = rv[k][2];
-      }
-      if (!kOne) {
-        o[6 * 256] = kheavy[k] ? rU[k] : 0.f;
-        o[7 * 256] = kheavy[k] ? rV[k] : 0.f;
-      }
+#pragma unroll
+      for (int q = 0; q < 3; q++) o[(3 * part2 + q) * 256] = g[k][q];
+      if (!kOne) o[(6 + part2) * 256] = kheavy[k] ? uv[k] : 0.f;
     }
   }
 }

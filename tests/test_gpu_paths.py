@@ -70,7 +70,7 @@ def test_descreening_of_few_tiles_equals_the_plain_kernel(natoms, rows):
 
 @pytest.mark.parametrize("natoms,mixed,fixed", [(8, False, False), (61, False, True), (300, True, False),
                                                 (513, False, False), (1777, True, True), (2000, False, False),
-                                                (4100, True, False), (4700, False, True)])
+                                                (4100, True, False), (4700, False, True), (6200, False, False)])
 def test_chain_rule_by_row_groups_equals_the_plain_kernel(natoms, mixed, fixed):
     """256 columns per item are what both routes use; asked for, they are the plain kernel's.  mixed: hydrogens with
     vdW terms, and some with a heavy atom's radius."""
