@@ -64,6 +64,8 @@ constexpr int kSplitItems = 384, kSplitSets = 6, kSplitFour = 256;
 // items, 215 -> 208 us, of 2,700, 66 items, 233 -> 234, of 4,000, 136 items, 259 -> 271),
 // and sets of 4 x 256 numbers that an item's sums take there
 constexpr int kGbSplitItems = 48, kGbSets = 5;
+// nodes of one order that the overlap tree's first tier holds in LDS
+constexpr int kLevelCap = 128;
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;
@@ -78,7 +80,7 @@ constexpr double kFixInv = 1.0 / 4294967296.0;
 // status word bits (device side capacity / topology checks)
 enum : int {
   ST_NBLIST_OVERFLOW = 1,   // a neighbour-list row exceeded the row capacity
-  ST_TREE_OVERFLOW = 2,     // an overlap group exceeded its LDS capacity
+  ST_TREE_OVERFLOW = 2,     // a root of pass B's first tier outgrew its buffers
   ST_WS_OVERFLOW = 4,       // a water site had more candidates than its buffer
   ST_GRID_OVERFLOW = 8,     // cell grid larger than allocated
 };
@@ -284,6 +286,7 @@ struct Dev {
                                        // [6], [7] roots walked depth first (pass A, B)
   int *tree_ovf;                       // [2][nh] heavy rows of the roots queued for the second tier, for pass B's depth-first walk
   uint2 *tree_cnt;                     // [nh] overlaps kept and evaluated by pass A's first tier (in A's memory, until k_q2ab)
+  int tree_cap_b;                      // nodes of one order pass B's first tier takes (kLevelCap; lower for tests)
   unsigned char *tree_tier;            // [nh] pass A's first tier: 0 walked there, 1 queued for the next
   double *volumep_raw, *sa_raw, *sa_f, *sp, *spe, *psvol, *gammap;   // [n]
   float *sp_f, *spe_f;                 // FP32 copies for pair kernels

@@ -391,7 +391,7 @@ __device__ __forceinline__ void vol_switch(float v, float &s, float &sp, float &
   if (v < kVolMinA) { s = 0.f; sp = 0.f; spp = 0.f; return; }
   const float d = 1.0f / (kVolMinB - kVolMinA);
   const float u = (v - kVolMinA) * d, u2 = u * u;
-  s = u2 * u * (10.f - 15.f * u + 6.f * u2);
+  s = u2 * u * fmaf(6.f, u2, fmaf(-15.f, u, 10.f));     // (fused as written: overlap(), k_tree.hip)
   sp = d * 30.f * u2 * (1.f - 2.f * u + u2);
   spp = d * d * 60.f * u * (1.f - 3.f * u + 2.f * u2);
 }

@@ -942,6 +942,13 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
     const int v = atoi(e);
     if (v >= 1 && v <= 128) d.ws_cap1 = v;
   }
+  // likewise the nodes that the derivative pass's first tier takes, from
+  // AGBNP3_TREE_DERIV_CAP, so a test can have a root outgrow it alone
+  d.tree_cap_b = kLevelCap;
+  if (const char *e = getenv("AGBNP3_TREE_DERIV_CAP")) {
+    const int v = atoi(e);
+    if (v >= 1 && v <= kLevelCap) d.tree_cap_b = v;
+  }
   std::vector<float> ty((size_t)P.ntypes * P.ntypes * kTblN), ty2(ty.size());
   for (int a = 0; a < P.ntypes; a++)
     for (int b = 0; b < P.ntypes; b++) {

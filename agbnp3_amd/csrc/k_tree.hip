@@ -69,30 +69,35 @@ struct Gauss {
   float a, p, x, y, z;
 };
 
-// FP32 Gaussian overlap of `par` with atom (ab, xb) (kernels.c:2418-2477)
+// FP32 Gaussian overlap of `par` with atom (ab, xb) (kernels.c:2418-2477).
+// What an overlap is and passes on (V, exponent, prefactor, centre, and with
+// vol_switch V') has its fused products written out and no others: this is
+// inlined into every walk of both passes, and all of them have to keep the same
+// overlaps (left to the compiler, a walk may fuse another product of a sum
+// than the next one, and pass B keep an overlap that pass A dropped).
 struct OvlOut {
   float V, Vp, fp, fpp, a, p, cx, cy, cz, dinv;
 };
 __device__ __forceinline__ OvlOut overlap(const Gauss &par, float ab, float xb, float yb, float zb) {
   OvlOut o;
-  const float dx = xb - par.x, dy = yb - par.y, dz = zb - par.z;
-  const float d2 = dx * dx + dy * dy + dz * dz;
-  const float a12 = par.a + ab;
-  const float dinv = __builtin_amdgcn_rcpf(a12);                    // hardware reciprocal, exp, sqrt (1-2 ulp)
-  const float p12 = par.p * kPFC * __expf(-par.a * ab * d2 * dinv);
-  const float u = kPiF * dinv;
-  o.V = p12 * u * __builtin_amdgcn_sqrtf(u);
   float s, sp, spp;
-  vol_switch(o.V, s, sp, spp);
-  o.Vp = s * o.V;
+  {
+#pragma clang fp contract(off)
+    const float dx = xb - par.x, dy = yb - par.y, dz = zb - par.z;
+    const float d2 = fmaf(dz, dz, fmaf(dx, dx, dy * dy));
+    o.a = par.a + ab;
+    o.dinv = __builtin_amdgcn_rcpf(o.a);                            // hardware reciprocal, exp, sqrt (1-2 ulp)
+    o.p = par.p * kPFC * __expf(-par.a * ab * d2 * o.dinv);
+    const float u = kPiF * o.dinv;
+    o.V = o.p * u * __builtin_amdgcn_sqrtf(u);
+    vol_switch(o.V, s, sp, spp);
+    o.Vp = s * o.V;
+    o.cx = o.dinv * fmaf(par.a, par.x, ab * xb);
+    o.cy = o.dinv * fmaf(par.a, par.y, ab * yb);
+    o.cz = o.dinv * fmaf(par.a, par.z, ab * zb);
+  }
   o.fp = s + o.V * sp;
   o.fpp = 2.f * sp + o.V * spp;
-  o.a = a12;
-  o.p = p12;
-  o.cx = dinv * (par.a * par.x + ab * xb);
-  o.cy = dinv * (par.a * par.y + ab * yb);
-  o.cz = dinv * (par.a * par.z + ab * zb);
-  o.dinv = dinv;
   return o;
 }
 
@@ -419,7 +424,6 @@ __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned
 }
 
 // ------------------------------------------------------ breadth-first tree
-constexpr int kLevelCap = 128;          // nodes of one order held in LDS
 constexpr int kLevelCapBig = 512;       // second tier (dynamic LDS) for the largest trees
 
 // slot accumulators: FP64 with one wave per root (FP64 LDS atomics measured
@@ -598,9 +602,14 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
   if (PB && list == 0 && __builtin_amdgcn_readfirstlane(tier)) return true;  // block-uniform
   // a root that outgrows these buffers: pass A's first tier queues it for the
   // second (and records that); past the second tier it is walked depth first,
-  // in pass A by the caller, in pass B from a list
+  // in pass A by the caller, in pass B from a list.  None does in pass B's first
+  // tier, which has the roots whose same walk fitted pass A's; one that did
+  // would find nothing behind it that walks it, and fails the call.
+  const int lc = PB && list == 0 ? d.tree_cap_b : LC;
   auto queue_next = [&]() {
-    if (tid == 0) {
+    if (PB && list == 0) {
+      if (tid == 0) atomicOr(d.status, ST_TREE_OVERFLOW);
+    } else if (tid == 0) {
       const bool first = !PB && list == 0;
       const unsigned k = atomicAdd(&d.counters[first ? 4 : 6 + (PB ? 1 : 0)], 1ull);
       if (first || PB) d.tree_ovf[(PB ? (size_t)d.nh : 0) + k] = h;
@@ -678,16 +687,16 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
       n += total;
     }
     nkept += (unsigned)n;
-    if (n > LC) ovf = true;
+    if (n > lc) ovf = true;
     for (int k = tid; k < n && k < LC; k += NT) S.gend[0][k] = (std::remove_reference_t<decltype(S.gend[0][0])>)n;
     __syncthreads();
   }
   if (!ovf && n > 1) {
     n = bfs_order<3, CAP, PB, LC, W, true>(S, 0, n, root, df, nkept, neval);
-    if (n > LC) ovf = true;
+    if (n > lc) ovf = true;
     else if (n > 1) {
       n = bfs_order<4, CAP, PB, LC, W, true>(S, 1, n, root, df, nkept, neval);
-      if (n > LC) ovf = true;
+      if (n > lc) ovf = true;
       else if (n > 1) bfs_order<5, CAP, PB, LC, W, false>(S, 0, n, root, df, nkept, neval);
     }
   }
