@@ -819,7 +819,14 @@ __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
   add_tree_counts(d, PB, tk, te);
 }
 
-// pass B's depth-first walk of the roots its second tier listed
+// pass B's depth-first walk of the roots its second tier listed: one wave each,
+// as many at a time as the CUs hold, since a root here takes a millisecond or
+// more where solutes are dense (coordinates of the synthetic solute scaled by
+// 0.8, so that a third of the roots come here; calls with 64, 256 and 1,024
+// blocks: 6,000 atoms by 0.75 74.4, 30.4 and 21.7 ms, 25,000 by 0.8 94.7, 33.5
+// and 21.5 ms).  Blocks without a root cost nothing: 6,000 and 25,000 atoms as
+// generated 299 and 945 us with either number.
+constexpr int kDfsBlocks = 1024;
 template <int CAP>
 __global__ __launch_bounds__(64) void k_tree_dfs(Dev d) {
   __shared__ TreeLds<CAP, true> S;
@@ -847,11 +854,11 @@ hipError_t prepare_tree() {
   return e;
 }
 
-// persistent grids: resident blocks for the breadth-first pass, two per CU
-// for the second tier
+// the first tier a block per root unless a grid is asked for; the second a
+// persistent grid of two blocks per CU
 template <int CAP>
 static void launch_tree_cap(const Dev &d, const Tuning &t, int pass, int tier, hipStream_t s) {
-  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : d.nh), gf = std::min(d.nh, 64);
+  const int g = std::min(d.nh, t.tree_grid > 0 ? t.tree_grid : d.nh), gf = std::min(d.nh, kDfsBlocks);
   const int gb = std::min(d.nh, 512);
   const size_t la = big_lds<CAP, false>(), lb = big_lds<CAP, true>();
   if (pass == 0) {
