@@ -245,3 +245,26 @@ def test_water_sites_past_the_first_launch_capacity():
     finally:
         small.delete()
         ref.delete()
+
+
+@pytest.mark.parametrize("natoms,chunk", [(3000, 512), (17001, 0)])
+def test_water_sites_listed_for_the_second_launch(natoms, chunk):
+    """Where the descreening is the plain kernel's (asked for, or in large calls, whose sites run on the second stream),
+    the sites past the first launch's capacity go to a launch of their own."""
+    s = synth.generate(20262900 + natoms, natoms)
+    insts = [api.Instance(s)]
+    os.environ["AGBNP3_WS_FIRST_CAP"] = "8"          # read when the instance is built
+    try:
+        insts.append(api.Instance(s))
+    finally:
+        del os.environ["AGBNP3_WS_FIRST_CAP"]
+    try:
+        for i in insts:
+            i.set_tuning(desc_chunk=chunk)
+        b, a = (i.ener() for i in insts)
+        for name in OUTS + api.ENERGY_NAMES:
+            assert np.array_equal(np.asarray(a[name]), np.asarray(b[name])), name
+        assert b["ehb"] != 0.0 and np.any(b["dehb"] != 0.0)
+    finally:
+        for i in insts:
+            i.delete()
