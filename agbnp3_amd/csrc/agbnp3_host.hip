@@ -1061,9 +1061,9 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   launch_sg_audit(d, s);
   if (fork) {
     HIPCHK(hipStreamWaitEvent(s, P.ev_join, 0));
-  } else if (!d.dt_on) {
-    launch_ws_free(d, s);
-    mark("ws_free");
+  } else {
+    if (!d.dt_on) launch_ws_free(d, s);
+    mark("ws_free");                     // (every call has the same marks: pack_kernel_times)
   }
   launch_chain(d, t, s);
   mark("chain");
