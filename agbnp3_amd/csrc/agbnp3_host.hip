@@ -991,6 +991,11 @@ int build_pack(Pack &P, const std::vector<const Model *> &ms, int options) {
 }
 
 // ---------------------------------------------------------- the pipeline
+// GB pairs by chunks, unless a grid is asked for
+bool gb_by_chunks(const Dev &d) {
+  return d.ngb_items <= kGbSplitItems && d.nchain_items <= kChainGroupItems && !d.sg_on;
+}
+
 // The kernels of one call on the pack's stream, with `d` the device view (the
 // pack's own, or a copy whose per-call state lies in the static scratch).
 // `capturing`: inside a graph capture (no timing events).
@@ -1003,7 +1008,7 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   d.reuse_every = P.reuse_every;
   d.dt_on = P.dt && !d.sg_on;
   d.split_on = P.split && !d.sg_on;
-  d.gbs_on = d.ngb_items <= kGbSplitItems && P.tune.gb_grid == 0 && d.nchain_items <= kChainGroupItems && !d.sg_on;
+  d.gbs_on = gb_by_chunks(d) && P.tune.gb_grid == 0;
   hipStream_t s = P.stream;
   const bool timed = !capturing && (P.options & AGBNP3_OPT_TIMING) != 0;
   int k = 0;
@@ -1375,25 +1380,47 @@ int pack_tune(Pack &P, const double *x, const double *y, const double *z, int re
     if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess)
       cu = prop.multiProcessorCount;
   }
-  // each step: a parameter, its candidates, the kernels whose time decides
+  // each step: a parameter, its candidates, the kernels whose time decides.
+  // Some candidates move work between kernels (the tiled descreening holds the
+  // water sites, the GB pairs by chunks what k_q2ab does), so these count
+  // together.  (The descreening by itself chose 1,024 columns at 61 atoms, on a
+  // tie: 120 -> 136 us a call.)
   struct Axis {
     int param;
     std::vector<int> cand;
     std::vector<std::string> kernels;
   };
   const std::vector<Axis> axes = {
-      {TUNE_ROWS, {64, 128, 256}, {"descreen"}},
-      {TUNE_DESC_CHUNK, {0, 512, 1024, 2048, 4096}, {"descreen"}},
-      {TUNE_DESC_GRID, {0, 2 * cu, 4 * cu, 8 * cu}, {"descreen"}},
-      {TUNE_GB_GRID, {0, 2 * cu, 4 * cu, 8 * cu}, {"gbpair"}},
+      {TUNE_ROWS, {64, 128, 256}, {"descreen", "ws_free"}},
+      {TUNE_DESC_CHUNK, {0, 512, 1024, 2048, 4096}, {"descreen", "ws_free"}},
+      {TUNE_DESC_GRID, {0, 2 * cu, 4 * cu, 8 * cu}, {"descreen", "ws_free"}},
+      {TUNE_GB_GRID, {0, 2 * cu, 4 * cu, 8 * cu}, {"gbpair", "q2ab"}},
       {TUNE_CHAIN_CHUNK, {0, 128, 64}, {"chain"}},
       {TUNE_CHAIN_GRID, {0, 2 * cu, 4 * cu, 8 * cu}, {"chain"}},
       {TUNE_TREE_GRID, {0, 8 * cu, 32 * cu}, {"tree_volumes", "tree_derivs"}},
   };
   for (const Axis &ax : axes) {
+    // grids of kernels that this pack's calls don't launch stay as they are, and
+    // candidates that are what 0 stands for are left out: a choice among equals
+    // would be recorded for the class's other packs, and may take another route
+    // from them
+    if (params_to_tuning(P, p) != AGBNP_OK) {
+      P.options = saved_opts;
+      return AGBNP_ERR;
+    }
+    if (!P.d.sg_on && ((ax.param == TUNE_DESC_GRID && P.dt) || (ax.param == TUNE_CHAIN_GRID && P.split))) continue;
+    const Dev &d = P.d;
+    int same = INT_MAX;                  // grids from here are a block per item
+    if (ax.param == TUNE_DESC_GRID) same = d.ndesc_items;
+    if (ax.param == TUNE_GB_GRID && !gb_by_chunks(d)) same = d.ngb_items;
+    if (ax.param == TUNE_CHAIN_GRID) same = d.nchain_items;
+    if (ax.param == TUNE_TREE_GRID) same = d.nh;
+    // and the columns that 0 stands for (with tiles it is another kernel)
+    const int cols = ax.param == TUNE_DESC_CHUNK && p[ax.param] == 0 && !(P.dt && !d.sg_on) ? 256 * d.dt_run : 0;
     int best = p[ax.param];
     double best_t = 1e30;
     for (int c : ax.cand) {
+      if (c > 0 && (c >= same || c == cols)) continue;
       int q[TUNE_COUNT];
       memcpy(q, p, sizeof(q));
       q[ax.param] = c;
@@ -1402,8 +1429,12 @@ int pack_tune(Pack &P, const double *x, const double *y, const double *z, int re
         return AGBNP_ERR;
       }
       double tt = 0.0;
-      for (const auto &kname : ax.kernels) tt += t[kname];
-      snprintf(line, sizeof(line), "param %d = %d: %.4f ms\n", ax.param, c, tt);
+      std::string counted;
+      for (const auto &kname : ax.kernels) {
+        tt += t[kname];
+        counted += " " + kname;
+      }
+      snprintf(line, sizeof(line), "param %d = %d: %.4f ms (%s)\n", ax.param, c, tt, counted.c_str() + 1);
       rep += line;
       if (tt < best_t) { best_t = tt; best = c; }
     }
