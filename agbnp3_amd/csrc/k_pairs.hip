@@ -192,7 +192,6 @@ void launch_descreen(const Dev &d, const Tuning &t, hipStream_t s) {
 __device__ __forceinline__ float wave_rot(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x13C, 0xF, 0xF, true));
 }
-__device__ __forceinline__ int wave_rot(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x13C, 0xF, 0xF, true); }
 
 // the same rotation through the LDS crossbar (rot_from: the byte address of
 // the lane that lane l takes its value from)

@@ -108,10 +108,10 @@ __device__ __forceinline__ float sa_term(const OvlOut &o, float sign, float a, f
   return sign * o.fp * a * o.V * (3.f * o.dinv + 2.f * t) * __builtin_amdgcn_rcpf(R);
 }
 
-// add to a per-slot accumulator: FP64 LDS atomics with one wave per root
-// (the lanes' order is fixed), or 64-bit fixed point with integer atomics
-// with several waves per root (the sum does not depend on their order; an
-// LDS add of a zero costs less than testing for it)
+// add to a per-slot accumulator: FP64 LDS atomics in the depth-first walk, one
+// wave per root (the lanes' order is fixed), or 64-bit fixed point with integer
+// atomics in the breadth-first ones with their several waves (the sum does not
+// depend on their order; an LDS add of a zero costs less than testing for it)
 __device__ __forceinline__ void slot_add(double *p, double v) { atomicAdd(p, v); }
 __device__ __forceinline__ void slot_add(long long *p, double v) {
   atomicAdd((unsigned long long *)p, (unsigned long long)__double2ll_rn(v * kFix));
@@ -122,7 +122,6 @@ __device__ __forceinline__ void slot_add(long long *p, double v) {
 // conversion's seven FP64 instructions, 12 times per member of every overlap.
 // 2,000 atoms: call 219 -> 216 us, 25,000 984 -> 977, 64 poses 800 -> 786.
 constexpr float kSmall = 524288.f;
-__device__ __forceinline__ void slot_add_small(double *p, double v) { atomicAdd(p, v); }
 __device__ __forceinline__ void slot_add_small(long long *p, double v) {
   constexpr double c = 1572864.0;
   atomicAdd((unsigned long long *)p,
@@ -426,11 +425,6 @@ __device__ void tree_dfs_root(const Dev &d, TreeLds<CAP, PB> &S, int h, unsigned
 // ------------------------------------------------------ breadth-first tree
 constexpr int kLevelCapBig = 512;       // second tier (dynamic LDS) for the largest trees
 
-// slot accumulators: FP64 with one wave per root (FP64 LDS atomics measured
-// faster than FP32 ones here), fixed point with several waves
-template <int W> struct SlotAcc { using T = long long; };
-template <> struct SlotAcc<1> { using T = double; };
-
 template <int CAP, bool PB, int LC, int W>
 struct BfsLds {
   int idx[CAP + 1];
@@ -439,7 +433,7 @@ struct BfsLds {
   float4 p[CAP + 1];
   float r[PB ? 1 : CAP + 1];
   float4 q[PB ? CAP + 1 : 1], w[PB ? CAP + 1 : 1];
-  typename SlotAcc<W>::T acc[PB ? TG_N : 2][CAP + 1];
+  long long acc[PB ? TG_N : 2][CAP + 1];
   // two node buffers: Gaussian, member slots (16 bits each, root excluded),
   // end of the node's sibling group, parent index in the previous order
   float ga[2][LC], gp[2][LC], gx[2][LC], gy[2][LC], gz[2][LC];
@@ -464,10 +458,6 @@ template <int W>
 __device__ __forceinline__ int pass_compact(int (&wcnt)[2][W], int parity, unsigned long long bal, int &total) {
   const int lane = threadIdx.x & 63;
   const int below = __popcll(bal & ((1ull << lane) - 1ull));
-  if (W == 1) {
-    total = __popcll(bal);
-    return below;
-  }
   const int w = threadIdx.x >> 6;
   if (lane == 0) wcnt[parity][w] = __popcll(bal);
   __syncthreads();
@@ -483,7 +473,6 @@ __device__ __forceinline__ int pass_compact(int (&wcnt)[2][W], int parity, unsig
 }
 
 // per-atom fixed-point totals from the slot accumulators
-__device__ __forceinline__ void scatter_add(long long *p, double v) { fix_add(p, v); }
 __device__ __forceinline__ void scatter_add(long long *p, long long q) {
   if (q != 0) atomicAdd((unsigned long long *)p, (unsigned long long)q);
 }
@@ -581,9 +570,9 @@ __device__ __forceinline__ int bfs_order(BfsLds<CAP, PB, LC, W> &S, int cb, int 
 }
 
 // one root of the breadth-first tree (the whole block); results scattered to
-// the atoms, or the root queued for the next tier on overflow.  With W > 1
-// the block's waves split every order's candidates and the per-slot sums are
-// fixed point, so the result does not depend on the waves' timing.
+// the atoms, or the root queued for the next tier on overflow.  The block's
+// waves split every order's candidates and the per-slot sums are fixed point,
+// so the result does not depend on the waves' timing.
 template <int CAP, bool PB, int LC, int W>
 __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, int list, unsigned long long &tk,
                               unsigned long long &te) {
@@ -705,33 +694,21 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
     return false;
   }
   if (!PB && list == 0 && tid == 0) d.tree_tier[h] = 0;
-  // the root's own sums (slot 0 takes no member adds): lane 0 of the wave,
-  // or with several waves fixed-point adds of each wave's sum
-  double rsum[TG_N];
+  // the root's own sums (slot 0 takes no member adds): each wave's
 #pragma unroll
   for (int v = 0; v < (PB ? TG_N : 2); v++) {
-    rsum[v] = wave_sum((double)root[v]);
-    if (W > 1 && lane == 0) slot_add(&S.acc[v][0], rsum[v]);
+    const double sum = wave_sum((double)root[v]);
+    if (lane == 0) slot_add(&S.acc[v][0], sum);
   }
-  if (W > 1 && lane == 0) S.wcnt[0][tid >> 6] = (int)neval;
-  if (W > 1) __syncthreads();
+  if (lane == 0) S.wcnt[0][tid >> 6] = (int)neval;
+  __syncthreads();
   if (!PB && list == 0 && tid == 0) {     // pass A's first tier: its counts, which k_scale adds up
     unsigned ev = 0;
 #pragma unroll
     for (int w = 0; w < W; w++) ev += (unsigned)S.wcnt[0][w];
     d.tree_cnt[h] = make_uint2(nkept, ev);
   }
-  if (W == 1 && tid == 0) {
-    const int at = S.idx[0];
-    if (!PB) {
-      fix_add(&d.acc_vol[at], rsum[0]);
-      fix_add(&d.acc_sa[at], rsum[1]);
-    } else {
-#pragma unroll
-      for (int v = 0; v < TG_N; v++) fix_add(&d.acc_grad[(size_t)at * TG_N + v], rsum[v]);
-    }
-  }
-  for (int s = (W == 1 ? 1 + tid : tid); s <= m; s += NT) {
+  for (int s = tid; s <= m; s += NT) {
     const int at = S.idx[s];
     if (!PB) {
       scatter_add(&d.acc_vol[at], S.acc[0][s]);
@@ -743,7 +720,7 @@ __device__ bool tree_bfs_root(const Dev &d, BfsLds<CAP, PB, LC, W> &S, int h, in
   }
   tk += nkept;                          // block-uniform: wave 0 reports it
   te += neval;                          // this wave's evaluations
-  if (W > 1) __syncthreads();           // the next root restages the slots
+  __syncthreads();                      // the next root restages the slots
   return true;
 }
 
