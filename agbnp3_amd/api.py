@@ -28,7 +28,7 @@ EXPORTED = (
     "agbnp3_set_options", "agbnp3_ener_device", "agbnp3_ener_static", "agbnp3_sync", "agbnp3_stream",
     "agbnp3_natoms",
     "agbnp3_get_int2ext", "agbnp3_get_near_list", "agbnp3_get_tables", "agbnp3_get_internal",
-    "agbnp3_get_counts", "agbnp3_kernel_times", "agbnp3_q4_tables",
+    "agbnp3_get_counts", "agbnp3_get_routes", "agbnp3_kernel_times", "agbnp3_q4_tables",
     "agbnp3_get_tuning", "agbnp3_set_tuning", "agbnp3_tune", "agbnp3_tune_table_save", "agbnp3_tune_table_load",
     "agbnp3_tune_table_clear",
     "agbnp3_batch_new", "agbnp3_batch_delete", "agbnp3_batch_offsets", "agbnp3_batch_set_options",
@@ -101,6 +101,7 @@ def load():
         L.agbnp3_get_tables.argtypes = [ci, vp, vp, vp]
         L.agbnp3_get_internal.argtypes = [ci, ctypes.c_char_p, vp]
         L.agbnp3_get_counts.argtypes = [ci, vp]
+        L.agbnp3_get_routes.argtypes = [ci, vp]
         L.agbnp3_kernel_times.argtypes = [ci, vp, ci, ctypes.c_char_p, ci]
         L.agbnp3_q4_tables.argtypes = [ci, vp, vp, vp, vp]
         L.agbnp3_get_tuning.argtypes = [ci, vp, ci]
@@ -341,6 +342,13 @@ class Instance:
         return dict(kept_overlaps=int(c[0]), evaluated_overlaps=int(c[1]), water_sites=int(c[2]),
                     near_pairs=int(c[3]), max_row=int(c[4]), tree_fallback_volumes=int(c[5]),
                     tree_fallback_derivatives=int(c[6]))
+
+    def routes(self):
+        """The sum of agbnp3_get_routes (agbnp3_amd.h) for the last call."""
+        r = ctypes.c_int(0)
+        if load().agbnp3_get_routes(self.tag, ctypes.byref(r)) != AGBNP_OK:
+            raise RuntimeError("agbnp3_get_routes failed")
+        return r.value
 
     def kernel_times(self):
         ms = np.zeros(64, np.float32)

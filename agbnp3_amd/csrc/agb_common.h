@@ -386,6 +386,7 @@ hipError_t prepare_pairs(int ntypes);
 void launch_ws_free(const Dev &d, hipStream_t s);
 // descreening by tiles and the water sites' free volumes (dt_on)
 void launch_desc_sites(const Dev &d, hipStream_t s);
+bool desc_sites_few(const Dev &d);       // 64 rows per block there
 hipError_t prepare_sites(int ntypes);
 void launch_sg_front(const Dev &d, hipStream_t s);
 void launch_sg_grad(const Dev &d, hipStream_t s);

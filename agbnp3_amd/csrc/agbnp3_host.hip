@@ -241,6 +241,7 @@ struct Pack {
   unsigned long long *hstat = nullptr; // pinned: status word and counters 0..3 of the last call
   std::vector<void *> pinned;          // what the two lie in
   bool host_status = false;            // the last call put its status there
+  int routes = 0;                      // agbnp3_get_routes
   // timing mode: one event set per recorded call, averaged when read back
   std::vector<std::vector<hipEvent_t>> ev_sets;
   std::vector<std::string> ev_names;
@@ -1094,7 +1095,12 @@ int run_pipeline_on(Pack &P, Dev &d, const double *x, const double *y, const dou
   mark("tree_derivs");
   launch_final(d, sp, br, sa, dgbdr, dvwdr, decav, dehb, energies, s);
   mark("final");
-  if (!capturing) P.host_status = d.hstat != nullptr;
+  if (!capturing) {
+    P.host_status = d.hstat != nullptr;
+    const bool group = d.nchain_items <= kChainGroupItems;
+    P.routes = (d.dt_on ? 1 | (desc_sites_few(d) ? 2 : 0) : (d.cull_desc ? 4 : 0)) | (d.gbs_on ? 8 : 0) |
+               (d.split_on ? 16 : (group ? 32 : (d.cull_chain ? 64 : 0)));
+  }
   HIPCHK(hipGetLastError());
   return AGBNP_OK;
 }
@@ -1946,6 +1952,13 @@ int agbnp3_get_counts(int tag, long long *counts) {
   counts[4] = (long long)c[3];
   counts[5] = (long long)(c[4] + c[6]);
   counts[6] = (long long)(c[4] + c[7]);
+  return AGBNP_OK;
+}
+
+int agbnp3_get_routes(int tag, int *routes) {
+  Instance *I = get_instance(tag, "agbnp3_get_routes()");
+  if (!I) return AGBNP_ERR;
+  *routes = I->p.routes;
   return AGBNP_OK;
 }
 

@@ -667,10 +667,14 @@ hipError_t prepare_sites(int ntypes) {
   return e;
 }
 
+// about a block per CU, which is what its LDS allows
+bool desc_sites_few(const Dev &d) {
+  return (d.nws + kWsWaves - 1) / kWsWaves + d.ndt_items * (d.rows / 64) <= kDtFew;
+}
+
 void launch_desc_sites(const Dev &d, hipStream_t s) {
   const int ns = (d.nws + kWsWaves - 1) / kWsWaves, subs = d.ndt_items * (d.rows / 64);
-  // few: about a block per CU, which is what its LDS allows
-  const bool few = ns + subs <= kDtFew;
+  const bool few = desc_sites_few(d);
   const int nb = ns + (few ? subs : d.ndt_items);
   if (nb)
     hipLaunchKernelGGL(few ? k_desc_sites<true> : k_desc_sites<false>, dim3(nb), dim3(256), desc_sites_lds(d.ntypes, few), s,

@@ -229,6 +229,13 @@ int agbnp3_get_internal(int tag, const char *name, double *out);
    [3] neighbour-list entries, [4] max row length, [5] [6] overlap-tree roots
    that outgrew the breadth-first level buffers (volumes, derivatives) */
 int agbnp3_get_counts(int tag, long long *counts);
+/* which of the kernels that a rule on sizes chooses between the last call took
+   (in agbnp3_ener_*, not a graph's replay): the sum of
+   1 descreening by tiles, 2 with 64 rows per block of those, 4 descreening
+   that passes over far columns, 8 GB pairs by chunks, 16 chain rule by row
+   groups, 32 chain rule with its lookups in groups, 64 chain rule that passes over far
+   columns; 0 before the first call */
+int agbnp3_get_routes(int tag, int *routes);
 /* per-kernel times (ms), averaged over the calls made since the previous
    read while AGBNP3_OPT_TIMING was set (HIP events on the instance stream);
    returns the number of kernels written; names joined by ';' */
