@@ -782,8 +782,7 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
     take(*q, n);
   take(d.dcol, n);
   take(d.dcw, n);
-  take(d.cbox, 2 * (size_t)std::max(nablk, 1) * (256 / kBoxCols));
-  take(d.chbox, 8 * (size_t)std::max(d.ncblk, 1));
+  if (d.cull_chain) take(d.chbox, 8 * (size_t)std::max(d.ncblk, 1));
   take(d.gb_epart, (size_t)std::max(ntile, 1));
   const size_t ngbs = ntile <= kGbSplitItems ? ntile : 0;
   take(d.gbsplit, ngbs * kGbSets * 1024);
@@ -793,6 +792,10 @@ size_t carve_call_state(Dev &d, char *base, int n_, int nh_, int nsys, int nws_,
   take(d.epart, (size_t)EP_COUNT * std::max(nablk, 1));
   take(d.dpart, ndpart);
   take(d.chpart, (size_t)nchain * 2 * 8 * 256);
+  // the descreening's boxes are read before the chain rule writes there
+  const size_t nbox = d.cull_desc ? 2 * (size_t)std::max(nablk, 1) * (256 / kBoxCols) : 0;
+  if (nbox * sizeof(float4) <= (size_t)nchain * 2 * 8 * 256 * sizeof(float)) d.cbox = reinterpret_cast<float4 *>(d.chpart);
+  else take(d.cbox, nbox);
   take(d.chsplit, nsplit);
   take(d.ch_done, (size_t)nchain);
   take(d.ch_flag, 4 * (size_t)std::max(d.ncblk, 1));

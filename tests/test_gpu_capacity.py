@@ -268,3 +268,23 @@ def test_water_sites_listed_for_the_second_launch(natoms, chunk):
     finally:
         for i in insts:
             i.delete()
+
+
+def test_static_scratch_of_few_heavy_atoms(capfd):
+    """A large solute with few heavy atoms and no water sites: the boxes of far columns take nothing from the static
+    scratch, or solutes at its limit would no longer fit (161,270,272 bytes without them)."""
+    n = 45000
+    s = synth.generate(77 + n, n)
+    heavy = np.setdiff1d(np.arange(n), s.ihydrogen)
+    more = np.random.default_rng(1).permutation(heavy)[int(0.6 * len(heavy)):]
+    s = dataclasses.replace(s, ihydrogen=np.sort(np.concatenate([s.ihydrogen, more])).astype(np.int32),
+                            hbtype=np.zeros_like(s.hbtype))
+    inst = api.Instance(s)
+    io = DeviceIO(n)
+    try:
+        io.set_xyz(s.x, s.y, s.z)
+        assert api.load().agbnp3_ener_static(inst.tag, *io.ptrs()) == api.AGBNP_ERR
+        assert int(capfd.readouterr().err.split(" needs ")[1].split()[0]) <= 161270272
+    finally:
+        io.free()
+        inst.delete()
