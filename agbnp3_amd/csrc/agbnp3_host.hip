@@ -578,7 +578,7 @@ int build_items(Pack &P) {
   for (int k = 0; k < (int)rblk.size() && (int)dt.size() <= kDtItems; k++) {
     const SysInfo &S = P.sinfo[rblk[k].y];
     for (int c = 0, t = 0; c < S.nh; c += 256, t++)
-      dt.push_back(make_int4(k, S.a0 + c, S.a0 + std::min(S.nh, c + 256), S.dp0 + t * S.n - S.a0));
+      dt.push_back(make_int4(k, S.a0 + c, S.a0 + std::min(S.nh, c + 256), (int)(S.dp0 + (long long)t * S.n - S.a0)));
   }
   P.dt = P.tune.desc_chunk <= 0 && P.ntypes <= kLdsTypes && (int)dt.size() <= kDtItems;
   if (!P.dt) dt.clear();
