@@ -22,19 +22,23 @@ constexpr double kTokcal = 332.0;
 constexpr double kRwNp = 1.4;           // water radius in the vdW term
 constexpr float kHbLength = 2.5f, kHbRadius = 1.4f;
 constexpr float kHbSwA = 0.65f, kHbSwB = 1.0f, kHbSwA0 = 0.6f;
-// per-call device counters: [0..7] scalars (see agbnp3_get_counts); the
-// overlap-tree kept / evaluated totals spread over kCountSlots 64-byte lines
-// (kCountBase + 8 s, + 1), so the blocks' adds at exit do not queue on one
-// address
 // atoms from which a call runs the water-site kernels on a second stream, and
-// from which the second tier of the derivative pass has that stream
+// from which one tier of the derivative pass has that stream.  A process's
+// streams share four hardware queues, so several instances in flight gain less
+// by it (us a call, with the stream against without: one of 2,000 atoms 200
+// against 210, four 97 to 103 against 113, eight 97 to 103 against 89 to 98; one
+// of 11,003 419 against 427, four 259 against 290)
 constexpr int kForkAtoms = 16384;
 constexpr int kSideAtoms = 512;
-// heavy atoms from which the derivative pass's second tier is launched first:
-// its blocks, two to a CU, otherwise find no room before the first tier ends
-// (40,000 atoms, 19,000 of them heavy, call 1994 -> 1966 us, 12 x 6000 1245 ->
-// 1224; 25,000 no change, 11,000 429 -> 437; in a replayed graph of 64 or 90
-// systems 1 % slower)
+// heavy atoms from which the derivative pass's second tier starts before the
+// first: its blocks, two to a CU, otherwise find no room before that one ends
+// (12 x 6000, 35,000 heavy atoms, call 1193 -> 1180 us, 64 systems of 2,000 1451
+// -> 1431, 60,000 atoms 3700 -> 3661, 40,000, 19,000 heavy, 1933 -> 1922; 25,000
+// and 34,000, 12,000 and 16,000 heavy, no change, 11,000 429 -> 437).  What the
+// call's own stream is given starts at once, the second stream's 6 us later,
+// behind its event; in a replayed graph the tier recorded first starts at once
+// (both seen in a kernel trace), so a capture keeps the second tier, recorded
+// first, on the side branch (the other way 24 x 6000 2230 -> 2272 us)
 constexpr int kBigFirst = 16384;
 // columns of a descreening group with a box of its own
 constexpr int kBoxCols = 16;
@@ -66,6 +70,10 @@ constexpr int kSplitItems = 384, kSplitSets = 6, kSplitFour = 256;
 constexpr int kGbSplitItems = 48, kGbSets = 5;
 // nodes of one order that the overlap tree's first tier holds in LDS
 constexpr int kLevelCap = 128;
+// per-call device counters: [0..7] scalars (see agbnp3_get_counts); the
+// overlap-tree kept / evaluated totals spread over kCountSlots 64-byte lines
+// (kCountBase + 8 s, + 1), so the blocks' adds at exit do not queue on one
+// address
 constexpr int kCountSlots = 32, kCountBase = 8;
 // water sites with more candidates than the first free-volume launch holds
 constexpr int kCountWs = kCountBase + 2;

@@ -212,10 +212,10 @@ struct Pack {
   std::vector<float> alpha_sum;        // per atom: ialpha + salpha
   std::vector<unsigned> curve;         // per atom: Model::curve
   hipStream_t stream = nullptr;
-  // second stream for the water-site kernels, which need only the self
-  // volumes: they run beside the descreening and pair kernels (fork and join
-  // events, also inside a captured graph); later the derivative pass's
-  // second tree tier runs on it beside the first tier
+  // second stream (fork and join events, also inside a captured graph): in
+  // large calls the water-site kernels, which need only the self volumes, run
+  // there beside the descreening and pair kernels; later one tier of the
+  // derivative pass beside the other
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_fork2 = nullptr, ev_join2 = nullptr;
   std::vector<void *> allocs, item_allocs;

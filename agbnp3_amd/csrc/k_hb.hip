@@ -11,10 +11,10 @@
 //
 // Free volume: heavy atoms passing the FP32 test
 // d2 < ((R + 1.4) * 1.6)^2 are collected from the cell grid and sorted by
-// atom index; their Gaussian overlaps are evaluated lane-parallel, then one
-// lane walks them in index order exactly as the reference does
-// (agbnp3_ws_free_volumes_scalev_ps, kernels.c:2774-2934): subtract
-// spe * V' while the free volume exceeds 0.6 V_w.  By default the spe read is
+// atom index; their Gaussian overlaps are evaluated lane-parallel, then taken
+// in index order exactly as the reference does
+// (agbnp3_ws_free_volumes_scalev_ps, kernels.c:2774-2934), every lane following
+// the same walk: subtract spe * V' while the free volume exceeds 0.6 V_w.  By default the spe read is
 // the previous overlap partner's (the reference's stale index, first one
 // given by the previous site's last parent); AGBNP3_OPT_HB_FIXED uses the
 // partner's own.  E_HB = sum khb s(V_free / V_w; 0.65, 1).
@@ -493,8 +493,8 @@ void launch_ws_free(const Dev &d, hipStream_t s) {
 // behind each scalar load, a branch and an LDS wait per column: that one
 // wave's latency, 100 us, is the launch's at 2,000 and at 8,000 atoms alike.
 // Here an item is a row block against one 256-column tile; its columns and
-// tables come to LDS in one round of vector loads, and the lookups of eight
-// columns are in flight together.  A row's FP32 sum runs over the tile's
+// tables come to LDS in one round of vector loads, and the lookups of
+// kDtUnroll columns are in flight together.  A row's FP32 sum runs over the tile's
 // columns in the same order, with the same operations, as k_descreen's, and
 // leaves as a plain store of the tile's sum (k_born adds the tiles).  The
 // water sites' free volumes, which need only the self volumes too, take the

@@ -176,9 +176,9 @@ void launch_descreen(const Dev &d, const Tuning &t, hipStream_t s) {
 // staged in LDS.  Wave w holds rows lane + 64 k, k = 0..3 -- every row of the
 // tile, four per lane -- and sweeps the 64 columns of chunk w: at step s lane
 // l reads column (l - s) mod 64 of the chunk, adds the four rows' terms to
-// the column's partial sums, and those move one lane per step with a DPP wave
-// rotation, so every lane meets every column once and the sums end where
-// they started (one column read and one rotation per four pairs).  A row's
+// the column's partial sums, and those move on by one lane per step, so every
+// lane meets every column once and the sums end where they started (one column
+// read and one rotation per four pairs).  A row's
 // sums over the four waves' chunks are added in wave order through LDS.
 // Diagonal tiles see each pair twice and keep only the row side.
 // Bound: VALU issue.  On this GPU two waves of a SIMD can each issue an FP32

@@ -22,8 +22,8 @@
 // root with order-independent fixed-point atomics; the root, a member of
 // every overlap, is summed in lane registers.  A root whose tree outgrows
 // the LDS level buffers is queued for the next tier, and past the second
-// tier for the depth-first kernel (one sibling group per pass), which holds
-// one group per order at a time.
+// tier walked depth first (one sibling group per pass), with one group per
+// order held at a time.
 //
 // Root frame: a root's slot atoms are staged at their positions relative to
 // the root (an FP32 difference of nearby coordinates, accurate to an ulp of
@@ -798,10 +798,9 @@ __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
 
 // pass B's depth-first walk of the roots its second tier listed: one wave each,
 // as many at a time as the CUs hold, since a root here takes a millisecond or
-// more where solutes are dense (coordinates of the synthetic solute scaled by
-// 0.8, so that a third of the roots come here; calls with 64, 256 and 1,024
-// blocks: 6,000 atoms by 0.75 74.4, 30.4 and 21.7 ms, 25,000 by 0.8 94.7, 33.5
-// and 21.5 ms).  Blocks without a root cost nothing: 6,000 and 25,000 atoms as
+// more where solutes are dense.  Calls of the synthetic solute, its coordinates
+// scaled, with 64, 256 and 1,024 blocks: 6,000 atoms by 0.75 (824 roots here)
+// 74.4, 30.4 and 21.7 ms, 25,000 by 0.8 (1,637 roots) 94.7, 33.5 and 21.5 ms.  Blocks without a root cost nothing: 6,000 and 25,000 atoms as
 // generated 299 and 945 us with either number.
 constexpr int kDfsBlocks = 1024;
 template <int CAP>

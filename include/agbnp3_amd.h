@@ -29,9 +29,9 @@ int agbnp3_set_options(int tag, int options);
    gradients [3*natoms], interleaved like float_i (*)[3]; energies[7] =
    egb, evdw, ecorr_vdw, ecav, ecorr_cav, ehb, mol_volume.  Enqueued on the
    instance stream and returns without waiting; call agbnp3_sync (or wait on
-   agbnp3_stream) before reading outputs.  (From 16384 atoms the water-site
+   agbnp3_stream) before reading outputs.  (From 512 atoms some of the
    kernels run on a second stream of the instance, joined into the instance
-   stream before the call's last kernels: waiting on the instance stream
+   stream before the call's last kernel: waiting on the instance stream
    covers them.)  Host-side errors (bad tag, HB
    topology) are reported immediately; device-side capacity errors by the
    next agbnp3_sync. */
@@ -86,7 +86,7 @@ int agbnp3_batch_set_nblist_reuse(int batch, float skin, int every);
    item (64, 128 or 256 of a 256-atom block, 0 = 256); persistent grid of the
    descreening, GB-pair and chain-rule kernels (blocks, 0 = one per work
    item); neighbour-list row capacity (64, 128, 256); persistent grid of the
-   first overlap-tree tier (blocks, 0 = 16 per CU).  No counterpart in the
+   first overlap-tree tier (blocks, 0 = one per heavy atom).  No counterpart in the
    reference. */
 #define AGBNP3_TUNING_PARAMS 8
 int agbnp3_get_tuning(int tag, int *params, int nparams);
