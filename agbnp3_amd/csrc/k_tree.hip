@@ -800,8 +800,9 @@ __global__ __launch_bounds__(64 * kBigWaves, 4) void k_tree_bfs_big(Dev d) {
 // as many at a time as the CUs hold, since a root here takes a millisecond or
 // more where solutes are dense.  Calls of the synthetic solute, its coordinates
 // scaled, with 64, 256 and 1,024 blocks: 6,000 atoms by 0.75 (824 roots here)
-// 74.4, 30.4 and 21.7 ms, 25,000 by 0.8 (1,637 roots) 94.7, 33.5 and 21.5 ms.  Blocks without a root cost nothing: 6,000 and 25,000 atoms as
-// generated 299 and 945 us with either number.
+// 74.4, 30.4 and 21.7 ms, 25,000 by 0.8 (1,637 roots) 94.7, 33.5 and 21.5 ms.
+// Blocks without a root cost nothing: 6,000 and 25,000 atoms as generated 299
+// and 945 us with either number.
 constexpr int kDfsBlocks = 1024;
 template <int CAP>
 __global__ __launch_bounds__(64) void k_tree_dfs(Dev d) {
